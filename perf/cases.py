@@ -167,6 +167,17 @@ class Weights:
             _abi.load().byhip_q4_resident_free(self.handle)
 
 
+class Table:
+    """A decode table uploaded through the session; freed with the object."""
+
+    def __init__(self, t):
+        self.h = gb.sessionUpload(gb.gbHip, t)
+
+    def __del__(self):
+        if getattr(self, "h", None):
+            gb.sessionFree(gb.gbHip, self.h)
+
+
 def _handle(t):
     return gb.SessionHandle(gb.gbHip, t.data_ptr(), t.numel() * t.element_size())
 
@@ -235,8 +246,8 @@ def prepare(case, seed):
         s["h"] = (_handle(s["y"]), _handle(s["blob"]), _handle(s["blob"]), _handle(s["x"]))
     elif k == "fp4km":
         s["x"], s["blob"], s["y"] = i["x"], i["w"], empty(c["M"], c["N"])
-        s["t"] = dev.DeviceBuffer.from_array(i["t"])
-        s["h"] = (_handle(s["x"]), _handle(s["blob"]), gb.SessionHandle(gb.gbHip, s["t"].ptr, s["t"].nbytes), _handle(s["y"]))
+        s["t"] = Table(i["t"])
+        s["h"] = (_handle(s["x"]), _handle(s["blob"]), s["t"].h, _handle(s["y"]))
     elif k == "f16":
         s["x"], s["w"], s["y"] = i["x"], i["w"], empty(c["M"], c["N"])
         s["h"] = (_handle(s["x"]), _handle(s["w"]), _handle(s["y"]))
