@@ -13,7 +13,8 @@ namespace byhip {
 
 // Weight formats of the LDS-staged fp16 MFMA GEMM (y[M, N] = x[M, K] . W^T, fp32 accumulation).
 enum class BFormat {
-    Q4Fast,     // Q4 nibbles, integer zero points, fp16 scales: (q - z) * s rounded once to fp16
+    Q4Fast,     // Q4 nibbles, integer zero points (one, or per group with the prefill copy), fp16
+                // scales: (q - z) * s rounded once to fp16
     Q4Generic,  // Q4 nibbles, any zeros / scales / group: ((float)q - z) * s rounded to fp16
     Fp4Km,      // FP4-KM nibbles + scale bytes + 272-float decode table
     F16         // IEEE halves [N, K]
@@ -37,7 +38,8 @@ struct GemmArgs {
     const void* sblk = nullptr;    // fp16 scales per 32-value chunk in blocks of 8 columns,
                                    // [ceil(N/8)][K/32][8] (byhip_q4w::sblk), or null
     const uint8_t* wpf = nullptr;  // the prefill copy of the nibbles and its scales
-    const void* spf = nullptr;     // (byhip_q4w::wpf, spf), or null
+    const void* spf = nullptr;     // (byhip_q4w::wpf, spf), or null; zpf its zeros when they differ
+    const void* zpf = nullptr;     // between groups (byhip_q4w::zpf)
     // FP4-KM
     const uint8_t* blob = nullptr;
     size_t scale_base = 0;

@@ -894,12 +894,12 @@ __host__ __device__ constexpr int wide_wplanes(int v) { return v == kWideHalf ? 
 
 // Sizes for FM row fragments (BM = 16 FM rows: 64 for prefill, 32 or 16 for small M), D
 // activation buffers per group (loads D - 1 sub-steps ahead) and operand kind V.
-template <int FM, int D, int V = kWideHalf>
+template <int FM, int D, int V = kWideHalf, bool ZG = false>
 struct WideShape {
     static constexpr int XS = wide_xplanes(V);
     static constexpr int kBM = 16 * FM;
     static constexpr int kXBuf = XS * kBM * kWideSub * 2;     // one activation buffer (all planes)
-    static constexpr int kLoads = XS * FM + 4 + 1;            // loads per wave and sub-step
+    static constexpr int kLoads = XS * FM + 4 + 1 + ZG;       // loads per wave and sub-step
     static constexpr int kLdsX = 4 * D * kXBuf;               // 4 groups x D buffers
     static constexpr int kLdsRed = 4 * kBM * kWidePitch * 4;  // 4 partial tiles
     static constexpr int kLds = kLdsX > kLdsRed ? kLdsX : kLdsRed;
@@ -910,10 +910,10 @@ struct WideShape {
 constexpr int wide_depth(int) { return 4; }
 
 // One wave's prefill-copy operands of one sub-step: per fragment 16 nibbles (two words), and the
-// four fragments' fp16 scales.
+// four fragments' fp16 scales (and zeros, when they differ between groups).
 struct WideW {
     v2u w[4];
-    v2u s;
+    v2u s, z;
 };
 
 // A sub-step's kind: whether it issues the loads of the sub-step a pipeline depth minus one ahead,
@@ -926,13 +926,17 @@ struct WideStep {
     static constexpr bool guard = G;
 };
 
-template <int FM, int YT, int D = wide_depth(FM), int V = kWideHalf>
+// ZG: a zero per group, in fp16 beside the scales (zpf): one more 8-byte load per sub-step and, per
+// fragment and K half, two packed additions that form the zeros' exponent-word terms. Everything
+// else is as with one zero. K = 4096, N = 11008, group 128, M = 251, fp16: 169 us on the general
+// kernel (gemm_f16_mfma), 43 here.
+template <int FM, int YT, int D = wide_depth(FM), int V = kWideHalf, bool ZG = false>
 __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
     static_assert(FM == 1 || FM == 2 || FM == 4, "q4_gemm_wide: 16, 32 or 64 rows");
     constexpr int XS = wide_xplanes(V), WS = wide_wplanes(V);  // activation and weight planes
     static_assert(V == kWideHalf || FM <= 2, "q4_gemm_wide: two operand planes up to 32 rows");
     constexpr int FN = 4;
-    using S = WideShape<FM, D, V>;
+    using S = WideShape<FM, D, V, ZG>;
     constexpr int BM = S::kBM, kXBuf = S::kXBuf, kLoads = S::kLoads;
     static_assert(D >= 4 && S::kLds <= 160 * 1024 && (D - 2) * kLoads <= 63,
                   "q4_gemm_wide: the buffers must fit LDS and the loads in flight the wait counter");
@@ -963,6 +967,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
     const rsrc_t xlr = make_rsrc(XS == 2 ? a.x_lo : a.x, XS == 2 ? (uint32_t)((size_t)a.M * K * 2) : 0u);
     const rsrc_t wr = make_rsrc(a.wpf, (uint32_t)(((size_t)a.N + 15) / 16 * nsub_all * 512));
     const rsrc_t sr = make_rsrc(a.spf, (uint32_t)(((size_t)a.N + 63) / 64 * nsub_all * 256));
+    const rsrc_t zr = make_rsrc(ZG ? a.zpf : a.spf, ZG ? (uint32_t)(((size_t)a.N + 63) / 64 * nsub_all * 256) : 0u);
     // Direct load q (0 .. FM - 1) of wave h: rows 8 FM h + 8 q + lane / 8 of the tile, LDS slot
     // lane % 8 (with two planes, the low plane's rows follow the high plane's in the buffer).
     uint32_t xo[FM];
@@ -1009,6 +1014,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
         for (int j = 0; j < FN; ++j)
             r.w[j] = __builtin_amdgcn_raw_buffer_load_b64(wr, wo, oob + 512u * u + (uint32_t)j * wfrag, 0);
         r.s = __builtin_amdgcn_raw_buffer_load_b64(sr, so, oob + 256u * u, 0);
+        if constexpr (ZG) r.z = __builtin_amdgcn_raw_buffer_load_b64(zr, so, oob + 256u * u, 0);
     };
 
     const _Float16 zlo = (_Float16)(1024.0f + a.zero_value), zhi = (_Float16)(64.0f + a.zero_value);
@@ -1032,11 +1038,18 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
         for (int j = 0; j < FN; ++j) {
             const _Float16 sc = bits_h((uint16_t)(r.s[j >> 1] >> (16 * (j & 1))));
             const h2 ss = {sc, sc};
+            h2 zlo2 = zz_lo, zhi2 = zz_hi;
+            if constexpr (ZG) {
+                const _Float16 zs = bits_h((uint16_t)(r.z[j >> 1] >> (16 * (j & 1))));
+                const h2 zz = {zs, zs};
+                zlo2 = zz + (h2){1024, 1024};
+                zhi2 = zz + (h2){64, 64};
+            }
             const uint32_t d = r.w[j][kk], d8 = d >> 8;
-            const h2 q0 = bits_h2((d & 0x000F000Fu) | mag_lo) - zz_lo;
-            const h2 q1 = bits_h2((d & 0x00F000F0u) | mag_hi) - zz_hi;
-            const h2 q2 = bits_h2((d8 & 0x000F000Fu) | mag_lo) - zz_lo;
-            const h2 q3 = bits_h2((d8 & 0x00F000F0u) | mag_hi) - zz_hi;
+            const h2 q0 = bits_h2((d & 0x000F000Fu) | mag_lo) - zlo2;
+            const h2 q1 = bits_h2((d & 0x00F000F0u) | mag_hi) - zhi2;
+            const h2 q2 = bits_h2((d8 & 0x000F000Fu) | mag_lo) - zlo2;
+            const h2 q3 = bits_h2((d8 & 0x00F000F0u) | mag_hi) - zhi2;
             const h2 w0 = q0 * ss, w1 = q1 * ss, w2 = q2 * ss, w3 = q3 * ss;
             const uint4 u = make_uint4(h2_bits(w0), h2_bits(w1), h2_bits(w2), h2_bits(w3));
             bw[0][j] = *reinterpret_cast<const h8*>(&u);
@@ -1094,7 +1107,8 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
     // wave's reads of t - 1 freed before the previous barrier. At the mid-step wait the loads of
     // t + 2 .. t + D - 1 may stay in flight, those that were issued.
     constexpr int kMfmas = (XS + WS - 1) * FM * FN;                                 // per K half
-    constexpr int kValuPerMfma = (FN * (WS == 2 ? 18 : 14) + kMfmas - 1) / kMfmas;  // a K half's dequantization
+    // a K half's dequantization
+    constexpr int kValuPerMfma = (FN * ((WS == 2 ? 18 : 14) + (ZG ? 3 : 0)) + kMfmas - 1) / kMfmas;
     auto step = [&](int t, auto kc, auto kind) __attribute__((always_inline)) {
         constexpr int k = decltype(kc)::value, k1 = (k + 1) % D, kp = (k + D - 1) % D;
         constexpr int kWait = decltype(kind)::wait;
@@ -1214,21 +1228,22 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
 //   Split-K: block z covers the sub-steps [z * split_steps, ...) and writes fp32 partials.
 constexpr int kTallBM = 128, kTallBN = 256;
 constexpr int kTallXBuf = kTallBM * kWideSub * 2;           // one activation buffer (16 KB)
-constexpr int kTallLoads = 2 + 2 + 1;                       // loads per wave and sub-step
+constexpr int tall_loads(bool zg) { return 2 + 2 + 1 + zg; }  // loads per wave and sub-step
 constexpr int kTallPitch = 32 + 4;                          // floats per row of a wave's staged block
 constexpr int kTallLdsOut = 8 * kTallBM * kTallPitch * 4;  // the eight waves' staged blocks
 constexpr int kTallDepth = 4;                               // activation buffers and operand sets
 constexpr int tall_lds(int depth) { return depth * kTallXBuf > kTallLdsOut ? depth * kTallXBuf : kTallLdsOut; }
 
 // One wave's prefill-copy operands of one sub-step: per fragment 16 nibbles (two words), and the
-// two fragments' fp16 scales.
+// two fragments' fp16 scales (and zeros, when they differ between groups).
 struct TallW {
     v2u w[2];
-    uint32_t s;
+    uint32_t s, z;
 };
 
-template <int YT, int D = kTallDepth>
+template <int YT, int D = kTallDepth, bool ZG = false>
 __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
+    constexpr int kTallLoads = tall_loads(ZG);
     static_assert(D >= 3 && D * kTallXBuf <= 160 * 1024, "q4_gemm_tall: 3 to 10 buffers");
     constexpr int FM = 8, FN = 2;
     __shared__ __attribute__((aligned(16))) uint8_t lds[tall_lds(D)];
@@ -1255,6 +1270,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
     const rsrc_t xr = make_rsrc(a.x, (uint32_t)((size_t)a.M * K * 2));
     const rsrc_t wr = make_rsrc(a.wpf, (uint32_t)(((size_t)a.N + 15) / 16 * nsub_all * 512));
     const rsrc_t sr = make_rsrc(a.spf, (uint32_t)(((size_t)a.N + 63) / 64 * nsub_all * 256));
+    const rsrc_t zr = make_rsrc(ZG ? a.zpf : a.spf, ZG ? (uint32_t)(((size_t)a.N + 63) / 64 * nsub_all * 256) : 0u);
     // Direct load q (0, 1) of wave w: rows 16 w + 8 q + lane / 8 of the tile, LDS slot lane % 8.
     uint32_t xo[2];
 #pragma unroll
@@ -1286,6 +1302,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
         for (int j = 0; j < FN; ++j)
             r.w[j] = __builtin_amdgcn_raw_buffer_load_b64(wr, wo, oob + 512u * u + (uint32_t)j * wfrag, 0);
         r.s = __builtin_amdgcn_raw_buffer_load_b32(sr, so, oob + 256u * u, 0);
+        if constexpr (ZG) r.z = __builtin_amdgcn_raw_buffer_load_b32(zr, so, oob + 256u * u, 0);
     };
 
     const _Float16 zlo = (_Float16)(1024.0f + a.zero_value), zhi = (_Float16)(64.0f + a.zero_value);
@@ -1306,13 +1323,20 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
         for (int j = 0; j < FN; ++j) {
             const _Float16 sc = bits_h((uint16_t)(r.s >> (16 * j)));
             const h2 ss = {sc, sc};
+            h2 zlo2 = zz_lo, zhi2 = zz_hi;
+            if constexpr (ZG) {
+                const _Float16 zs = bits_h((uint16_t)(r.z >> (16 * j)));
+                const h2 zz = {zs, zs};
+                zlo2 = zz + (h2){1024, 1024};
+                zhi2 = zz + (h2){64, 64};
+            }
             const uint32_t d = r.w[j][kk], d8 = d >> 8;
             const h2 q0 = bits_h2((d & 0x000F000Fu) | mag_lo);
             const h2 q1 = bits_h2((d & 0x00F000F0u) | mag_hi);
             const h2 q2 = bits_h2((d8 & 0x000F000Fu) | mag_lo);
             const h2 q3 = bits_h2((d8 & 0x00F000F0u) | mag_hi);
-            const uint4 u = make_uint4(h2_bits((q0 - zz_lo) * ss), h2_bits((q1 - zz_hi) * ss),
-                                       h2_bits((q2 - zz_lo) * ss), h2_bits((q3 - zz_hi) * ss));
+            const uint4 u = make_uint4(h2_bits((q0 - zlo2) * ss), h2_bits((q1 - zhi2) * ss),
+                                       h2_bits((q2 - zlo2) * ss), h2_bits((q3 - zhi2) * ss));
             bw[j] = *reinterpret_cast<const h8*>(&u);
         }
     };
@@ -1344,7 +1368,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
     read_x(0, 0, ax0);
     dequant(rs[0], 0, bw0);
 
-    constexpr int kValuPerMfma = (FN * 14 + FM * FN - 1) / (FM * FN);  // a K half's dequantization
+    constexpr int kValuPerMfma = (FN * (ZG ? 17 : 14) + FM * FN - 1) / (FM * FN);  // a K half's dequantization
     // Sub-step t = base + k (base a multiple of D) with register sets rs[k] (t's operands),
     // rs[k + 1] (t + 1's) and rs[k - 1] (refilled with t + D - 1's weights), all indices mod D;
     // t + D - 1's activations go to buffer k - 1, which every wave's reads of t - 1 freed before the
@@ -1430,15 +1454,17 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
     }
 }
 
-// Whether the pipelined Q4 kernel takes these arguments.
-bool q4_pipe_ok(const GemmArgs& a) {
+// What the fp16 kernels for the benchmark format ask of a call, whatever its zeros.
+bool q4_half_ok(const GemmArgs& a) {
     const bool pow2_group = a.group % 32 == 0 && ((a.group >> 5) & ((a.group >> 5) - 1)) == 0;
-    return a.x_dtype == BYHIP_F16 && a.K % PBK == 0 && a.scale_f16 && !a.zeros &&
-           (a.group == 0 || pow2_group) && a.row_bytes % 16 == 0 &&
+    return a.x_dtype == BYHIP_F16 && a.K % PBK == 0 && a.scale_f16 && (a.group == 0 || pow2_group) && a.row_bytes % 16 == 0 &&
            reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.wq) % 16 == 0 &&
            (uint64_t)(a.M + 64) * a.K * 2 < kOutOfRange && (uint64_t)(a.N + 128) * a.row_bytes < kOutOfRange &&
            (uint64_t)(a.N + 128) * a.gpr * 2 < kOutOfRange;
 }
+
+// Whether the pipelined Q4 kernel takes these arguments.
+bool q4_pipe_ok(const GemmArgs& a) { return !a.zeros && q4_half_ok(a); }
 
 template <int BM, int FN>
 void launch_q4_skinny_shape(const GemmArgs& a, int splits) {
@@ -1451,16 +1477,22 @@ void launch_q4_skinny_shape(const GemmArgs& a, int splits) {
     BYHIP_LAUNCHED("q4_gemm_skinny");
 }
 
-template <int FM, int V = kWideHalf>
-void launch_q4_wide_shape(const GemmArgs& a, int splits) {
+template <int FM, int V, bool ZG>
+void launch_q4_wide_zeros(const GemmArgs& a, int splits) {
     const dim3 grid((a.N + kWideBN - 1) / kWideBN, (a.M + 16 * FM - 1) / (16 * FM), splits);
     constexpr int D = wide_depth(FM);
     switch (a.y_dtype) {
-    case BYHIP_F32: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_F32, D, V>), grid, dim3(512), 0, a); break;
-    case BYHIP_F16: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_F16, D, V>), grid, dim3(512), 0, a); break;
-    default: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_BF16, D, V>), grid, dim3(512), 0, a); break;
+    case BYHIP_F32: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_F32, D, V, ZG>), grid, dim3(512), 0, a); break;
+    case BYHIP_F16: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_F16, D, V, ZG>), grid, dim3(512), 0, a); break;
+    default: launch("q4_gemm_wide", (q4_gemm_wide<FM, BYHIP_BF16, D, V, ZG>), grid, dim3(512), 0, a); break;
     }
     BYHIP_LAUNCHED("q4_gemm_wide");
+}
+
+template <int FM, int V = kWideHalf>
+void launch_q4_wide_shape(const GemmArgs& a, int splits) {
+    if (a.zeros) launch_q4_wide_zeros<FM, V, true>(a, splits);
+    else launch_q4_wide_zeros<FM, V, false>(a, splits);
 }
 
 // Rows per tile: 16 or 32 when M fits, else 64.
@@ -1553,12 +1585,12 @@ bool q4_skinny_ok(const GemmArgs& a) {
            (uint64_t)(a.N + 64) * a.gpr * 2 < kLim;
 }
 
-// Whether the wide tile takes the call: the weights' prefill copy (K % 64 == 0), the pipelined
-// kernel's conditions and all operand offsets, including the rows and columns a tile reaches past
+// Whether the wide tile takes the call: the weights' prefill copy (K % 64 == 0; zeros that differ
+// between groups must be in it), the pipelined kernel's other conditions and all operand offsets, including the rows and columns a tile reaches past
 // M and N, below 2^31.
 bool q4_wide_ok(const GemmArgs& a) {
     constexpr uint64_t kLim = 0x80000000u;
-    return a.wpf && a.spf && a.K % kWideSub == 0 && q4_pipe_ok(a) && (uint64_t)(a.M + 64) * a.K * 2 < kLim &&
+    return a.wpf && a.spf && (!a.zeros || a.zpf) && a.K % kWideSub == 0 && q4_half_ok(a) && (uint64_t)(a.M + 64) * a.K * 2 < kLim &&
            (uint64_t)(a.N + 128) * a.row_bytes < kLim && (uint64_t)(a.N + 128) * a.gpr * 2 < kLim;
 }
 
@@ -1571,6 +1603,17 @@ bool q4_big_ok(const GemmArgs& a) {
 
 int q4_big_splits(const GemmArgs& a);
 
+template <bool ZG>
+void launch_q4_tall_zeros(const GemmArgs& a, dim3 grid) {
+    constexpr int D = kTallDepth;
+    switch (a.y_dtype) {
+    case BYHIP_F32: launch("q4_gemm_tall", (q4_gemm_tall<BYHIP_F32, D, ZG>), grid, dim3(512), 0, a); break;
+    case BYHIP_F16: launch("q4_gemm_tall", (q4_gemm_tall<BYHIP_F16, D, ZG>), grid, dim3(512), 0, a); break;
+    default: launch("q4_gemm_tall", (q4_gemm_tall<BYHIP_BF16, D, ZG>), grid, dim3(512), 0, a); break;
+    }
+    BYHIP_LAUNCHED("q4_gemm_tall");
+}
+
 // The 128 x 256 tile (the tall kernel) with one block per CU, K split as q4_big_splits says (or
 // `split_choice`).
 void launch_q4_big(const GemmArgs& a0, int split_choice = 0) {
@@ -1579,12 +1622,8 @@ void launch_q4_big(const GemmArgs& a0, int split_choice = 0) {
     const int forced = split_choice > 0 ? split_choice : q4_big_splits(a);
     const int splits = choose_split(a, tiles, a.K / kWideSub, 8, forced);
     const dim3 grid((a.N + kTallBN - 1) / kTallBN, (a.M + kTallBM - 1) / kTallBM, splits);
-    switch (a.y_dtype) {
-    case BYHIP_F32: launch("q4_gemm_tall", q4_gemm_tall<BYHIP_F32>, grid, dim3(512), 0, a); break;
-    case BYHIP_F16: launch("q4_gemm_tall", q4_gemm_tall<BYHIP_F16>, grid, dim3(512), 0, a); break;
-    default: launch("q4_gemm_tall", q4_gemm_tall<BYHIP_BF16>, grid, dim3(512), 0, a); break;
-    }
-    BYHIP_LAUNCHED("q4_gemm_tall");
+    if (a.zeros) launch_q4_tall_zeros<true>(a, grid);
+    else launch_q4_tall_zeros<false>(a, grid);
     if (a.part) launch_splitk_sum(a, splits);
 }
 
@@ -1652,7 +1691,7 @@ bool q4_small_wide(const GemmArgs& a) {
 // conditions), K % 64 == 0, 16-byte aligned activation rows, and the operand offsets below 2^31.
 bool q4_wide_f32_ok(const GemmArgs& a) {
     constexpr uint64_t kLim = 0x80000000u;
-    return a.x_dtype == BYHIP_F32 && a.wpf && a.spf && a.K % kWideSub == 0 && a.scale_f16 && !a.zeros &&
+    return a.x_dtype == BYHIP_F32 && a.wpf && a.spf && a.K % kWideSub == 0 && a.scale_f16 && (!a.zeros || a.zpf) &&
            reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && (uint64_t)(a.M + 32) * a.K * 2 < kLim &&
            (uint64_t)(a.N + 128) * a.row_bytes < kLim && (uint64_t)(a.N + 128) * a.gpr * 2 < kLim;
 }
@@ -1823,8 +1862,8 @@ bool launch_q4_choice(BFormat fmt, const GemmArgs& a, int kind, int tile, int sp
         launch_q4_stream(a, splits);
         return true;
     case kQ4General:
-        if (fmt == BFormat::Q4Fast) launch_f<BFormat::Q4Fast>(a);
-        else if (fmt == BFormat::Q4Generic) launch_f<BFormat::Q4Generic>(a);
+        if (fmt == BFormat::Q4Fast && !a.zeros) launch_f<BFormat::Q4Fast>(a);
+        else if (fmt == BFormat::Q4Fast || fmt == BFormat::Q4Generic) launch_f<BFormat::Q4Generic>(a);
         else return false;
         return true;
     default:
@@ -1871,7 +1910,10 @@ void launch_gemm(BFormat fmt, const GemmArgs& a) {
         case kQ4Big: launch_q4_big(a); break;
         case kQ4Wide: launch_q4_skinny(a, 0, true); break;
         case kQ4Pipe: launch_q4_pipe(a); break;
-        default: launch_f<BFormat::Q4Fast>(a); break;
+        default:
+            if (a.zeros) launch_f<BFormat::Q4Generic>(a);  // it reads the zeros, Q4Fast one for all
+            else launch_f<BFormat::Q4Fast>(a);
+            break;
         }
         break;
     case BFormat::Q4Generic: launch_f<BFormat::Q4Generic>(a); break;

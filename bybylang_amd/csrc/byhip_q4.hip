@@ -85,18 +85,20 @@ __global__ void q4_unpack(const uint8_t* __restrict__ wq, size_t row_bytes, int 
 //   3  the largest |scale| (float bits)
 //   4  the smallest nonzero |scale| (float bits; +inf when every scale is zero)
 //   5, 6  the smallest and largest zero (float bits)
+//   7  every zero is a whole number
 // The host combines the blocks.
 __global__ __launch_bounds__(256) void q4_classify(const float* __restrict__ sc, const float* __restrict__ ze,
                                                    size_t ng, int* __restrict__ flags) {
     __shared__ float red[4][4];
     const uint32_t z0 = __builtin_bit_cast(uint32_t, ze[0]);
-    int ok_s = 1, ok_z = 1, fin = 1;
+    int ok_s = 1, ok_z = 1, fin = 1, whole = 1;
     float smax = 0.0f, smin = __builtin_inff(), zmin = __builtin_inff(), zmax = -__builtin_inff();
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < ng; i += (size_t)gridDim.x * 256) {
         const float s = sc[i], z = ze[i];
         ok_s &= (__builtin_isfinite(s) && (float)(_Float16)s == s) ? 1 : 0;
         ok_z &= __builtin_bit_cast(uint32_t, z) == z0 ? 1 : 0;
         fin &= (__builtin_isfinite(s) && __builtin_isfinite(z)) ? 1 : 0;
+        whole &= z == rintf(z) ? 1 : 0;
         const float as = fabsf(s);
         smax = fmaxf(smax, as);
         if (as > 0.0f) smin = fminf(smin, as);
@@ -117,6 +119,7 @@ __global__ __launch_bounds__(256) void q4_classify(const float* __restrict__ sc,
     ok_s = __syncthreads_and(ok_s);
     ok_z = __syncthreads_and(ok_z);
     fin = __syncthreads_and(fin);
+    whole = __syncthreads_and(whole);
     if (threadIdx.x == 0) {
         int* f = flags + 8 * blockIdx.x;
         f[0] = ok_s;
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(256) void q4_classify(const float* __restrict__ sc,
         f[4] = __builtin_bit_cast(int, fminf(fminf(red[1][0], red[1][1]), fminf(red[1][2], red[1][3])));
         f[5] = __builtin_bit_cast(int, fminf(fminf(red[2][0], red[2][1]), fminf(red[2][2], red[2][3])));
         f[6] = __builtin_bit_cast(int, fmaxf(fmaxf(red[3][0], red[3][1]), fmaxf(red[3][2], red[3][3])));
-        f[7] = 0;
+        f[7] = whole;
     }
 }
 
@@ -164,11 +167,12 @@ __global__ __launch_bounds__(256) void q4_pack_scales(const float* __restrict__ 
 // scales [N * gpr]: word i of wpf holds, for fragment f, sub-step u, lane l = c + 16 g and half d,
 // the nibbles of column 16 f + c at K positions p0 .. p0 + 7 (p0 = 64 u + 16 g + 8 d), position
 // p0 + k at bits 4 (k / 2) for even k and 16 + 4 (k / 2) for odd k; half i of spf the scale of
-// column 64 q + 16 j + c at K position 64 u + 32 t. Columns past N are zeros.
+// column 64 q + 16 j + c at K position 64 u + 32 t, and half i of zpf (when given) that column's zero
+// there. Columns past N are zeros.
 __global__ __launch_bounds__(256) void q4_pack_prefill(const uint8_t* __restrict__ wq, size_t row_bytes,
-                                                       const float* __restrict__ sc, int N, int K, int gpr,
-                                                       int group, uint32_t* __restrict__ wpf,
-                                                       _Float16* __restrict__ spf) {
+                                                       const float* __restrict__ sc, const float* __restrict__ ze,
+                                                       int N, int K, int gpr, int group, uint32_t* __restrict__ wpf,
+                                                       _Float16* __restrict__ spf, _Float16* __restrict__ zpf) {
     const size_t nsub = (size_t)K / 64;
     const size_t nw = (size_t)(N + 15) / 16 * nsub * 128, ns = (size_t)(N + 63) / 64 * nsub * 128;
     const size_t total = nw > ns ? nw : ns;
@@ -187,7 +191,9 @@ __global__ __launch_bounds__(256) void q4_pack_prefill(const uint8_t* __restrict
         if (i < ns) {
             const size_t j = i & 3, c = (i >> 2) & 15, t = (i >> 6) & 1, u = (i >> 7) % nsub, q = (i >> 7) / nsub;
             const size_t n = 64 * q + 16 * j + c, p = 64 * u + 32 * t;
-            spf[i] = n < (size_t)N ? (_Float16)sc[n * gpr + (group ? p / (size_t)group : 0)] : (_Float16)0.0f;
+            const size_t src = n * gpr + (group ? p / (size_t)group : 0);
+            spf[i] = n < (size_t)N ? (_Float16)sc[src] : (_Float16)0.0f;
+            if (zpf) zpf[i] = n < (size_t)N ? (_Float16)ze[src] : (_Float16)0.0f;
         }
     }
 }
@@ -233,13 +239,14 @@ byhip_q4w* build_resident_dev(const void* wq_src, bool wq_on_device, const float
         throw;
     }
     device_free(d_flags);
-    bool sf16 = true, zu = true, finite = true;
+    bool sf16 = true, zu = true, finite = true, whole = true;
     float smax = 0.0f, smin = INFINITY, zmin = INFINITY, zmax = -INFINITY;
     for (int b = 0; b < cblocks; ++b) {
         const int* f = &flags[8 * b];
         sf16 = sf16 && f[0];
         zu = zu && f[1];
         finite = finite && f[2];
+        whole = whole && f[7];
         smax = std::fmax(smax, bits_float(f[3]));
         smin = std::fmin(smin, bits_float(f[4]));
         zmin = std::fmin(zmin, bits_float(f[5]));
@@ -259,14 +266,18 @@ byhip_q4w* build_resident_dev(const void* wq_src, bool wq_on_device, const float
     const size_t G = (size_t)K / 32, n_pad = ((size_t)N + 7) / 8 * 8;
     const size_t sb_bytes = blk ? n_pad * G * (sf16 ? 2 : 4) : 0;
     const size_t zb_bytes = blk && !zu ? n_pad * G * 4 : 0;
-    // Prefill copy (byhip_q4w::wpf, spf) for the fp16 MFMA prefill kernels.
-    const bool pf = f16_safe && sf16 && zu && K % 64 == 0 && (group == 0 || group % 32 == 0) && row_bytes % 4 == 0;
+    // Prefill copy (byhip_q4w::wpf, spf, zpf) for the fp16 MFMA prefill kernels. A zero per group must
+    // be one the kernels subtract exactly: they form 1024 + z and 64 + z in fp16.
+    const bool zg = !zu && whole && zmin >= -1024.0f && zmax <= 1024.0f;
+    const bool pf = f16_safe && sf16 && (zu || zg) && K % 64 == 0 && (group == 0 || group % 32 == 0) && row_bytes % 4 == 0;
     const size_t nsub = (size_t)K / 64;
     const size_t wpf_bytes = pf ? ((size_t)N + 15) / 16 * nsub * 512 : 0;
     const size_t spf_bytes = pf ? ((size_t)N + 63) / 64 * nsub * 256 : 0;
+    const size_t zpf_bytes = pf && zg ? spf_bytes : 0;
     const size_t o_s = align256(wq_bytes), o_z = o_s + align256(s_bytes), o_sb = o_z + align256(z_bytes),
                  o_zb = o_sb + align256(sb_bytes), o_wpf = o_zb + align256(zb_bytes),
-                 o_spf = o_wpf + align256(wpf_bytes), total = o_spf + align256(spf_bytes);
+                 o_spf = o_wpf + align256(wpf_bytes), o_zpf = o_spf + align256(spf_bytes),
+                 total = o_zpf + align256(zpf_bytes);
     uint8_t* base = static_cast<uint8_t*>(device_alloc(total));
     byhip_q4w* w = new byhip_q4w{};
     w->K = K; w->N = N; w->group = group; w->gpr = gpr; w->row_bytes = row_bytes;
@@ -283,6 +294,7 @@ byhip_q4w* build_resident_dev(const void* wq_src, bool wq_on_device, const float
     w->f16_safe = f16_safe;
     w->wpf = pf ? base + o_wpf : nullptr;
     w->spf = pf ? base + o_spf : nullptr;
+    w->zpf = pf && zg ? base + o_zpf : nullptr;
     try {
         BYHIP_HIP(hipMemcpyAsync(w->wq, wq_src, wq_bytes, wq_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                                  stream()));
@@ -294,8 +306,9 @@ byhip_q4w* build_resident_dev(const void* wq_src, bool wq_on_device, const float
         if (pf) {
             const size_t pw = std::max(((size_t)N + 15) / 16 * nsub * 128, ((size_t)N + 63) / 64 * nsub * 128);
             const int fblocks = (int)std::min<size_t>((pw + 255) / 256, (size_t)compute_units() * 16);
-            launch("q4_pack_prefill", q4_pack_prefill, dim3(fblocks), dim3(256), 0, w->wq, row_bytes, d_sc, N, K,
-                               gpr, group, reinterpret_cast<uint32_t*>(w->wpf), static_cast<_Float16*>(w->spf));
+            launch("q4_pack_prefill", q4_pack_prefill, dim3(fblocks), dim3(256), 0, w->wq, row_bytes, d_sc, d_ze, N,
+                               K, gpr, group, reinterpret_cast<uint32_t*>(w->wpf), static_cast<_Float16*>(w->spf),
+                               static_cast<_Float16*>(w->zpf));
             BYHIP_LAUNCHED("q4_pack_prefill");
         }
         BYHIP_HIP(hipStreamSynchronize(stream()));  // the source may be pageable host memory
@@ -371,7 +384,7 @@ void launch_generic(const void* x, int x_dtype, const byhip_q4w* w, void* y, int
 
 // Zero points the fp16 MFMA path subtracts exactly: integers with |1024 + z| representable.
 bool zeros_integral(const byhip_q4w* w) {
-    if (!w->zero_uniform) return false;  // per-group zeros: the generic dequant handles them
+    if (!w->zero_uniform) return false;  // per-group zeros: the prefill copy, else the generic dequant
     const float z = w->zero_value;
     return std::floor(z) == z && z >= -1024.0f && z <= 1024.0f;
 }
@@ -385,13 +398,14 @@ GemmArgs q4_gemm_args(const void* x, int x_dtype, const byhip_q4w* w, void* y, i
     a.sblk = w->blk_scale_f16 ? w->sblk : nullptr;
     a.wpf = w->wpf;
     a.spf = w->spf;
+    a.zpf = w->zpf;
     return a;
 }
 
-// Weights the fp16 MFMA kernels take in the Q4Fast form: fp16 scales, an integral uniform zero,
-// group 0 or a multiple of 32.
+// Weights the fp16 MFMA kernels take in the Q4Fast form: fp16 scales, an integral uniform zero (or
+// zeros in the prefill copy), group 0 or a multiple of 32.
 bool q4_fast(const byhip_q4w* w) {
-    return w->scale_f16 && zeros_integral(w) && (w->group == 0 || w->group % 32 == 0);
+    return w->scale_f16 && (zeros_integral(w) || w->zpf) && (w->group == 0 || w->group % 32 == 0);
 }
 
 // Routes y = x . W^T. Decode shapes (M <= 8) take the GEMV, whose arithmetic is exact (fp32 scales,

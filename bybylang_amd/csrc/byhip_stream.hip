@@ -334,7 +334,7 @@ int stream_fn(const GemmArgs& a, int row_blocks) {
 
 bool q4_stream_ok(const GemmArgs& a) {
     constexpr uint64_t kLim = 0x80000000u;  // offsets stay below 2^31 (the kernel's out-of-range steps)
-    return a.x_dtype == BYHIP_F16 && a.wpf && a.spf && a.M >= 1 && a.M <= 32 && a.K % kSub == 0 &&
+    return a.x_dtype == BYHIP_F16 && a.wpf && a.spf && !a.zeros && a.M >= 1 && a.M <= 32 && a.K % kSub == 0 &&
            (uint64_t)32 * a.K * 2 < kLim && (uint64_t)(a.N + 16 * kMaxFN) * a.K / 2 < kLim &&
            (uint64_t)(a.N + 64 * kMaxFN) / 64 * (a.K / kSub) * 256 < kLim;
 }
