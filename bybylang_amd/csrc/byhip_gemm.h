@@ -60,6 +60,8 @@ struct GemmArgs {
     // The wide tile on fp32 activations: x holds the high fp16 plane of the shifted activations and
     // x_lo the low one (x * 2^t = hi + lo, t per row in row_shift).
     const void* x_lo = nullptr;
+    // gemm_planes: the fp32 activations themselves (x and x_lo hold their planes).
+    const void* x_raw = nullptr;
     // A device-side route choice: when gate is set, the general fp16 MFMA GEMM, the exact GEMM and
     // their split-K sum do nothing unless *gate == gate_want (the flag a classification kernel
     // earlier on the stream wrote), so two routes can be queued and only the chosen one runs.
@@ -179,6 +181,13 @@ bool q4_stream_ok(const GemmArgs& a);
 int stream_fn(const GemmArgs& a, int row_blocks);
 int stream_row_blocks(const GemmArgs& a);
 void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
+
+// fp32 activations as two fp16 planes against FP4-KM weights with an E2M1 table, or half weights
+// (byhip_planes.hip): whether the kernel takes the call (K % 128 == 0 for FP4-KM, K % 64 == 0 for F16,
+// 16-byte aligned operands, offsets below 2^31), and the launch. FP4-KM tables other than E2M1 give
+// the same results, slowly.
+bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
+void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
 
 // Native MXFP4 GEMM (E2M1 x E2M1 with E8M0 block scales): x and w in the FP4-KM packing.
 // K % 128 == 0 is required.

@@ -1,0 +1,604 @@
+// byhip_planes.hip - fp32 activations as two fp16 planes against quantized or half weights (gfx950).
+//
+// y[M, N] = x[M, K] . W^T. Each row of x is brought onto fp16's range by an exact power of two
+// (undone on the output) and split into hi = fp16(x) and lo = fp16(x - hi), about 23 bits of x
+// (split_planes); hi . w + lo . w in v_mfma_f32_16x16x32_f16 with fp32 accumulation then keeps
+// them, for weights that are exact in fp16:
+//   FP4-KM with an E2M1 table and scales whose products with it are halves (checked per scale byte
+//          while it is used; a block that meets another scale, or a table that is not E2M1,
+//          computes its tile again in fp32 arithmetic as the reference does)
+//   F16
+//
+// Block: 16 FM rows x 128 columns, eight waves, two per SIMD. Waves w, w + 2, .. (p = w % 2) form K
+// group p, which takes every other 128-value step of the block; wave h = w / 2 of the group owns
+// columns 32 h .. 32 h + 31 (2 fragments) and all rows: each decoded weight fragment feeds 2 FM
+// MFMAs (hi and lo), and each activation fragment read from LDS 2. Two K groups rather than four
+// (the wide tile) halve the LDS the activations need, so two planes of 64 rows fit four buffers.
+//
+// A 128-value step is two sub-steps of 64 values (one 128-byte line of each plane row); the group's
+// slice of both planes moves straight into LDS by direct loads, 16-byte chunk k of row r at slot
+// k ^ x_swizzle(r), four buffers, loads three sub-steps ahead. Lane (c, g) = (lane % 16, lane / 16)
+// multiplies chunks 2 g and 2 g + 1 of the slice with its weights of column c:
+//   F16     16 halves of the weight row, in natural order
+//   FP4-KM  the four lane groups hold the step's four 32-value groups, one 16-byte load per column
+//           and step: bytes 4 q .. 4 q + 3 of the group are elements 4 q .. 4 q + 3 (low nibbles)
+//           and 16 + 4 q .. (high); sub-step e multiplies q = 2 e and 2 e + 1. split_planes writes the
+//           planes in that order, chunk 8 (q / 2) + 2 g + q % 2 of a 128-value block holding elements
+//           4 q, 16 + 4 q, 4 q + 1, .. of group g. One lane then needs one scale per step.
+// Sub-steps run in two halves around one block barrier, as in the wide tile (byhip_gemm.hip).
+#include <algorithm>
+
+#include "byhip_gemm.h"
+#include "byhip_internal.h"
+#include "byhip_kernels.h"
+
+namespace byhip {
+namespace {
+
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+constexpr int kBN = 128;
+constexpr int kSub = 64;              // K values per sub-step
+constexpr int kDepth = 4;             // activation buffers per K group
+constexpr int kSets = 4;              // weight register sets
+constexpr int kUnroll = 8;            // sub-steps per loop iteration
+constexpr int kPitch = kBN + 4;       // floats per row of a staged partial tile
+constexpr uint32_t kUnsafe = 0xFFFFu;      // (a NaN) a scale whose products with E2M1 are not all halves
+constexpr uint32_t kPast = 0x80000000u;    // added to an offset: every resource here rejects it
+
+template <int FM>
+struct PlaneShape {
+    static constexpr int kBM = 16 * FM;
+    static constexpr int kXBuf = 2 * kBM * kSub * 2;     // one buffer: both planes' slices
+    static constexpr int kLdsX = 2 * kDepth * kXBuf;     // two K groups
+    static constexpr int kLdsRed = 2 * kBM * kPitch * 4; // two partial tiles
+    static constexpr int kLds = kLdsX > kLdsRed ? kLdsX : kLdsRed;
+};
+
+__device__ constexpr uint32_t e2m1_bits(int i) {  // fp32 bits of the E2M1 value of code i
+    constexpr uint32_t v[8] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u, 0x40C00000u};
+    return v[i & 7] | (i & 8 ? 0x80000000u : 0u);
+}
+
+// The block's tile in fp32 arithmetic, each weight lut[code] * lut[16 + scale byte] as the
+// reference forms it, x in fp32, v_mfma_f32_16x16x4_f32: wave w computes columns 16 w .. + 15 over
+// 32-value groups g0 .. g1 - 1 and leaves its sums in `red`.
+template <int FM>
+__device__ __forceinline__ void fp4_tile_exact(const GemmArgs& a, int m0, int n0, int g0, int g1,
+                                               float* red) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int n = n0 + 16 * wid + c;
+    const float* const x = static_cast<const float*>(a.x_raw);
+    const float* const lut = a.lut;
+    f4 acc[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) acc[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int G = g0; G < g1; ++G) {
+        uint32_t w = 0;
+        float s = 0.0f;
+        if (n < a.N) {
+            w = *reinterpret_cast<const uint32_t*>(a.blob + (size_t)n * (a.K >> 1) + 16 * (size_t)G + 4 * g);
+            s = lut[16 + a.blob[a.scale_base + (size_t)n * (a.K >> 5) + G]];
+        }
+        float wl[4], wh[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            wl[j] = n < a.N ? lut[(w >> (8 * j)) & 15u] * s : 0.0f;
+            wh[j] = n < a.N ? lut[(w >> (8 * j + 4)) & 15u] * s : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int m = m0 + 16 * i + c;
+            float4 xl = make_float4(0.0f, 0.0f, 0.0f, 0.0f), xh = xl;
+            if (m < a.M) {
+                const float* r = x + (size_t)m * a.K + 32 * (size_t)G + 4 * g;
+                xl = *reinterpret_cast<const float4*>(r);
+                xh = *reinterpret_cast<const float4*>(r + 16);
+            }
+            const float al[4] = {xl.x, xl.y, xl.z, xl.w}, ah[4] = {xh.x, xh.y, xh.z, xh.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(al[j], wl[j], acc[i], 0, 0, 0);
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[j], wh[j], acc[i], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int at = (16 * i + 4 * g + r) * kPitch + 16 * wid + c;
+            red[at] = acc[i][r];
+            red[16 * FM * kPitch + at] = 0.0f;  // the second K group's partial tile
+        }
+}
+
+template <BFormat F, int FM, int YT>
+__global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 4 : 2) void gemm_planes(GemmArgs a) {
+    if (a.gate && *a.gate != a.gate_want) return;  // another route was chosen (whole grid)
+    constexpr bool FP4 = F == BFormat::Fp4Km;
+    constexpr int FN = 2;
+    using S = PlaneShape<FM>;
+    constexpr int BM = S::kBM, kXBuf = S::kXBuf;
+    // One LDS array for everything, the eight waves' `bad` words at its end: beside a second array (a
+    // table of its own, or the one inside __syncthreads_or) the compiler no longer told the direct
+    // loads from the fragment reads apart and waited for every load in flight before each read: 47 us
+    // instead of 43 at M = 512, K = N = 4096.
+    __shared__ __attribute__((aligned(16))) uint8_t lds[S::kLds + 32];
+
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = wid & 1, h = wid >> 1;
+    const int c = lane & 15, g = lane >> 4;
+    int bx = blockIdx.x, by = blockIdx.y;
+    {
+        // the wide tile's XCD-grouped tile order
+        const int gx = gridDim.x, gy = gridDim.y, tiles = gx * gy, id = bx + gx * by;
+        const int j = tiles % 8 == 0 ? (id % 8) * (tiles / 8) + id / 8 : id;
+        const int grp = j / (4 * gx), rows = min(4, gy - 4 * grp), r = j % (4 * gx);
+        by = 4 * grp + r % rows;
+        bx = r / rows;
+    }
+    const int n0 = bx * kBN, m0 = by * BM;
+    const int K = a.K;
+    // the block's 128-value steps (the last one half empty when K / 64 is odd) and 64-value slices
+    const int step0 = a.part ? (int)blockIdx.z * a.split_steps : 0;
+    const int steps_all = (K + 127) / 128;
+    const int steps = a.part ? min(a.split_steps, steps_all - step0) : steps_all;
+    const int slices = min(2 * steps, K / kSub - 2 * step0);
+    const int pairs_all = (steps + 1) / 2, nt_all = 2 * pairs_all;  // per K group: its steps, sub-steps
+
+    // The table lives in registers: lane l holds scale entries 4 l .. 4 l + 3 as halves (kUnsafe: its
+    // products with E2M1 are not all halves), looked up across lanes.
+    float lut_v[FP4 ? 4 : 1];
+    uint32_t lut_h[FP4 ? 2 : 1];
+    bool bad = false;
+    if constexpr (FP4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lut_v[i] = a.lut[16 + 4 * lane + i];
+        bad = lane < 16 && __builtin_bit_cast(uint32_t, a.lut[lane & 15]) != e2m1_bits(lane & 15);
+    }
+
+    const rsrc_t xr = make_rsrc(h < 2 ? a.x : a.x_lo, (uint32_t)((size_t)a.M * K * 2));
+    const rsrc_t wr = FP4 ? make_rsrc(a.blob, (uint32_t)((size_t)a.N * (K >> 1)))
+                          : make_rsrc(a.w16, (uint32_t)((size_t)a.N * K * 2));
+    const rsrc_t sr = FP4 ? make_rsrc(a.blob + a.scale_base, (uint32_t)((size_t)a.N * (K >> 5))) : wr;
+    // Direct load q (0 .. FM - 1) of wave h: stacked rows 8 FM h + 8 q + lane / 8 of the slice (the
+    // high plane's BM rows, then the low plane's), LDS slot lane % 8.
+    uint32_t xo[FM];
+#pragma unroll
+    for (int q = 0; q < FM; ++q) {
+        const int r = 8 * FM * (h & 1) + 8 * q + (lane >> 3), chunk = (lane & 7) ^ x_swizzle(r);
+        xo[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + 16u * chunk;
+    }
+    uint32_t wo[FN], so[FN];
+    bool col_ok[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int n = n0 + 32 * h + 16 * j + c;
+        col_ok[j] = n < a.N;
+        wo[j] = FP4 ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g : (uint32_t)n * (uint32_t)K * 2u + 32u * g;
+        so[j] = (uint32_t)n * (uint32_t)(K >> 5) + 8u * g;
+    }
+    uint8_t* const xgrp = lds + p * kDepth * kXBuf;
+    const int rd0 = 128 * c + 16 * ((2 * g) ^ x_swizzle(c)), rd1 = 128 * c + 16 * ((2 * g + 1) ^ x_swizzle(c));
+
+    // The group's sub-step t is slice 2 p + 4 (t / 2) + t % 2 of the block; past the last it reads zeros.
+    auto load_x = [&](int t, int buf) __attribute__((always_inline)) {
+        const int sl = 2 * p + 4 * (t >> 1) + (t & 1);
+        const uint32_t off = sl < slices ? 128u * (uint32_t)(2 * step0 + sl) : kPast;
+#pragma unroll
+        for (int q = 0; q < FM; ++q) lds_dma16(xr, xgrp + buf * kXBuf + 1024 * (FM * h + q), xo[q], off);
+    };
+    // FP4-KM: the 16 bytes per column of the group's step q (sub-steps 2 q and 2 q + 1); F16: the
+    // sub-step's 32 bytes.
+    v4u wv[kSets][FP4 ? FN : 2 * FN];
+    auto load_w = [&](v4u (&w)[FP4 ? FN : 2 * FN], int t) __attribute__((always_inline)) {
+        if constexpr (FP4) {
+            const int s = p + 2 * t;
+            const uint32_t off = s < steps ? 64u * (uint32_t)(step0 + s) : kPast;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) w[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off, 0);
+        } else {
+            const int sl = 2 * p + 4 * (t >> 1) + (t & 1);
+            const uint32_t off = sl < slices ? 128u * (uint32_t)(2 * step0 + sl) : kPast;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                w[2 * j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off, 0);
+                w[2 * j + 1] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off + 16u, 0);
+            }
+        }
+    };
+    // FP4-KM scale bytes: the dword of lane (c, i) holds the four bytes (groups 0 .. 3) of column c in
+    // the group's step 4 v + i, so one load per column and four steps; lane (c, g) fetches byte g
+    // of the step's dword from lane (c, q % 4).
+    uint32_t sb[FP4 ? FN : 1], sbn[FP4 ? FN : 1], ss[FP4 ? FN : 1];
+    auto load_sb = [&](uint32_t (&d)[FP4 ? FN : 1], int v) __attribute__((always_inline)) {
+        const int s0 = p + 8 * v;  // step of lane group 0; the lane's own is s0 + 2 g
+        const uint32_t past = s0 + 2 * g >= steps ? kPast : 0u;
+#pragma unroll
+        for (int j = 0; j < (FP4 ? FN : 0); ++j)
+            d[j] = __builtin_amdgcn_raw_buffer_load_b32(sr, so[j] | past, 4u * (uint32_t)(step0 + s0), 0);
+    };
+    auto scale_of = [&](const uint32_t (&d)[FP4 ? FN : 1], int q, uint32_t (&s)[FP4 ? FN : 1]) __attribute__((always_inline)) {
+        const bool live = p + 2 * q < steps;
+#pragma unroll
+        for (int j = 0; j < (FP4 ? FN : 0); ++j) {
+            const uint32_t b = ((uint32_t)__builtin_amdgcn_ds_bpermute(4 * (16 * (q & 3) + c), (int)d[j]) >> (8 * g)) & 255u;
+            const uint32_t v0 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(b & 252u), (int)lut_h[0]);
+            const uint32_t v1 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(b & 252u), (int)lut_h[FP4 ? 1 : 0]);
+            const uint32_t v = (((b & 2u) ? v1 : v0) >> (16 * (b & 1u))) & 0xFFFFu;
+            const bool use = live && col_ok[j];
+            bad = bad || (use && v == kUnsafe);
+            s[j] = use ? v | (v << 16) : 0u;
+        }
+    };
+
+    f4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+
+    // Weights of MFMA kk of sub-step parity e.
+    auto decode = [&](const v4u (&w)[FP4 ? FN : 2 * FN], int e, int kk, h8 (&b)[FN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            if constexpr (FP4) {
+                const uint32_t d = w[j][2 * e + kk];
+                const h2 s2 = bits_h2(ss[j]);
+                const uint4 u = make_uint4(h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 0) * s2),
+                                           h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 1) * s2),
+                                           h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 2) * s2),
+                                           h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 3) * s2));
+                b[j] = *reinterpret_cast<const h8*>(&u);
+            } else {
+                b[j] = __builtin_bit_cast(h8, w[2 * j + kk]);
+            }
+        }
+    };
+    auto read_x = [&](int buf, int kk, h8 (&x)[2][FM]) __attribute__((always_inline)) {
+        const uint8_t* src = xgrp + buf * kXBuf + (kk ? rd1 : rd0);
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+            for (int i = 0; i < FM; ++i) x[pl][i] = *reinterpret_cast<const h8*>(src + 128 * BM * pl + 2048 * i);
+    };
+    auto mfmas = [&](const h8 (&x)[2][FM], const h8 (&b)[FN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[pl][i], b[j], acc[i][j], 0, 0, 0);
+    };
+
+    // Loads of a sub-step at position k of the unrolled loop (weights first, then activations): the
+    // activations of sub-step t + 3, the weights of t + 3 (F16) or, on even t, of step t / 2 + 3
+    // (FP4-KM, with the next four steps' scale bytes at k = 0).
+    constexpr int kXLoads = FM;
+    auto issued = [](int k) constexpr {
+        return kXLoads + (FP4 ? ((k & 1) ? 0 : FN) + (k == 0 ? FN : 0) : 2 * FN);
+    };
+
+    h8 ax0[2][FM], ax1[2][FM], bw0[FN], bw1[FN];
+    if constexpr (FP4) load_sb(sb, 0);
+    static_for<3>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        load_w(wv[k], k);
+        load_x(k, k);
+    });
+    if constexpr (FP4) {
+        uint32_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // every product with E2M1 is a half when 0.5 v and 1.5 v are and 6 v is in range
+            const float v = lut_v[i], v1 = 0.5f * v, v3 = 1.5f * v;
+            const bool ok = fabsf(6.0f * v) <= 65504.0f && (float)(_Float16)v1 == v1 && (float)(_Float16)v3 == v3;
+            b[i] = ok ? h_bits((_Float16)v) : kUnsafe;
+        }
+        lut_h[0] = b[0] | (b[1] << 16);
+        lut_h[1] = b[2] | (b[3] << 16);
+    }
+    wait_vmcnt<2 * (kXLoads + (FP4 ? FN : 2 * FN))>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (FP4) scale_of(sb, 0, ss);
+    read_x(0, 0, ax0);
+    decode(wv[0], 0, 0, bw0);
+
+    constexpr int kMfmas = 2 * FM * FN;  // per K half
+    constexpr int kValuPerMfma = FP4 ? (FN * 9 + kMfmas - 1) / kMfmas : 1;
+    // Sub-step t = base + k. Its loads, in `wait` order: at the mid-step wait those of this and of the
+    // previous sub-step may stay in flight, which leaves t + 1's activations landed.
+    auto step = [&](int t, auto kc, auto guard) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value, e = k & 1;
+        constexpr int set = FP4 ? (k >> 1) % kSets : k % kSets;             // t's weights
+        constexpr int set1 = FP4 ? ((k + 1) >> 1) % kSets : (k + 1) % kSets;  // t + 1's
+        const bool live = !decltype(guard)::value || t < nt_all;
+        uint32_t sn[FP4 ? FN : 1];
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!FP4) load_w(wv[(k + 3) % kSets], t + 3);
+        if constexpr (FP4 && e == 0) load_w(wv[((k >> 1) + 3) % kSets], (t >> 1) + 3);
+        if constexpr (FP4 && k == 0) load_sb(sbn, (t >> 3) + 1);
+        load_x(t + 3, (k + 3) % kDepth);
+        if (live) {
+            mfmas(ax0, bw0);
+            read_x(k % kDepth, 1, ax1);
+            decode(wv[set], e, 1, bw1);
+            if constexpr (FP4 && e == 1) scale_of(k == 7 ? sbn : sb, (t >> 1) + 1, sn);
+#pragma unroll
+            for (int m = 0; m < kMfmas; ++m) {
+                __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);                   // one MFMA
+                if (m < 2 * FM) __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);   // a fragment read
+                if (m < issued(k)) __builtin_amdgcn_sched_group_barrier(0x0010, 1, 0);  // a load
+                __builtin_amdgcn_sched_group_barrier(0x0002, kValuPerMfma, 0);        // its share of the VALU
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<issued((k + 7) % 8) + issued(k)>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (live) {
+            if constexpr (FP4 && e == 1) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j) ss[j] = sn[j];
+            }
+            mfmas(ax1, bw1);
+            read_x((k + 1) % kDepth, 0, ax0);
+            decode(wv[set1], e ^ 1, 0, bw0);
+#pragma unroll
+            for (int m = 0; m < kMfmas; ++m) {
+                __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);                  // one MFMA
+                if (m < 2 * FM) __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);  // a fragment read
+                __builtin_amdgcn_sched_group_barrier(0x0002, kValuPerMfma, 0);       // its share of the VALU
+            }
+        }
+        if constexpr (FP4 && k == 7) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) sb[j] = sbn[j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int t = 0;
+    for (; t + kUnroll <= nt_all; t += kUnroll)
+        static_for<kUnroll>([&](auto kc) { step(t + decltype(kc)::value, kc, std::false_type{}); });
+    if (t < nt_all)
+        static_for<kUnroll>([&](auto kc) { step(t + decltype(kc)::value, kc, std::true_type{}); });
+
+    // Partial tiles -> LDS, once every wave's loads have landed and every wave is done with the
+    // buffers -> the two groups' sums -> y or the split-K partials.
+    wait_vmcnt<0>();
+    uint32_t* const bads = reinterpret_cast<uint32_t*>(lds + S::kLds);
+    if constexpr (FP4) {
+        const bool any = __any(bad);
+        if (lane == 0) bads[wid] = any ? 1u : 0u;
+    }
+    __syncthreads();
+    bool redo = false;
+    if constexpr (FP4) {
+        const uint4 b0 = reinterpret_cast<const uint4*>(bads)[0], b1 = reinterpret_cast<const uint4*>(bads)[1];
+        redo = (b0.x | b0.y | b0.z | b0.w | b1.x | b1.y | b1.z | b1.w) != 0u;
+    }
+    float* red = reinterpret_cast<float*>(lds);  // [2 groups][BM rows][kPitch]
+    if (redo) {
+        fp4_tile_exact<FM>(a, m0, n0, 4 * step0, min(4 * (step0 + steps), K / 32), red);
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    red[(p * BM + 16 * i + 4 * g + r) * kPitch + 32 * h + 16 * j + c] = acc[i][j][r];
+    }
+    __syncthreads();
+    float* part = a.part ? a.part + (size_t)blockIdx.z * splitk_stride(a.M, a.N) : nullptr;
+    const bool vec = out8_vector_ok<YT>(a, part);
+#pragma unroll
+    for (int k = 0; k < (BM * 16 + 511) / 512; ++k) {
+        const int u = tid + 512 * k;  // chunk of 8 outputs: row u / 16, columns 8 (u % 16)
+        if (u >= BM * 16) break;
+        const int row = u >> 4, col = (u & 15) * 8;
+        const int m = m0 + row;
+        if (m >= a.M) continue;
+        const float* src = red + row * kPitch + col;
+        const int sh = redo ? 0 : a.row_shift[m];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const float4 s0 = *reinterpret_cast<const float4*>(src + e);
+            const float4 s1 = *reinterpret_cast<const float4*>(src + BM * kPitch + e);
+            v[e] = __builtin_amdgcn_ldexpf(s0.x + s1.x, -sh);
+            v[e + 1] = __builtin_amdgcn_ldexpf(s0.y + s1.y, -sh);
+            v[e + 2] = __builtin_amdgcn_ldexpf(s0.z + s1.z, -sh);
+            v[e + 3] = __builtin_amdgcn_ldexpf(s0.w + s1.w, -sh);
+        }
+        store_out8<YT>(a, part, vec, m, n0 + col, v);
+    }
+}
+
+// Rows of fp32 activations as two fp16 planes (one block per row): the row's power-of-two shift t
+// brings its largest magnitude into [2^14, 2^15); hi = fp16(x 2^t), lo = fp16(x 2^t - hi), and an
+// infinite x gives an infinite hi and lo = 0. A thread makes 16-byte chunks of 8 values: elements
+// 8 i .. 8 i + 7 (natural order), or for FP4-KM (FP4) elements 4 q .. and 16 + 4 q .. of a 32-value
+// group interleaved, chunk i = 4 G + q of the row at 16 (G / 4) + 8 (q / 2) + 2 (G % 4) + q % 2. The
+// first kHeld chunks of a thread stay in registers between the maximum and the split.
+constexpr int kHeld = 4;
+template <bool FP4>
+__global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x, int K, int* __restrict__ shifts,
+                                                   uint4* __restrict__ hi, uint4* __restrict__ lo) {
+    __shared__ float part[4];
+    const size_t row = (size_t)blockIdx.x * K;
+    const float4* r = reinterpret_cast<const float4*>(x + row);
+    const int nc = K / 8;
+    auto first = [](int i) { return FP4 ? 8 * (i >> 2) + (i & 3) : 2 * i; };  // float4 index of a chunk
+    constexpr int second = FP4 ? 4 : 1;
+    float4 ha[kHeld], hb[kHeld];
+    float mx = 0.0f;
+    auto most = [&](const float4& v) {
+        mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int i = (int)threadIdx.x + 256 * u;
+        ha[u] = i < nc ? r[first(i)] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        hb[u] = i < nc ? r[first(i) + second] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        most(ha[u]);
+        most(hb[u]);
+    }
+    for (int i = (int)threadIdx.x + 256 * kHeld; i < nc; i += 256) {
+        most(r[first(i)]);
+        most(r[first(i) + second]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    const int t = fp16_range_shift(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+    if (threadIdx.x == 0) shifts[blockIdx.x] = t;
+    auto split = [&](int i, const float4& va, const float4& vb) {
+        const float s[8] = {va.x, FP4 ? vb.x : va.y, FP4 ? va.y : va.z, FP4 ? vb.y : va.w,
+                            FP4 ? va.z : vb.x, FP4 ? vb.z : vb.y, FP4 ? va.w : vb.z, vb.w};
+        uint32_t hw[4], lw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint16_t hh[2], ll[2];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const float v = __builtin_amdgcn_ldexpf(s[2 * e + d], t);
+                const _Float16 he = (_Float16)v;
+                const float rest = __builtin_isinf(v) ? 0.0f : v - (float)he;
+                hh[d] = h_bits(he);
+                ll[d] = h_bits((_Float16)rest);
+            }
+            hw[e] = hh[0] | ((uint32_t)hh[1] << 16);
+            lw[e] = ll[0] | ((uint32_t)ll[1] << 16);
+        }
+        const size_t at = row / 8 + (FP4 ? 16 * (i >> 4) + 8 * ((i & 3) >> 1) + 2 * ((i >> 2) & 3) + (i & 1) : i);
+        hi[at] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+        lo[at] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int i = (int)threadIdx.x + 256 * u;
+        if (i < nc) split(i, ha[u], hb[u]);
+    }
+    for (int i = (int)threadIdx.x + 256 * kHeld; i < nc; i += 256) split(i, r[first(i)], r[first(i) + second]);
+}
+
+template <BFormat F, int FM>
+void launch_planes_y(const GemmArgs& a, int splits) {
+    const dim3 grid((a.N + kBN - 1) / kBN, (a.M + 16 * FM - 1) / (16 * FM), splits);
+    switch (a.y_dtype) {
+    case BYHIP_F32: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F32>), grid, dim3(512), 0, a); break;
+    case BYHIP_F16: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F16>), grid, dim3(512), 0, a); break;
+    default: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_BF16>), grid, dim3(512), 0, a); break;
+    }
+    BYHIP_LAUNCHED("gemm_planes");
+}
+
+template <BFormat F>
+void launch_planes_fm(const GemmArgs& a, int fm, int splits) {
+    switch (fm) {
+    case 1: launch_planes_y<F, 1>(a, splits); break;
+    case 2: launch_planes_y<F, 2>(a, splits); break;
+    case 3: launch_planes_y<F, 3>(a, splits); break;
+    default: launch_planes_y<F, 4>(a, splits); break;
+    }
+}
+
+// Row fragments per tile: the fewest padded rows, the larger tile among equals.
+int planes_fm(int M) {
+    int best = 1, best_rows = 1 << 30;
+    for (int fm = 4; fm >= 1; --fm) {
+        const int rows = (M + 16 * fm - 1) / (16 * fm) * fm;
+        if (rows < best_rows) best = fm, best_rows = rows;
+    }
+    // small tiles read the weights once per tile: past 64 rows at least 48
+    return M > 64 ? std::max(best, 3) : best;
+}
+
+// K splits, in 128-value steps: the count that minimises rounds of blocks x (steps per split + 12)
+// (12 for a block's fixed cost: first loads, epilogue), plus 6 steps for the sum's launch.
+int planes_splits(const GemmArgs& a, long tiles) {
+    const int steps = (a.K + 127) / 128;
+    const long cus = compute_units();
+    int best = 1;
+    double best_t = 1e300;
+    for (int s = 1; s <= std::max(1, steps / 4); ++s) {
+        const int per = (steps + s - 1) / s;
+        if ((steps + per - 1) / per != s) continue;  // the same split as a smaller s
+        const double t = (double)((tiles * s + cus - 1) / cus) * (per + 12) + (s > 1 ? 6.0 : 0.0);
+        if (t < 0.97 * best_t) best = s, best_t = t;
+    }
+    return best;
+}
+
+template <BFormat F>
+void launch_planes_rows(const GemmArgs& a0) {
+    GemmArgs a = a0;
+    const int fm = planes_fm(a.M);
+    const long tiles = (long)((a.N + kBN - 1) / kBN) * ((a.M + 16 * fm - 1) / (16 * fm));
+    const int forced = env_int("BYHIP_Q4_SPLIT", 0);
+    const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : planes_splits(a, tiles), 1);
+    if (splits == 1) a.part = nullptr;
+    launch_planes_fm<F>(a, fm, splits);
+    if (a.part) launch_splitk_sum(a, splits);
+}
+
+}  // namespace
+
+bool gemm_planes_ok(BFormat fmt, const GemmArgs& a) {
+    constexpr uint64_t kLim = kPast;  // offsets stay below 2^31 (loads past the end)
+    if (a.x_dtype != BYHIP_F32 || reinterpret_cast<uintptr_t>(a.x) % 16 != 0) return false;
+    if ((uint64_t)(a.K) * 2 * 128 >= kLim) return false;
+    if (fmt == BFormat::Fp4Km)
+        return a.K % 128 == 0 && reinterpret_cast<uintptr_t>(a.blob) % 16 == 0 && a.scale_base % 4 == 0 &&
+               (uint64_t)(a.N + kBN) * (a.K / 2) < kLim;
+    if (fmt == BFormat::F16)
+        return a.K % kSub == 0 && reinterpret_cast<uintptr_t>(a.w16) % 16 == 0 && (uint64_t)(a.N + kBN) * a.K * 2 < kLim;
+    return false;
+}
+
+void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
+    uint8_t* const work = static_cast<uint8_t*>(a0.work ? a0.work : workspace());
+    const size_t work_bytes = a0.work ? a0.work_bytes : kWorkspaceBytes;
+    const size_t es = dtype_bytes(a0.y_dtype);
+    // Row blocks whose planes fit half the scratch (the rest holds split-K partials) and whose
+    // offsets stay below 2^31.
+    const size_t row_planes = (size_t)a0.K * 4;
+    size_t rows = std::min<size_t>(work_bytes / 2 / (row_planes + sizeof(int)), ((size_t)kPast / 2) / ((size_t)a0.K * 2));
+    rows = std::min<size_t>(rows, 65535 * 16);
+    if (rows > 64) rows = rows / 64 * 64;
+    if (rows == 0) fail("byhip: K=%d rows of fp32 activations exceed the scratch", a0.K);
+    for (size_t m = 0; m < (size_t)a0.M; m += rows) {
+        GemmArgs a = a0;
+        a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);
+        a.x_raw = static_cast<const float*>(a0.x) + m * a0.K;
+        a.y = static_cast<uint8_t*>(a0.y) + m * a0.N * es;
+        const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256;
+        const size_t plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
+        int* const shifts = reinterpret_cast<int*>(work);
+        uint8_t* const hi = work + shift_bytes;
+        uint8_t* const lo = hi + plane;
+        if (fmt == BFormat::Fp4Km)
+            launch("split_planes", split_planes<true>, dim3((unsigned)a.M), dim3(256), 0,
+                   static_cast<const float*>(a.x_raw), a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
+        else
+            launch("split_planes", split_planes<false>, dim3((unsigned)a.M), dim3(256), 0,
+                   static_cast<const float*>(a.x_raw), a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
+        BYHIP_LAUNCHED("split_planes");
+        a.x = hi;
+        a.x_lo = lo;
+        a.row_shift = shifts;
+        a.work = lo + plane;
+        a.work_bytes = work_bytes - shift_bytes - 2 * plane;
+        if (fmt == BFormat::Fp4Km) launch_planes_rows<BFormat::Fp4Km>(a);
+        else launch_planes_rows<BFormat::F16>(a);
+    }
+}
+
+}  // namespace byhip

@@ -1,0 +1,115 @@
+"""fp32 activations as two fp16 planes (FP4-KM with an E2M1 table, half weights) on the MI355X against
+the oracle, at the edges of the tiles and of the table's scales.
+
+Bar: the reference test's tolerance (max|diff| <= 1e-4 * max(1, peak)); a tile that meets a scale
+whose products are not halves is computed in fp32 arithmetic, inf and NaN included.
+"""
+import numpy as np
+import pytest
+
+from parity import ref_check
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 128, 16), (16, 256, 128), (17, 384, 130), (33, 1280, 129), (48, 1024, 264), (64, 2048, 127), (65, 640, 300),
+          (130, 1152, 520)]
+
+
+def fp4_case(M, K, N, scales, seed):
+    from bybylang_amd import synth
+    g = synth.rng(seed)
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    t = np.zeros(272, np.float32)
+    t[:16] = synth.E2M1
+    i = np.arange(256)
+    with np.errstate(over="ignore"):
+        t[16:] = np.ldexp(np.float32(1), i - 127) if scales != "ref" else (1 + i % 13) / 64
+    sb = {"ref": g.integers(0, 256, (N, K // 32)), "mx": g.integers(104, 141, (N, K // 32)),
+          "edge": g.integers(100, 150, (N, K // 32)), "one": g.integers(120, 130, (N, K // 32))}[scales].astype(np.uint8)
+    if scales == "one":
+        sb[N // 2, (K // 32) // 2] = 150  # one scale past the halves: one tile takes fp32 arithmetic
+    x = synth.activations(g, M, K, np.float32)
+    return x, np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.reshape(-1)]), t
+
+
+def run_fp4(hip, x, blob, t, M, K, N, mirror):
+    """With a host copy of the table the host chooses the route, without one the device does."""
+    import ctypes as C
+    from bybylang_amd import _abi
+    y = hip.DeviceBuffer(M * N * 4)
+    lut = hip.DeviceBuffer.from_array(t)
+    p = C.c_void_p()
+    if mirror:
+        _abi.check(_abi.load().byhip_session_upload(t.ctypes.data, t.size, C.byref(p)))
+    bd, xd = hip.DeviceBuffer.from_array(blob), hip.DeviceBuffer.from_array(x.reshape(-1))
+    _abi.check(_abi.load().byhip_fp4km_tile_gemm(xd.ptr, hip.F32, bd.ptr, bd.nbytes, N * (K // 2), p.value or lut.ptr, 272, 0,
+                                                 y.ptr, hip.F32, M, K, N))
+    out = y.read(np.float32)
+    if mirror:
+        _abi.check(_abi.load().byhip_session_free(p))
+    return out
+
+
+@pytest.mark.parametrize("mirror", [True, False])
+@pytest.mark.parametrize("scales", ["ref", "mx", "edge", "one"])
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_fp4km_planes(hip, oracle, M, K, N, scales, mirror):
+    x, blob, t = fp4_case(M, K, N, scales, M + K + N)
+    want = oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x)
+    ref_check(run_fp4(hip, x, blob, t, M, K, N, mirror), want)
+
+
+@pytest.mark.parametrize("splits", [2, 3])
+def test_fp4km_planes_split_k(hip, oracle, monkeypatch, splits):
+    M, K, N = 70, 1408, 200
+    x, blob, t = fp4_case(M, K, N, "one", 5)
+    monkeypatch.setenv("BYHIP_Q4_SPLIT", str(splits))
+    want = oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x)
+    ref_check(run_fp4(hip, x, blob, t, M, K, N, True), want)
+
+
+def test_fp4km_planes_other_table_and_nonfinite(hip, oracle):
+    """A table that is not E2M1, the same table through both choices of the route, and scales and
+    activations that are not finite: finite where the oracle is, with its infinities and NaNs."""
+    M, K, N = 20, 256, 130
+    x, blob, t = fp4_case(M, K, N, "mx", 9)
+    t2 = t.copy()
+    t2[1] = 0.75
+    want = oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t2, x)
+    for mirror in (True, False):
+        ref_check(run_fp4(hip, x, blob, t2, M, K, N, mirror), want)
+    sb = blob[N * (K // 2):].reshape(N, K // 32)
+    sb[3, 1] = 255                  # infinite scale: NaN where a code is 0 or signs differ
+    x[5, 40] = np.inf               # an infinite activation
+    x[6, 7] = np.nan
+    want = np.asarray(oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x)).reshape(-1)
+    for mirror in (True, False):
+        got = run_fp4(hip, x, blob, t, M, K, N, mirror)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.isinf(got), np.isinf(want))
+        fin = np.isfinite(want)
+        assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+        ref_check(got[fin], want[fin])
+
+
+def test_planes_in_row_blocks(hip, oracle):
+    """More rows than the scratch holds planes for: the rows go in blocks."""
+    M, K, N = 1200, 4096, 48        # 19.7 MB of planes against half of 32 MB
+    x, blob, t = fp4_case(M, K, N, "ref", 11)
+    got = run_fp4(hip, x, blob, t, M, K, N, True).reshape(M, N)
+    for r in (0, 959, 960, 1023, 1024, 1199):
+        want = oracle.tile_gemm(0, 1, K, N, N * (K // 2), 0, blob, t, x[r])
+        ref_check(got[r], want)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 64, 16), (16, 192, 128), (20, 320, 130), (40, 1088, 129), (64, 640, 264), (130, 1152, 520)])
+def test_f16_planes(hip, oracle, M, K, N):
+    from bybylang_amd import synth
+    g = synth.rng(M + K)
+    x = synth.activations(g, M, K, np.float32) * np.float32(300.0)
+    w = (g.standard_normal((N, K)) * 0.05).astype(np.float16)
+    want = oracle.tile_gemm(1, M, K, N, 0, 0, w.view(np.uint8).reshape(-1), None, x)
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.f16_tile_gemm(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.DeviceBuffer.from_array(w.reshape(-1)), y, hip.F32,
+                      M, K, N)
+    ref_check(y.read(np.float32), want)
