@@ -31,9 +31,13 @@
 // and the results are waited out before they are read. Register dependencies of the operands
 // (LDS reads feeding an MFMA) are tracked by the compiler as for any instruction.
 //
+// Products with few such tiles take smaller ones (mxfp4_gemm_mid below).
+//
 // Tile order: blocks are handed to the 8 XCDs round-robin; block b works on tile
 // (b % 8) * ceil(T/8) + b / 8 in column-major tile order, so each XCD owns a run of column tiles and
 // its L2 serves the x and W slices its CUs share.
+#include <algorithm>
+
 #include "byhip_gemm.h"
 #include "byhip_internal.h"
 #include "byhip_kernels.h"
@@ -369,6 +373,200 @@ __global__ __launch_bounds__(256) void mxfp4_gemm(MxArgs a) {
     }
 }
 
+// Row fragments of the smaller tiles for a call (0: the 256 x 256 tiles): the fewest 64-row tiles,
+// cut to the rows there are (a 48-row tile loads 176 lines per pair, a 64-row one 192, so fewer row
+// tiles beat fuller ones). They win while there are up to 2.5 of them per CU (us, 256 x 256 tiles / these;
+// K = N = 8192): M = 16 38.0 / 10.2, 100 40.2 / 14.9, 256 44.5 / 18.3, 512 44.5 / 30.7, 640 44.2 / 42.5,
+// 768 44.8 / 45.5, 1024 45.5 / 59.5; 1024 x 4096 x 4096 26.2 / 18.0; 2048 x 1024 x 2048 11.9 / 7.8.
+// BYHIP_MX_MID forces the fragments (0: the large tiles).
+int mx_mid(int M, int K, int N) {
+    const int forced = env_int("BYHIP_MX_MID", -1);
+    if ((uint64_t)(M + 64) * (K / 2) >= 0x80000000u || (uint64_t)(N + 128) * (K / 2) >= 0x80000000u) return 0;
+    if (forced >= 0) return forced;
+    const int row_tiles = (M + 63) / 64;
+    if ((long)row_tiles * ((N + 127) / 128) * 2 > 5L * compute_units()) return 0;
+    return (M + 16 * row_tiles - 1) / (16 * row_tiles);
+}
+
+// K splits of the smaller tiles: as many as leave one block per CU, each of at least two units of four
+// steps (M = 47, K = 8192, N = 8200, 65 tiles, 1 / 2 / 3 / 4 splits: 16.4 / 13.6 / 12.7 / 16.2 us; M = 1,
+// K = N = 4096, 32 tiles of 8 units, 2 / 4 / 8: 8.4 / 6.0 / 7.2; M = 256, K = N = 8192, 256 tiles, 1 / 2:
+// 18.3 / 24.9).
+int mx_mid_splits(long tiles, int units) {
+    return (int)std::max<long>(1, std::min<long>(compute_units() / tiles, units / 2));
+}
+
+// Smaller tiles, for products whose 256 x 256 tiles leave most of the chip idle: 16 FM rows x 128
+// columns per block of eight waves, two blocks per CU, K split over the grid when the tiles are few.
+//   Waves: w and w + 2, .. form K group p = w % 2, which multiplies the p-th 128-value step of each pair;
+//   wave h = w / 2 of the group owns columns 32 h .. 32 h + 31 and all rows, as FM x 2 fragments of
+//   v_mfma_scale_f32_16x16x128_f8f6f4 (lane l: row or column l % 16, 32-value group l / 16).
+//   Operands: a pair of steps is one 128-byte line of each row; the block's 16 FM + 128 lines move
+//   straight into LDS (16-byte chunk k of row r at slot k ^ x_swizzle(r)), three buffers, loads two
+//   pairs ahead, one barrier per pair. The 16 scale bytes of a row for two pairs follow every
+//   second pair. Loads straight into operand registers, 16 rows x 64 bytes each and without a barrier,
+//   were slower (M = 47, K = 8192, N = 8192: 16.8 us): half lines cost the load unit as much as whole.
+//   What bounds it: at few rows the weights' bytes and a launch's fixed costs (M = 47, K = 8192,
+//   N = 8200: 12.7 us with the sum, 39.0 on 256 x 256 tiles); with more the lines a CU can load.
+template <int FM>
+struct MidShape {
+    static constexpr int kBM = 16 * FM, kBN = 128, kRows = kBM + kBN;
+    static constexpr int kBuf = kRows * 128;                 // one pair of steps
+    static constexpr int kScale = (64 + kBN) * 16;           // two pairs' scale bytes, x rows then W rows
+    static constexpr int kPitch = kBN + 4;
+    static constexpr int kData = 3 * kBuf + 2 * kScale;
+    static constexpr int kRed = 2 * kBM * kPitch * 4;
+    static constexpr int kLds = kData > kRed ? kData : kRed;
+    static constexpr int kLoads = 3;                         // per wave and pair: the kRows / 8 line groups over 8 waves
+};
+
+template <int FM, int YT>
+__global__ __launch_bounds__(512, 4) void mxfp4_gemm_mid(MxArgs a, GemmArgs out) {
+    using S = MidShape<FM>;
+    constexpr int BM = S::kBM, FN = 2;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[S::kLds];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = wid & 1, h = wid >> 1, c = lane & 15, g = lane >> 4;
+    const int t = (blockIdx.x % kXcds) * a.per_xcd + blockIdx.x / kXcds;
+    if (t >= a.tiles) return;  // whole block
+    const int m0 = (t % a.tiles_m) * BM, n0 = (t / a.tiles_m) * S::kBN;
+    const uint32_t kb = (uint32_t)a.K >> 1, kg = (uint32_t)a.K >> 5;
+    // the block's pairs of steps, from an even one on
+    const int steps_all = a.K / KSTEP;
+    const int q0 = out.part ? 2 * (int)blockIdx.y * out.split_steps : 0;
+    const int pairs_all = (steps_all + 1) / 2;
+    const int nq = out.part ? min(2 * out.split_steps, pairs_all - q0) : pairs_all;
+
+    const rsrc_t xr = make_rsrc(a.x, (uint32_t)a.M * kb), wr = make_rsrc(a.w, (uint32_t)a.N * kb);
+    const rsrc_t xsr = make_rsrc(a.xs, (uint32_t)a.M * kg), wsr = make_rsrc(a.ws, (uint32_t)a.N * kg);
+    // Line group i of the block: rows 8 i .. 8 i + 7, the x rows first; a wave takes groups w, w + 8,
+    // w + 16 (past the last: the last again, so that every wave has the same loads in flight). Rows
+    // past M or N read zeros.
+    uint32_t off[S::kLoads];
+    bool is_x[S::kLoads];
+    int grp[S::kLoads];
+#pragma unroll
+    for (int i = 0; i < S::kLoads; ++i) {
+        grp[i] = min(wid + 8 * i, S::kRows / 8 - 1);
+        is_x[i] = grp[i] < BM / 8;
+        const int r = 8 * grp[i] + (lane >> 3);  // row of the buffer
+        const uint32_t row = (uint32_t)(is_x[i] ? m0 + r : n0 + r - BM);
+        off[i] = row * kb + 16u * (uint32_t)((lane & 7) ^ x_swizzle(r & 15));
+    }
+    // scale line group: 64 x rows (those past the tile are not read), W rows 0 .. 63, 64 .. 127
+    const int sgrp = min(wid, 2);
+    const uint32_t soff = (uint32_t)(sgrp == 0 ? m0 + lane : n0 + 64 * (sgrp - 1) + lane) * kg;
+    auto load = [&](int q, int buf) __attribute__((always_inline)) {
+        const uint32_t o = q < nq ? 128u * (uint32_t)(q0 + q) : 0x80000000u;
+#pragma unroll
+        for (int i = 0; i < S::kLoads; ++i) lds_dma16(is_x[i] ? xr : wr, lds + buf * S::kBuf + 1024 * grp[i], off[i], o);
+    };
+    auto load_scales = [&](int q, int buf) __attribute__((always_inline)) {  // pairs q, q + 1 (q even)
+        lds_dma16(sgrp == 0 ? xsr : wsr, lds + 3 * S::kBuf + buf * S::kScale + 1024 * sgrp, soff,
+                  q < nq ? 8u * (uint32_t)(q0 + q) : 0x80000000u);
+    };
+
+    f4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    const int rd = 128 * c + 16 * ((4 * p + g) ^ x_swizzle(c));
+    const int wrow = BM + 32 * h;
+    auto wide8 = [](const v4u& v) __attribute__((always_inline)) {
+        return (i8v){(int)v[0], (int)v[1], (int)v[2], (int)v[3], 0, 0, 0, 0};
+    };
+
+    load_scales(0, 0);
+    load(0, 0);
+    load(1, 1);
+    // Pair q = base + k: the wait leaves the loads of pair q + 1 in flight (with the scales issued
+    // beside them, for odd q); the barrier publishes every wave's lines of pair q and frees the buffer
+    // of pair q - 1, which the loads of q + 2 go to.
+    auto pair = [&](int q, auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+        wait_vmcnt<S::kLoads + (k & 1)>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr ((k & 1) == 0) load_scales(q + 2, (k / 2 + 1) % 2);
+        load(q + 2, (k + 2) % 3);
+        if (2 * (q0 + q) + p < steps_all) {  // the last pair may have one step
+            const uint8_t* const d = lds + (k % 3) * S::kBuf + rd;
+            const uint8_t* const s = lds + 3 * S::kBuf + ((k / 2) % 2) * S::kScale + 16 * c + 8 * (k & 1) + 4 * p + g;
+            v4u x[FM], w[FN];
+            int sx[FM], sw[FN];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                w[j] = *reinterpret_cast<const v4u*>(d + 128 * (wrow + 16 * j));
+                sw[j] = s[16 * (64 + 32 * h + 16 * j)];
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                x[i] = *reinterpret_cast<const v4u*>(d + 128 * 16 * i);
+                sx[i] = s[16 * 16 * i];
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wide8(x[i]), wide8(w[j]), acc[i][j], 4, 4, 0, sx[i],
+                                                                                 0, sw[j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int q = 0;
+    for (; q + 12 <= nq; q += 12) static_for<12>([&](auto kc) { pair(q + decltype(kc)::value, kc); });
+    static_for<12>([&](auto kc) {
+        if (q + decltype(kc)::value < nq) pair(q + decltype(kc)::value, kc);
+    });
+
+    // the two groups' partial tiles -> LDS -> y or the split-K partials
+    wait_vmcnt<0>();
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[(p * BM + 16 * i + 4 * g + r) * S::kPitch + 32 * h + 16 * j + c] = acc[i][j][r];
+    __syncthreads();
+    float* part = out.part ? out.part + (size_t)blockIdx.y * splitk_stride(out.M, out.N) : nullptr;
+    const bool vec = out8_vector_ok<YT>(out, part);
+    for (int u = tid; u < BM * 16; u += 512) {
+        const int row = u >> 4, col = (u & 15) * 8;
+        if (m0 + row >= a.M) continue;
+        const float* src = red + row * S::kPitch + col;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const float4 s0 = *reinterpret_cast<const float4*>(src + e);
+            const float4 s1 = *reinterpret_cast<const float4*>(src + BM * S::kPitch + e);
+            v[e] = s0.x + s1.x; v[e + 1] = s0.y + s1.y; v[e + 2] = s0.z + s1.z; v[e + 3] = s0.w + s1.w;
+        }
+        store_out8<YT>(out, part, vec, m0 + row, n0 + col, v);
+    }
+}
+
+template <int FM>
+void launch_mxfp4_mid(MxArgs a, GemmArgs out) {
+    a.tiles_m = (a.M + 16 * FM - 1) / (16 * FM);
+    a.tiles = a.tiles_m * ((a.N + 127) / 128);
+    a.per_xcd = (a.tiles + kXcds - 1) / kXcds;
+    // K split, in units of four steps, so that the grid holds up to two blocks per CU
+    const int units = (a.K / KSTEP + 3) / 4;
+    const int splits = choose_split(out, a.tiles, units, 1, env_int("BYHIP_MX_SPLIT", mx_mid_splits(a.tiles, units)), 1);
+    if (splits == 1) out.part = nullptr;
+    const dim3 grid(kXcds * a.per_xcd, splits);
+    switch (out.y_dtype) {
+    case BYHIP_F32: launch("mxfp4_gemm_mid", (mxfp4_gemm_mid<FM, BYHIP_F32>), grid, dim3(512), 0, a, out); break;
+    case BYHIP_F16: launch("mxfp4_gemm_mid", (mxfp4_gemm_mid<FM, BYHIP_F16>), grid, dim3(512), 0, a, out); break;
+    default: launch("mxfp4_gemm_mid", (mxfp4_gemm_mid<FM, BYHIP_BF16>), grid, dim3(512), 0, a, out); break;
+    }
+    BYHIP_LAUNCHED("mxfp4_gemm_mid");
+    if (out.part) launch_splitk_sum(out, splits);
+}
+
 }  // namespace
 
 void launch_mxfp4(const uint8_t* x, const uint8_t* x_scales, const uint8_t* w,
@@ -382,6 +580,17 @@ void launch_mxfp4(const uint8_t* x, const uint8_t* x_scales, const uint8_t* w,
     MxArgs a;
     a.x = x; a.xs = x_scales; a.w = w; a.ws = w_scales; a.y = y;
     a.M = M; a.K = K; a.N = N;
+    if (const int fm = mx_mid(M, K, N)) {
+        GemmArgs out;
+        out.y = y; out.y_dtype = y_dtype; out.M = M; out.N = N; out.K = K;
+        switch (fm) {
+        case 1: launch_mxfp4_mid<1>(a, out); break;
+        case 2: launch_mxfp4_mid<2>(a, out); break;
+        case 3: launch_mxfp4_mid<3>(a, out); break;
+        default: launch_mxfp4_mid<4>(a, out); break;
+        }
+        return;
+    }
     a.tiles_m = (M + TM - 1) / TM;
     a.tiles = a.tiles_m * ((N + TN - 1) / TN);
     a.per_xcd = (a.tiles + kXcds - 1) / kXcds;
