@@ -78,20 +78,21 @@ bool table_products_are_halves(const float* t) {
     return ok;
 }
 
-// The route of a decode table: kTableE2m1 when its 16 values are E2M1's bit for bit (gemm_planes),
+// The route of a decode table: kTableE2m1 when its 16 values are E2M1's bit for bit (gemm_planes, fp4_gemv),
 // else kTableHalves when every product is a half, else kTableAny.
 enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2 };
 
 bool table_is_e2m1(const float* t) { return memcmp(t, kE2M1, sizeof kE2M1) == 0; }
 
 // Device-side form of the choice: thread b checks the 16 products with scale entry b (finite, and
-// exact in fp16), and the block's AND goes to *flag; `planes`: whether gemm_planes takes the call.
-__global__ __launch_bounds__(256) void fp4km_classify(const float* __restrict__ t, int planes, int* flag) {
+// exact in fp16), and the block's AND goes to *flag; `e2m1_route`: whether a kernel for E2M1's values
+// takes the call.
+__global__ __launch_bounds__(256) void fp4km_classify(const float* __restrict__ t, int e2m1_route, int* flag) {
     constexpr uint32_t e2m1[16] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u,
                                    0x40C00000u, 0x80000000u, 0xBF000000u, 0xBF800000u, 0xBFC00000u, 0xC0000000u,
                                    0xC0400000u, 0xC0800000u, 0xC0C00000u};
     const float s = t[16 + threadIdx.x];
-    bool ok = true, same = planes != 0;
+    bool ok = true, same = e2m1_route != 0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const float p = t[i] * s;
@@ -132,7 +133,7 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
     GemmArgs a;
     a.x = x; a.x_dtype = x_dtype; a.y = y; a.y_dtype = y_dtype; a.M = M; a.K = K; a.N = N;
     a.blob = blob; a.scale_base = scale_base; a.lut = lut + lut_base;
-    // fp32 activations and an E2M1 table: the two-plane kernel. Else the general fp16 MFMA kernel when
+    // fp32 activations and an E2M1 table: the decode GEMV for one row, else the two-plane kernel. Else the general fp16 MFMA kernel when
     // every decoded weight is a half, otherwise the exact fp32 GEMM. The table is classified on the
     // host from its host copy, outside recordings; otherwise on the device, by a kernel that writes
     // the choice to a flag, with all routes queued behind it and each gated on the flag, so that a
@@ -140,11 +141,15 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
     // waits for the device to read the table.
     const bool aligned = reinterpret_cast<uintptr_t>(blob) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
     if (aligned && env_int("BYHIP_TILE_EXACT", 0) == 0) {
-        const bool planes = gemm_planes_ok(BFormat::Fp4Km, a);
+        const bool gemv = fp4_gemv_ok(a), e2m1 = gemv || gemm_planes_ok(BFormat::Fp4Km, a);
+        auto launch_e2m1 = [&](const GemmArgs& g) {
+            if (gemv) launch_fp4_gemv(g);
+            else launch_gemm_planes(BFormat::Fp4Km, g);
+        };
         float t[272];
         if (!session_recording() && mirror_read(lut, lut_base * 4, t, sizeof t)) {
-            if (planes && table_is_e2m1(t)) {
-                launch_gemm_planes(BFormat::Fp4Km, a);
+            if (e2m1 && table_is_e2m1(t)) {
+                launch_e2m1(a);
                 return;
             }
             if (table_products_are_halves(t)) {
@@ -154,12 +159,12 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
         } else {
             int* flag = device_flags();
             launch("fp4km_classify", fp4km_classify, dim3(1), dim3(256), 0, static_cast<const float*>(lut + lut_base),
-                   (int)planes, flag);
+                   (int)e2m1, flag);
             GemmArgs g = a;
             g.gate = flag;
-            if (planes) {
+            if (e2m1) {
                 g.gate_want = kTableE2m1;
-                launch_gemm_planes(BFormat::Fp4Km, g);
+                launch_e2m1(g);
             }
             g.gate_want = kTableHalves;
             launch_gemm(BFormat::Fp4Km, g);

@@ -189,6 +189,16 @@ void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
 
+// The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, a table with E2M1's values
+// and any scales, K % 32 == 0 up to 15,360.
+bool fp4_gemv_ok(const GemmArgs& a);
+void launch_fp4_gemv(const GemmArgs& a);
+
+// The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, a table with E2M1's values
+// and any scales, K % 32 == 0 up to 15,360.
+bool fp4_gemv_ok(const GemmArgs& a);
+void launch_fp4_gemv(const GemmArgs& a);
+
 // Native MXFP4 GEMM (E2M1 x E2M1 with E8M0 block scales): x and w in the FP4-KM packing.
 // K % 128 == 0 is required.
 void launch_mxfp4(const uint8_t* x, const uint8_t* x_scales, const uint8_t* w,

@@ -113,3 +113,24 @@ def test_f16_planes(hip, oracle, M, K, N):
     hip.f16_tile_gemm(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.DeviceBuffer.from_array(w.reshape(-1)), y, hip.F32,
                       M, K, N)
     ref_check(y.read(np.float32), want)
+
+
+@pytest.mark.parametrize("scales", ["ref", "mx", "edge"])
+@pytest.mark.parametrize("K,N", [(32, 1), (96, 9), (2048, 65), (2080, 16), (4096, 130), (6176, 7), (8224, 24), (15360, 17), (15392, 17)])
+def test_fp4km_decode_row(hip, oracle, K, N, scales):
+    """One row at each count of groups per lane, past the decode GEMV's K, and with inf and NaN."""
+    x, blob, t = fp4_case(1, K, N, scales, K + N)
+    for mirror in (True, False):
+        want = oracle.tile_gemm(0, 1, K, N, N * (K // 2), 0, blob, t, x)
+        ref_check(run_fp4(hip, x, blob, t, 1, K, N, mirror), want)
+    if scales == "mx":
+        blob[N * (K // 2) + K // 32 - 1] = 255  # row 0's last group: an infinite scale
+        want = np.asarray(oracle.tile_gemm(0, 1, K, N, N * (K // 2), 0, blob, t, x)).reshape(-1)
+        got = run_fp4(hip, x, blob, t, 1, K, N, True)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ref_check(got[np.isfinite(want)], want[np.isfinite(want)])
+        x[0, K - 1] = np.inf
+        want = np.asarray(oracle.tile_gemm(0, 1, K, N, N * (K // 2), 0, blob, t, x)).reshape(-1)
+        got = run_fp4(hip, x, blob, t, 1, K, N, True)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.isinf(got), np.isinf(want))
