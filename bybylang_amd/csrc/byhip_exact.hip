@@ -187,6 +187,152 @@ __global__ __launch_bounds__(256) void gemm_f32_exact(GemmArgs a) {
         }
 }
 
+// The same arithmetic for Q4 weights in whole 128-value steps (groups of 32 2^j values, or one per
+// row), with loads in flight beside the math: 16 FM rows x 128 columns per block, eight waves, wave w
+// owning columns 16 w .. 16 w + 15 and all rows.
+//   A step is 128 values: lane (c, g) = (lane % 16, lane / 16) takes the step's 32-value chunk g of
+//   column c, one 16-byte load and one scale and zero, and supplies position 32 g + t in MFMA t
+//   (0 .. 31). Activations move straight into LDS (2 rows of 512 bytes per load, whole lines; 16-byte
+//   chunk k of row r at slot k ^ (r % 16), so the 16 rows of a fragment read hit distinct banks),
+//   three buffers, loads two steps ahead, one barrier per step.
+//   What bounds it: a launch's ramp and the split-K sum at few rows, the fp32 MFMAs with more.
+//   Group 32, fp32 scales and zeros (us with the sum, gemm_f32_exact / here): K = N = 4096 M = 16
+//   26.7 / 13.3, M = 64 60.0 / 28.1; K = N = 8192, M = 64 204.8 / 77.4; K = 2048, N = 600, M = 33 19.5 / 13.0.
+constexpr int kRStep = 128;
+
+template <int FM>
+struct RowsShape {
+    static constexpr int kBM = 16 * FM, kBN = 128;
+    static constexpr int kBuf = kBM * kRStep * 4;
+};
+
+template <int FM, bool ZU>
+__global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) {
+    using S = RowsShape<FM>;
+    constexpr int kLoads = FM + 2 + (ZU ? 0 : 1);  // per wave and step
+    __shared__ __attribute__((aligned(16))) uint8_t lds[3 * S::kBuf];
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * S::kBN, m0 = blockIdx.y * S::kBM, n = n0 + 16 * wid + c;
+    const int total = a.K / kRStep;
+    const int s_first = a.part ? (int)blockIdx.z * a.split_steps : 0;
+    const int nt = a.part ? min(a.split_steps, total - s_first) : total;
+    const int gshift = a.group ? 31 - __builtin_clz((uint32_t)a.group >> 5) : 0;  // chunks per group, log2
+
+    // Rows past M and columns past N read zeros through the range checks.
+    const rsrc_t xr = make_rsrc(a.x, (uint32_t)((size_t)a.M * a.K * 4));
+    const rsrc_t wr = make_rsrc(a.wq, (uint32_t)((size_t)a.N * a.row_bytes));
+    const rsrc_t sr = make_rsrc(a.scales, (uint32_t)((size_t)a.N * a.gpr * 4));
+    const rsrc_t zr = make_rsrc(ZU ? a.scales : (const void*)a.zeros, ZU ? 0u : (uint32_t)((size_t)a.N * a.gpr * 4));
+    // direct load q of wave w: rows 2 (FM w + q) and the next one
+    uint32_t xo[FM];
+#pragma unroll
+    for (int q = 0; q < FM; ++q) {
+        const int r = 2 * (FM * wid + q) + (lane >> 5);
+        xo[q] = (uint32_t)(m0 + r) * (uint32_t)a.K * 4u + 16u * (uint32_t)((lane & 31) ^ (r & 15));
+    }
+    const uint32_t wo = (uint32_t)n * (uint32_t)a.row_bytes + 16u * (uint32_t)g;
+    const uint32_t so = (uint32_t)n * (uint32_t)a.gpr * 4u;
+    struct W {
+        v4u q;
+        uint32_t s, z;
+    };
+    auto load = [&](W& w, int t, int buf) __attribute__((always_inline)) {
+        const bool ok = t < nt;
+        const uint32_t u = (uint32_t)(s_first + (ok ? t : 0)), past = ok ? 0u : 0x80000000u;
+        w.q = __builtin_amdgcn_raw_buffer_load_b128(wr, wo, past + 64u * u, 0);
+        const uint32_t grp = a.group ? (4u * u + (uint32_t)g) >> gshift : 0u;
+        w.s = __builtin_amdgcn_raw_buffer_load_b32(sr, so + 4u * grp, past, 0);
+        if constexpr (!ZU) w.z = __builtin_amdgcn_raw_buffer_load_b32(zr, so + 4u * grp, past, 0);
+#pragma unroll
+        for (int q = 0; q < FM; ++q) lds_dma16(xr, lds + buf * S::kBuf + 1024 * (FM * wid + q), xo[q], past + 512u * u);
+    };
+
+    f4 acc[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) acc[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    W w[3];
+    load(w[0], 0, 0);
+    load(w[1], 1, 1);
+    auto step = [&](int t, auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+        wait_vmcnt<kLoads>();  // the loads of step t + 1 may stay in flight
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        load(w[(k + 2) % 3], t + 2, (k + 2) % 3);
+        const float s = __builtin_bit_cast(float, w[k].s), z = ZU ? a.zero_value : __builtin_bit_cast(float, w[k].z);
+        const uint8_t* const x = lds + k * S::kBuf + 512 * c;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const uint32_t even = w[k].q[d] & 0x0F0F0F0Fu, odd = (w[k].q[d] >> 4) & 0x0F0F0F0Fu;
+            float wf[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                wf[2 * e] = ((float)((even >> (8 * e)) & 255u) - z) * s;
+                wf[2 * e + 1] = ((float)((odd >> (8 * e)) & 255u) - z) * s;
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                // chunks 8 g + 2 d and the next one of row 16 i + c (read as compiler vectors: before
+                // HIP's float4 the compiler waits for every direct load in flight)
+                const f4 x0 = *reinterpret_cast<const f4*>(x + 8192 * i + 16 * ((8 * g + 2 * d) ^ c));
+                const f4 x1 = *reinterpret_cast<const f4*>(x + 8192 * i + 16 * ((8 * g + 2 * d + 1) ^ c));
+                const float xv[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[e], wf[e], acc[i], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int t = 0;
+    for (; t + 3 <= nt; t += 3) static_for<3>([&](auto kc) { step(t + decltype(kc)::value, kc); });
+    static_for<2>([&](auto kc) {
+        if (t + decltype(kc)::value < nt) step(t + decltype(kc)::value, kc);
+    });
+    wait_vmcnt<0>();
+
+    float* part = a.part ? a.part + (size_t)blockIdx.z * splitk_stride(a.M, a.N) : nullptr;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + 16 * i + 4 * g + r;
+            if (m < a.M && n < a.N) {
+                if (part) part[(size_t)m * a.N + n] = acc[i][r];
+                else store_any(a.y, a.y_dtype, (size_t)m * a.N + n, acc[i][r]);
+            }
+        }
+}
+
+template <int FM>
+void launch_f32_q4_fm(const GemmArgs& a, dim3 grid) {
+    if (a.zeros) launch("gemm_f32_q4", (gemm_f32_q4<FM, false>), grid, dim3(512), 0, a);
+    else launch("gemm_f32_q4", (gemm_f32_q4<FM, true>), grid, dim3(512), 0, a);
+    BYHIP_LAUNCHED("gemm_f32_q4");
+}
+
+// K splits: as many as leave one block per CU, each of at least two steps (K = N = 4096, M = 16, 4 / 8 /
+// 16 splits: 18.3 / 13.4 / 14.6 us).
+void launch_f32_q4(GemmArgs a) {
+    const int row_tiles = (a.M + 63) / 64, fm = (a.M + 16 * row_tiles - 1) / (16 * row_tiles);
+    const int rows = (a.M + 16 * fm - 1) / (16 * fm);
+    const long tiles = (long)((a.N + 127) / 128) * rows;
+    const int steps = a.K / kRStep;
+    const int forced = env_int("BYHIP_Q4_SPLIT", 0);
+    const int want = (int)std::max<long>(1, std::min<long>(compute_units() / tiles, steps / 2));
+    const int splits = choose_split(a, tiles, steps, 1, forced > 0 ? forced : want, 1);
+    if (splits == 1) a.part = nullptr;
+    const dim3 grid((unsigned)((a.N + 127) / 128), (unsigned)rows, (unsigned)splits);
+    switch (fm) {
+    case 1: launch_f32_q4_fm<1>(a, grid); break;
+    case 2: launch_f32_q4_fm<2>(a, grid); break;
+    case 3: launch_f32_q4_fm<3>(a, grid); break;
+    default: launch_f32_q4_fm<4>(a, grid); break;
+    }
+    if (a.part) launch_splitk_sum(a, splits);
+}
+
 template <BFormat F, bool XF32>
 void launch_exact_bm(const GemmArgs& a, int bm, dim3 grid) {
     switch (bm) {
@@ -205,11 +351,23 @@ void launch_exact_x(const GemmArgs& a, int bm, dim3 grid) {
 
 }  // namespace
 
+bool gemm_f32_q4_ok(const GemmArgs& a) {
+    constexpr uint64_t kLim = 0x80000000u;
+    const int chunks = a.group >> 5;
+    return a.x_dtype == BYHIP_F32 && !a.scale_f16 && a.K % kRStep == 0 &&
+           (a.group == 0 || (a.group % 32 == 0 && (chunks & (chunks - 1)) == 0)) &&
+           reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.wq) % 16 == 0 && a.row_bytes % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(a.scales) % 4 == 0 && reinterpret_cast<uintptr_t>(a.zeros) % 4 == 0 &&
+           (uint64_t)(a.M + 64) * a.K * 4 < kLim && (uint64_t)(a.N + 128) * a.row_bytes < kLim &&
+           (uint64_t)(a.N + 128) * a.gpr * 4 < kLim;
+}
+
 void launch_gemm_exact(BFormat fmt, const GemmArgs& a0) {
     GemmArgs a = a0;
     if (a.M <= 0 || a.N <= 0 || a.K <= 0) return;
     if (fmt != BFormat::Q4Fast && fmt != BFormat::Q4Generic && a.K % 32 != 0)
         fail("byhip: internal: the exact FP4-KM / F16 GEMM needs K %% 32 == 0 (K=%d)", a.K);
+    if ((fmt == BFormat::Q4Fast || fmt == BFormat::Q4Generic) && gemm_f32_q4_ok(a)) return launch_f32_q4(a);
     const int bm = a.M <= 16 ? 16 : (a.M <= 32 ? 32 : 64);
     if ((a.M + bm - 1) / bm > 65535) fail("byhip: M=%d too large for one launch", a.M);
     const long tiles = (long)((a.N + 63) / 64) * ((a.M + bm - 1) / bm);

@@ -161,6 +161,9 @@ bool launch_q4_wide_exact_weights(const GemmArgs& a);
 // F16 halves), fp32 activations as they are (fp16 widened), fp32 products and accumulation in
 // v_mfma_f32_16x16x4_f32. Any K (Q4; FP4-KM and F16 need K % 32 == 0), M, N.
 void launch_gemm_exact(BFormat fmt, const GemmArgs& a);
+// Whether launch_gemm_exact(Q4) takes the pipelined kernel (gemm_f32_q4): fp32 activations and scales,
+// K % 128 == 0, groups of 32 2^j values or one per row, 16-byte aligned rows, offsets below 2^31.
+bool gemm_f32_q4_ok(const GemmArgs& a);
 
 // The Q4 GEMM kernels by explicit choice (a tuned plan's candidates): kQ4Pipe, the LDS-staged
 // pipelined kernel with `tile` 1..4 (64x128, 64x64, 32x128, 32x64) and `splits`; kQ4Skinny (M <= 32,

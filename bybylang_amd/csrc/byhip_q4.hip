@@ -460,6 +460,10 @@ void q4_matmul_impl(const void* x, int x_dtype, const byhip_q4w* w, void* y, int
             launch_q4_wide_exact_weights(ga))
             return;
     }
+    // fp32 scales (micro-VM slots, weights outside fp16's range) have no wide tile: from three rows on the
+    // pipelined fp32 GEMM, whose time barely moves with the rows, where the GEMV's grows (K = N = 4096,
+    // M = 1 / 2 / 4 / 8: GEMV 6.0 / 8.7 / 17.3 / 34.6 us, GEMM 11.6 / 12.0 / 12.1 / 12.4).
+    if (mode == 0 && M > 2 && M <= 8 && aligned && gemm_f32_q4_ok(ga)) return launch_gemm_exact(BFormat::Q4Generic, ga);
     if (gemv && (mode == 1 || (mode == 0 && M <= 8)))
         return launch_q4_gemv(x, x_dtype, w, y, y_dtype, M, work, work_bytes);
     // Decode shapes the GEMV does not take (K or the group not a multiple of 32, unaligned rows or

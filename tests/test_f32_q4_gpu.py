@@ -1,0 +1,54 @@
+"""The pipelined fp32 GEMM for Q4 weights with fp32 scales (micro-VM slots, weights outside fp16's
+range) on the MI355X against the oracle, at the edges of its tiles, steps and splits.
+
+Bar: the reference test's tolerance; the arithmetic is fp32 as in the reference.
+"""
+import numpy as np
+import pytest
+
+from oracle_lib import OP_Q4_COOP_GEMM, q4_blob, shape_op_program
+from parity import ref_check
+
+pytestmark = pytest.mark.gpu
+
+
+def slots(seed, M, K, N, group, spread):
+    from bybylang_amd import synth
+    g = synth.rng(seed)
+    ng = K // group
+    wq, _, _, _ = synth.q4_weights(g, N, K, group)
+    sc = (g.standard_normal(N * ng) * 0.02).astype(np.float32)
+    if spread:
+        sc *= (10.0 ** g.uniform(-6, 6, N * ng)).astype(np.float32)
+    ze = (8 + g.standard_normal(N * ng)).astype(np.float32)
+    return synth.activations(g, M, K, np.float32), wq, sc, ze
+
+
+@pytest.mark.parametrize("spread", [False, True])
+@pytest.mark.parametrize("M,K,N,group", [(3, 128, 16, 32), (8, 256, 130, 64), (16, 640, 127, 128), (17, 1024, 40, 32), (48, 384, 300, 32),
+                                         (64, 2048, 128, 256), (65, 512, 136, 512), (130, 896, 72, 128)])
+@pytest.mark.parametrize("splits", [0, 3])
+def test_f32_q4_program(hip, oracle, monkeypatch, M, K, N, group, spread, splits):
+    x, wq, sc, ze = slots(M + K, M, K, N, group, spread)
+    if splits:
+        monkeypatch.setenv("BYHIP_Q4_SPLIT", str(splits))
+    by, fl = q4_blob(wq, sc, ze, K, N, K // group)
+    mem = hip.DeviceBuffer(M * N * 4)
+    hip.program_dispatch(shape_op_program(OP_Q4_COOP_GEMM, M, K, N, group, K // group), mem, hip.DeviceBuffer.from_array(by),
+                         hip.DeviceBuffer.from_array(fl), hip.DeviceBuffer.from_array(x.reshape(-1)))
+    want = oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, K // group)
+    ref_check(mem.read(np.float32), want)
+
+
+@pytest.mark.parametrize("M,K,N,group,zeros", [(5, 256, 40, 0, "one"), (20, 1152, 130, 32, "one"), (40, 512, 100, 0, "group")])
+def test_f32_q4_resident(hip, oracle, M, K, N, group, zeros):
+    """Resident weights outside fp16's range: one zero for all, or one per group; one group per row."""
+    x, wq, sc, ze = slots(M, M, K, N, group or K, True)
+    if zeros == "one":
+        ze[:] = 7.5
+    w = hip.Q4Weights(wq, sc, ze, K, N, group, K // group if group else 1)
+    assert not w.info()["f16_safe"]
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, w, y, hip.F32, M)
+    want = oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, K // group if group else 1)
+    ref_check(y.read(np.float32), want)
