@@ -254,6 +254,7 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
     for (int i = 0; i < FM; ++i) acc[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     W w[3];
     load(w[0], 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // the first wait counts on this order
     load(w[1], 1, 1);
     auto step = [&](int t, auto kc) __attribute__((always_inline)) {
         constexpr int k = decltype(kc)::value;

@@ -1095,6 +1095,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
         constexpr int k = decltype(kc)::value;
         load_x(k, k);
         load_ws(rs[k], k);
+        __builtin_amdgcn_sched_barrier(0);  // the wait below counts on this order
     });
     wait_vmcnt<(D - 2) * kLoads>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -1362,6 +1363,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_tall(GemmArgs a) {
         constexpr int k = decltype(kc)::value;
         load_x(k, k);
         load_ws(rs[k], k);
+        __builtin_amdgcn_sched_barrier(0);  // the wait below counts on this order
     });
     wait_vmcnt<(D - 2) * kTallLoads>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

@@ -479,6 +479,7 @@ __global__ __launch_bounds__(512, 4) void mxfp4_gemm_mid(MxArgs a, GemmArgs out)
 
     load_scales(0, 0);
     load(0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // the first wait counts on this order
     load(1, 1);
     // Pair q = base + k: the wait leaves the loads of pair q + 1 in flight (with the scales issued
     // beside them, for odd q); the barrier publishes every wave's lines of pair q and frees the buffer

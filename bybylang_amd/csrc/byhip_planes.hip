@@ -287,6 +287,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         constexpr int k = decltype(kc)::value;
         load_w(wv[k], k);
         load_x(k, k);
+        __builtin_amdgcn_sched_barrier(0);  // the wait below counts on this order
     });
     if constexpr (FP4) {
         uint32_t b[4];
