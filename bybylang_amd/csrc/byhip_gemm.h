@@ -168,10 +168,11 @@ bool gemm_f32_q4_ok(const GemmArgs& a);
 // The Q4 GEMM kernels by explicit choice (a tuned plan's candidates): kQ4Pipe, the LDS-staged
 // pipelined kernel with `tile` 1..4 (64x128, 64x64, 32x128, 32x64) and `splits`; kQ4Skinny (M <= 32,
 // `splits`); kQ4General, the general LDS-staged kernel; kQ4Big, the 128 x 256 prefill tile, and
-// kQ4Wide, the 64 x 128 skinny tile (`splits`); kQ4Stream, the small-M streaming GEMM (`splits`).
+// kQ4Wide, the 64 x 128 skinny tile (`splits`); kQ4Stream, the small-M streaming GEMM (`splits`);
+// kQ4Planes, the two-plane GEMM on fp32 activations.
 // tile / splits 0 keep the default choice.
 // Returns false, queueing nothing, when that kernel does not take the call.
-enum { kQ4Pipe = 1, kQ4Skinny = 2, kQ4General = 3, kQ4Big = 4, kQ4Wide = 5, kQ4Stream = 6 };
+enum { kQ4Pipe = 1, kQ4Skinny = 2, kQ4General = 3, kQ4Big = 4, kQ4Wide = 5, kQ4Stream = 6, kQ4Planes = 7 };
 bool launch_q4_choice(BFormat fmt, const GemmArgs& a, int kind, int tile, int splits);
 
 // The small-M streaming Q4 GEMM (q4_gemm_stream): up to 32 rows of fp16 activations on weights

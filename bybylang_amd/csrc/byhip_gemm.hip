@@ -1863,6 +1863,10 @@ bool launch_q4_choice(BFormat fmt, const GemmArgs& a, int kind, int tile, int sp
         if (fmt != BFormat::Q4Fast || !q4_stream_ok(a)) return false;
         launch_q4_stream(a, splits);
         return true;
+    case kQ4Planes:
+        if (fmt != BFormat::Q4Fast || !gemm_planes_ok(fmt, a)) return false;
+        launch_gemm_planes(fmt, a);
+        return true;
     case kQ4General:
         if (fmt == BFormat::Q4Fast && !a.zeros) launch_f<BFormat::Q4Fast>(a);
         else if (fmt == BFormat::Q4Fast || fmt == BFormat::Q4Generic) launch_f<BFormat::Q4Generic>(a);
@@ -1899,6 +1903,20 @@ void launch_gemm(BFormat fmt, const GemmArgs& a) {
     switch (fmt) {
     case BFormat::Q4Fast:
         // fp32 activations: the wide tile on two fp16 planes where the scratch holds them
+        // fp32 activations: the two-plane kernel (two MFMAs per product) when its 64 x 128 tiles fill half
+        // the CUs, else the 16- or 32-row wide tile (three, but twice the blocks) where the scratch holds
+        // its planes. us, wide / planes: K = N = 4096, M = 64 18.3 / 22.7, 128 24.3 / 25.0, 256 32.2 / 32.2,
+        // 300 45.5 / 33.3, 512 58.1 / 44.9; K = 4096, N = 14336, M = 64 25.3 / 26.4, 128 46.6 / 37.2, 509
+        // 176.7 / 152.4; K = 14336, N = 4096, M = 256 82.4 / 69.0; K = N = 1024, M = 700 13.5 / 17.2.
+        // BYHIP_Q4_PLANES=0 / 1 leaves every call to the wide tile / gives the planes every call.
+        if (q4_f32_wide_takes(a) && gemm_planes_ok(fmt, a)) {
+            const int forced = env_int("BYHIP_Q4_PLANES", -1);
+            const long tiles = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
+            if (forced == 1 || (forced < 0 && 2 * tiles >= compute_units())) {
+                launch_gemm_planes(fmt, a);
+                break;
+            }
+        }
         if (q4_f32_wide_takes(a) && launch_q4_wide_f32(a)) break;
         if (q4_stream_takes(a)) {
             launch_q4_stream(a);

@@ -8,6 +8,9 @@
 //          while it is used; a block that meets another scale, or a table that is not E2M1,
 //          computes its tile again in fp32 arithmetic as the reference does)
 //   F16
+//   Q4     on the prefill copy: the codes less their zero (whole numbers) go through the MFMAs, and each
+//          32-value group's sums are scaled in fp32. Two MFMAs per product where weights as two fp16
+//          terms (the wide tile on fp32 activations) take three.
 //
 // Block: 16 FM rows x 128 columns, eight waves, two per SIMD. Waves w, w + 2, .. (p = w % 2) form K
 // group p, which takes every other 128-value step of the block; wave h = w / 2 of the group owns
@@ -20,6 +23,10 @@
 // k ^ x_swizzle(r), four buffers, loads three sub-steps ahead. Lane (c, g) = (lane % 16, lane / 16)
 // multiplies chunks 2 g and 2 g + 1 of the slice with its weights of column c:
 //   F16     16 halves of the weight row, in natural order
+//   Q4      chunks g and 4 + g instead: MFMA kk then covers one 32-value group, positions 32 kk + 8 g ..
+//           + 7 per lane, one dword of the prefill copy (a fragment's 64 dwords are 256 contiguous
+//           bytes). Its sums wait in registers of their own and are scaled and added during the next K
+//           half's MFMAs, which start from zero.
 //   FP4-KM  the four lane groups hold the step's four 32-value groups, one 16-byte load per column
 //           and step: bytes 4 q .. 4 q + 3 of the group are elements 4 q .. 4 q + 3 (low nibbles)
 //           and 16 + 4 q .. (high); sub-step e multiplies q = 2 e and 2 e + 1. split_planes writes the
@@ -113,11 +120,12 @@ __device__ __forceinline__ void fp4_tile_exact(const GemmArgs& a, int m0, int n0
         }
 }
 
-template <BFormat F, int FM, int YT>
+template <BFormat F, int FM, int YT, bool ZG = false>
 __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 4 : 2) void gemm_planes(GemmArgs a) {
     if (a.gate && *a.gate != a.gate_want) return;  // another route was chosen (whole grid)
-    constexpr bool FP4 = F == BFormat::Fp4Km;
+    constexpr bool FP4 = F == BFormat::Fp4Km, Q4 = F == BFormat::Q4Fast;
     constexpr int FN = 2;
+    constexpr int WV = FP4 ? FN : Q4 ? 2 : 2 * FN;  // weight registers of a set, in 16-byte units
     using S = PlaneShape<FM>;
     constexpr int BM = S::kBM, kXBuf = S::kXBuf;
     // One LDS array for everything, the eight waves' `bad` words at its end: beside a second array (a
@@ -159,9 +167,15 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     }
 
     const rsrc_t xr = make_rsrc(h < 2 ? a.x : a.x_lo, (uint32_t)((size_t)a.M * K * 2));
-    const rsrc_t wr = FP4 ? make_rsrc(a.blob, (uint32_t)((size_t)a.N * (K >> 1)))
-                          : make_rsrc(a.w16, (uint32_t)((size_t)a.N * K * 2));
-    const rsrc_t sr = FP4 ? make_rsrc(a.blob + a.scale_base, (uint32_t)((size_t)a.N * (K >> 5))) : wr;
+    const uint32_t nsub = (uint32_t)K / kSub;
+    const uint32_t wpf_bytes = ((uint32_t)a.N + 15) / 16 * nsub * 512, spf_bytes = ((uint32_t)a.N + 63) / 64 * nsub * 256;
+    const rsrc_t wr = FP4  ? make_rsrc(a.blob, (uint32_t)((size_t)a.N * (K >> 1)))
+                      : Q4 ? make_rsrc(a.wpf, wpf_bytes)
+                           : make_rsrc(a.w16, (uint32_t)((size_t)a.N * K * 2));
+    const rsrc_t sr = FP4  ? make_rsrc(a.blob + a.scale_base, (uint32_t)((size_t)a.N * (K >> 5)))
+                      : Q4 ? make_rsrc(a.spf, spf_bytes)
+                           : wr;
+    const rsrc_t zr = ZG ? make_rsrc(a.zpf, spf_bytes) : sr;
     // Direct load q (0 .. FM - 1) of wave h: stacked rows 8 FM h + 8 q + lane / 8 of the slice (the
     // high plane's BM rows, then the low plane's), LDS slot lane % 8.
     uint32_t xo[FM];
@@ -176,11 +190,16 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     for (int j = 0; j < FN; ++j) {
         const int n = n0 + 32 * h + 16 * j + c;
         col_ok[j] = n < a.N;
-        wo[j] = FP4 ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g : (uint32_t)n * (uint32_t)K * 2u + 32u * g;
+        wo[j] = FP4  ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g
+                : Q4 ? ((uint32_t)n >> 4) * nsub * 512u + 8u * c + 128u * (uint32_t)(g >> 1) + 4u * (uint32_t)(g & 1)
+                     : (uint32_t)n * (uint32_t)K * 2u + 32u * g;
         so[j] = (uint32_t)n * (uint32_t)(K >> 5) + 8u * g;
     }
+    // Q4 scales (and zeros): the wave's 2 fragments are fragments 2 (h % 2) and the next of their quad
+    const uint32_t sq = (uint32_t)(n0 + 32 * h) / 64u * nsub * 256u + 8u * c + 4u * (uint32_t)(h & 1);
     uint8_t* const xgrp = lds + p * kDepth * kXBuf;
-    const int rd0 = 128 * c + 16 * ((2 * g) ^ x_swizzle(c)), rd1 = 128 * c + 16 * ((2 * g + 1) ^ x_swizzle(c));
+    const int rd0 = 128 * c + 16 * ((Q4 ? g : 2 * g) ^ x_swizzle(c));
+    const int rd1 = 128 * c + 16 * ((Q4 ? 4 + g : 2 * g + 1) ^ x_swizzle(c));
 
     // The group's sub-step t is slice 2 p + 4 (t / 2) + t % 2 of the block; past the last it reads zeros.
     auto load_x = [&](int t, int buf) __attribute__((always_inline)) {
@@ -190,10 +209,21 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         for (int q = 0; q < FM; ++q) lds_dma16(xr, xgrp + buf * kXBuf + 1024 * (FM * h + q), xo[q], off);
     };
     // FP4-KM: the 16 bytes per column of the group's step q (sub-steps 2 q and 2 q + 1); F16: the
-    // sub-step's 32 bytes.
-    v4u wv[kSets][FP4 ? FN : 2 * FN];
-    auto load_w = [&](v4u (&w)[FP4 ? FN : 2 * FN], int t) __attribute__((always_inline)) {
-        if constexpr (FP4) {
+    // sub-step's 32 bytes; Q4: per MFMA kk a dword per fragment, w[kk][j], the fragments' scales
+    // w[kk][2] and zeros w[kk][3].
+    v4u wv[kSets][WV];
+    auto load_w = [&](v4u (&w)[WV], int t) __attribute__((always_inline)) {
+        if constexpr (Q4) {
+            const int sl = 2 * p + 4 * (t >> 1) + (t & 1);
+            const uint32_t u = (uint32_t)(2 * step0 + (sl < slices ? sl : 0)), past = sl < slices ? 0u : kPast;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j) w[kk][j] = __builtin_amdgcn_raw_buffer_load_b32(wr, wo[j], past + 512u * u + 256u * kk, 0);
+                w[kk][2] = __builtin_amdgcn_raw_buffer_load_b32(sr, sq, past + 256u * u + 128u * kk, 0);
+                if constexpr (ZG) w[kk][3] = __builtin_amdgcn_raw_buffer_load_b32(zr, sq, past + 256u * u + 128u * kk, 0);
+            }
+        } else if constexpr (FP4) {
             const int s = p + 2 * t;
             const uint32_t off = s < steps ? 64u * (uint32_t)(step0 + s) : kPast;
 #pragma unroll
@@ -239,11 +269,29 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
 
-    // Weights of MFMA kk of sub-step parity e.
-    auto decode = [&](const v4u (&w)[FP4 ? FN : 2 * FN], int e, int kk, h8 (&b)[FN]) __attribute__((always_inline)) {
+    const _Float16 zlo = (_Float16)(1024.0f + a.zero_value), zhi = (_Float16)(64.0f + a.zero_value);
+    uint32_t mag_lo = 0, mag_hi = 0;
+    if constexpr (Q4) {
+        asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(mag_lo));
+        asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(mag_hi));
+    }
+    // Weights of MFMA kk of sub-step parity e (Q4: q - zero, and the fragments' scales of its group).
+    auto decode = [&](const v4u (&w)[WV], int e, int kk, h8 (&b)[FN], float (&s)[FN]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            if constexpr (FP4) {
+            if constexpr (Q4) {
+                s[j] = (float)bits_h((uint16_t)(w[kk][2] >> (16 * j)));
+                h2 z0 = {zlo, zlo}, z1 = {zhi, zhi};
+                if constexpr (ZG) {
+                    const _Float16 z = bits_h((uint16_t)(w[kk][3] >> (16 * j)));
+                    z0 = (h2){z, z} + (h2){1024, 1024};
+                    z1 = (h2){z, z} + (h2){64, 64};
+                }
+                const uint32_t d = w[kk][j], d8 = d >> 8;
+                const uint4 u = make_uint4(h2_bits(bits_h2((d & 0x000F000Fu) | mag_lo) - z0), h2_bits(bits_h2((d & 0x00F000F0u) | mag_hi) - z1),
+                                           h2_bits(bits_h2((d8 & 0x000F000Fu) | mag_lo) - z0), h2_bits(bits_h2((d8 & 0x00F000F0u) | mag_hi) - z1));
+                b[j] = *reinterpret_cast<const h8*>(&u);
+            } else if constexpr (FP4) {
                 const uint32_t d = w[j][2 * e + kk];
                 const h2 s2 = bits_h2(ss[j]);
                 const uint4 u = make_uint4(h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 0) * s2),
@@ -263,7 +311,35 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
 #pragma unroll
             for (int i = 0; i < FM; ++i) x[pl][i] = *reinterpret_cast<const h8*>(src + 128 * BM * pl + 2048 * i);
     };
-    auto mfmas = [&](const h8 (&x)[2][FM], const h8 (&b)[FN]) __attribute__((always_inline)) {
+    // Q4: the group's sums of the last K half, not yet scaled, and their scales.
+    f4 sums[Q4 ? FM : 1][FN];
+    float sc[FN] = {};
+#pragma unroll
+    for (int i = 0; i < (Q4 ? FM : 1); ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) sums[i][j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    auto scale_sums = [&](int i, int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(sc[j], sums[i][j][r], acc[i][j][r]);
+    };
+    auto mfmas = [&](const h8 (&x)[2][FM], const h8 (&b)[FN], const float (&s)[FN]) __attribute__((always_inline)) {
+        if constexpr (Q4) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    scale_sums(i, j);
+                    sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[1][i], b[j], (f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[0][i], b[j], sums[i][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) sc[j] = s[j];
+            return;
+        }
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
@@ -278,10 +354,11 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     // (FP4-KM, with the next four steps' scale bytes at k = 0).
     constexpr int kXLoads = FM;
     auto issued = [](int k) constexpr {
-        return kXLoads + (FP4 ? ((k & 1) ? 0 : FN) + (k == 0 ? FN : 0) : 2 * FN);
+        return kXLoads + (FP4 ? ((k & 1) ? 0 : FN) + (k == 0 ? FN : 0) : Q4 ? 2 * (FN + 1 + ZG) : 2 * FN);
     };
 
     h8 ax0[2][FM], ax1[2][FM], bw0[FN], bw1[FN];
+    float s0[FN] = {}, s1[FN] = {};
     if constexpr (FP4) load_sb(sb, 0);
     static_for<3>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
@@ -301,14 +378,15 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         lut_h[0] = b[0] | (b[1] << 16);
         lut_h[1] = b[2] | (b[3] << 16);
     }
-    wait_vmcnt<2 * (kXLoads + (FP4 ? FN : 2 * FN))>();
+    wait_vmcnt<2 * (kXLoads + (FP4 ? FN : Q4 ? 2 * (FN + 1 + ZG) : 2 * FN))>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (FP4) scale_of(sb, 0, ss);
     read_x(0, 0, ax0);
-    decode(wv[0], 0, 0, bw0);
+    decode(wv[0], 0, 0, bw0, s0);
 
     constexpr int kMfmas = 2 * FM * FN;  // per K half
-    constexpr int kValuPerMfma = FP4 ? (FN * 9 + kMfmas - 1) / kMfmas : 1;
+    // VALU operations beside each MFMA; Q4: the first half of the MFMAs beside the scaling
+    constexpr int kValuPerMfma = FP4 ? (FN * 9 + kMfmas - 1) / kMfmas : Q4 ? 4 : 1;
     // Sub-step t = base + k. Its loads, in `wait` order: at the mid-step wait those of this and of the
     // previous sub-step may stay in flight, which leaves t + 1's activations landed.
     auto step = [&](int t, auto kc, auto guard) __attribute__((always_inline)) {
@@ -323,9 +401,9 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         if constexpr (FP4 && k == 0) load_sb(sbn, (t >> 3) + 1);
         load_x(t + 3, (k + 3) % kDepth);
         if (live) {
-            mfmas(ax0, bw0);
+            mfmas(ax0, bw0, s0);
             read_x(k % kDepth, 1, ax1);
-            decode(wv[set], e, 1, bw1);
+            decode(wv[set], e, 1, bw1, s1);
             if constexpr (FP4 && e == 1) scale_of(k == 7 ? sbn : sb, (t >> 1) + 1, sn);
 #pragma unroll
             for (int m = 0; m < kMfmas; ++m) {
@@ -344,9 +422,9 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
 #pragma unroll
                 for (int j = 0; j < FN; ++j) ss[j] = sn[j];
             }
-            mfmas(ax1, bw1);
+            mfmas(ax1, bw1, s1);
             read_x((k + 1) % kDepth, 0, ax0);
-            decode(wv[set1], e ^ 1, 0, bw0);
+            decode(wv[set1], e ^ 1, 0, bw0, s0);
 #pragma unroll
             for (int m = 0; m < kMfmas; ++m) {
                 __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);                  // one MFMA
@@ -366,6 +444,12 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     if (t < nt_all)
         static_for<kUnroll>([&](auto kc) { step(t + decltype(kc)::value, kc, std::true_type{}); });
 
+    if constexpr (Q4) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) scale_sums(i, j);
+    }
     // Partial tiles -> LDS, once every wave's loads have landed and every wave is done with the
     // buffers -> the two groups' sums -> y or the split-K partials.
     wait_vmcnt<0>();
@@ -490,36 +574,33 @@ __global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x,
     for (int i = (int)threadIdx.x + 256 * kHeld; i < nc; i += 256) split(i, r[first(i)], r[first(i) + second]);
 }
 
-template <BFormat F, int FM>
+template <BFormat F, int FM, bool ZG>
 void launch_planes_y(const GemmArgs& a, int splits) {
     const dim3 grid((a.N + kBN - 1) / kBN, (a.M + 16 * FM - 1) / (16 * FM), splits);
     switch (a.y_dtype) {
-    case BYHIP_F32: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F32>), grid, dim3(512), 0, a); break;
-    case BYHIP_F16: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F16>), grid, dim3(512), 0, a); break;
-    default: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_BF16>), grid, dim3(512), 0, a); break;
+    case BYHIP_F32: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F32, ZG>), grid, dim3(512), 0, a); break;
+    case BYHIP_F16: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_F16, ZG>), grid, dim3(512), 0, a); break;
+    default: launch("gemm_planes", (gemm_planes<F, FM, BYHIP_BF16, ZG>), grid, dim3(512), 0, a); break;
     }
     BYHIP_LAUNCHED("gemm_planes");
 }
 
-template <BFormat F>
+template <BFormat F, bool ZG = false>
 void launch_planes_fm(const GemmArgs& a, int fm, int splits) {
     switch (fm) {
-    case 1: launch_planes_y<F, 1>(a, splits); break;
-    case 2: launch_planes_y<F, 2>(a, splits); break;
-    case 3: launch_planes_y<F, 3>(a, splits); break;
-    default: launch_planes_y<F, 4>(a, splits); break;
+    case 1: launch_planes_y<F, 1, ZG>(a, splits); break;
+    case 2: launch_planes_y<F, 2, ZG>(a, splits); break;
+    case 3: launch_planes_y<F, 3, ZG>(a, splits); break;
+    default: launch_planes_y<F, 4, ZG>(a, splits); break;
     }
 }
 
-// Row fragments per tile: the fewest padded rows, the larger tile among equals.
+// Row fragments per tile: the fewest tiles of up to 64 rows, cut to the rows there are (a tile's time
+// hangs on its K more than on its rows: Q4, M = 100, K = 4096, N = 14336, 336 tiles of 48 rows 54.8 us, 224
+// of 64 rows 36.5).
 int planes_fm(int M) {
-    int best = 1, best_rows = 1 << 30;
-    for (int fm = 4; fm >= 1; --fm) {
-        const int rows = (M + 16 * fm - 1) / (16 * fm) * fm;
-        if (rows < best_rows) best = fm, best_rows = rows;
-    }
-    // small tiles read the weights once per tile: past 64 rows at least 48
-    return M > 64 ? std::max(best, 3) : best;
+    const int row_tiles = (M + 63) / 64;
+    return (M + 16 * row_tiles - 1) / (16 * row_tiles);
 }
 
 // K splits, in 128-value steps: the count that minimises rounds of blocks x (steps per split + 12)
@@ -546,7 +627,12 @@ void launch_planes_rows(const GemmArgs& a0) {
     const int forced = env_int("BYHIP_Q4_SPLIT", 0);
     const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : planes_splits(a, tiles), 1);
     if (splits == 1) a.part = nullptr;
-    launch_planes_fm<F>(a, fm, splits);
+    if constexpr (F == BFormat::Q4Fast) {
+        if (a.zeros) launch_planes_fm<F, true>(a, fm, splits);
+        else launch_planes_fm<F>(a, fm, splits);
+    } else {
+        launch_planes_fm<F>(a, fm, splits);
+    }
     if (a.part) launch_splitk_sum(a, splits);
 }
 
@@ -559,6 +645,8 @@ bool gemm_planes_ok(BFormat fmt, const GemmArgs& a) {
     if (fmt == BFormat::Fp4Km)
         return a.K % 128 == 0 && reinterpret_cast<uintptr_t>(a.blob) % 16 == 0 && a.scale_base % 4 == 0 &&
                (uint64_t)(a.N + kBN) * (a.K / 2) < kLim;
+    if (fmt == BFormat::Q4Fast)
+        return a.wpf && a.spf && (!a.zeros || a.zpf) && a.scale_f16 && a.K % kSub == 0 && (uint64_t)(a.N + kBN) * a.K / 2 < kLim;
     if (fmt == BFormat::F16)
         return a.K % kSub == 0 && reinterpret_cast<uintptr_t>(a.w16) % 16 == 0 && (uint64_t)(a.N + kBN) * a.K * 2 < kLim;
     return false;
@@ -598,6 +686,7 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
         a.work = lo + plane;
         a.work_bytes = work_bytes - shift_bytes - 2 * plane;
         if (fmt == BFormat::Fp4Km) launch_planes_rows<BFormat::Fp4Km>(a);
+        else if (fmt == BFormat::Q4Fast) launch_planes_rows<BFormat::Q4Fast>(a);
         else launch_planes_rows<BFormat::F16>(a);
     }
 }

@@ -17,7 +17,8 @@ enum Q4PlanKind : int {
     kPlanWide = 7,     // the wide tile (128 columns; 16, 32 or 64 rows)
     kPlanExact = 8,    // the exact fp32 MFMA GEMM
     kPlanStream = 9,   // the small-M streaming GEMM (M <= 32, one column strip per CU over all of K)
-    kPlanLast = kPlanStream
+    kPlanPlanes = 10,  // the two-plane GEMM (fp32 activations)
+    kPlanLast = kPlanPlanes
 };
 struct Q4Plan {
     int kind = 0;

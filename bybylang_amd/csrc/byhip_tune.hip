@@ -86,6 +86,7 @@ std::string plan_name(const Q4Plan& p) {
         snprintf(buf, sizeof buf, "wide-s%d", p.splits);
         return buf;
     case kPlanExact: return "exact";
+    case kPlanPlanes: return "planes";
     case kPlanStream:
         snprintf(buf, sizeof buf, "stream-s%d", p.splits);
         return buf;
@@ -217,6 +218,7 @@ std::vector<Candidate> candidates(int mt, int x_dtype) {
     } else {
         // fp32 activations: the wide tile on two fp16 planes keeps the fp32 tolerance
         for (int sp : {0, 1, 2, 4}) c.push_back({{kPlanWide, 0, sp}, 1e-4f});
+        c.push_back({{kPlanPlanes, 0, 0}, 1e-4f});
     }
     c.push_back({{kPlanGemm, 0, 0}, 3e-3f});
     c.push_back({{kPlanExact, 0, 0}, 1e-4f});

@@ -134,3 +134,35 @@ def test_fp4km_decode_row(hip, oracle, K, N, scales):
         got = run_fp4(hip, x, blob, t, 1, K, N, True)
         assert np.array_equal(np.isnan(got), np.isnan(want))
         assert np.array_equal(np.isinf(got), np.isinf(want))
+
+
+@pytest.mark.parametrize("zeros", ["one", "group"])
+@pytest.mark.parametrize("splits", [0, 2])
+@pytest.mark.parametrize("M,K,N,group", [(1, 64, 16, 32), (16, 192, 130, 64), (17, 256, 127, 0), (40, 1344, 264, 32), (64, 1024, 129, 128),
+                                         (65, 576, 72, 192), (130, 640, 300, 32)])
+def test_q4_planes(hip, oracle, monkeypatch, M, K, N, group, zeros, splits):
+    """The prefill copy's weights through the planes, activations over a wide range; every output type."""
+    from bybylang_amd import synth
+    g = synth.rng(M + K + N)
+    wq, sc, ze, _ = synth.q4_weights(g, N, K, group or K)
+    if zeros == "group":
+        ze = g.integers(0, 16, ze.size).astype(np.float32)
+    x = (synth.activations(g, M, K, np.float32) * 10.0 ** g.uniform(-8, 6, (M, 1))).astype(np.float32)
+    gpr = K // group if group else 1
+    monkeypatch.setenv("BYHIP_Q4_PLANES", "1")
+    monkeypatch.setenv("BYHIP_Q4_ROUTE", "2")
+    if splits:
+        monkeypatch.setenv("BYHIP_Q4_SPLIT", str(splits))
+    w = hip.Q4Weights(wq, sc, ze, K, N, group, gpr)
+    xd = hip.DeviceBuffer.from_array(x.reshape(-1))
+    want = oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, gpr)
+    outs = {}
+    for yt, nbytes in ((hip.F32, 4), (hip.BF16, 2)):
+        y = hip.DeviceBuffer(M * N * nbytes)
+        hip.q4_matmul(xd, hip.F32, w, y, yt, M)
+        outs[yt] = y.read(hip.np_dtype(yt)).reshape(M, N)
+    for m in range(M):  # row by row: each at its own magnitude
+        scale = max(1e-30, float(np.max(np.abs(want[m]))))
+        ref_check(outs[hip.F32][m] / scale, want[m] / scale)
+    from parity import f32_to_bf16_rne
+    assert np.array_equal(outs[hip.BF16], (f32_to_bf16_rne(outs[hip.F32]).view(np.uint32) >> 16).astype(np.uint16))
