@@ -306,6 +306,102 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
         }
 }
 
+// The same for up to 16 rows and so few columns that 128-column blocks would need K split over the grid:
+// a block owns 16 columns over all of K and its eight waves split K (wave w takes steps w, w + 8, ..), each
+// with two activation buffers of its own and no barrier; the partial tiles are added in wave order
+// through LDS, so there is no second launch. K = N = 4096, M = 16: 11.3 us against 13.2 with 8 K
+// splits and their sum; the fp32 MFMAs and the weights' decoding take 5.6 of it per 4,096 of K.
+template <bool ZU>
+__global__ __launch_bounds__(512, 2) void gemm_f32_q4_cols(GemmArgs a) {
+    constexpr int kBuf = 16 * kRStep * 4, kLoads = 8 + 2 + (ZU ? 0 : 1);  // per wave and step
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    __shared__ __attribute__((aligned(16))) uint8_t lds[8 * 2 * kBuf];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16, n = n0 + c;
+    const int total = a.K / kRStep, nt = total > wid ? (total - wid + 7) / 8 : 0;
+    const int gshift = a.group ? 31 - __builtin_clz((uint32_t)a.group >> 5) : 0;
+
+    const rsrc_t xr = make_rsrc(a.x, (uint32_t)((size_t)a.M * a.K * 4));
+    const rsrc_t wr = make_rsrc(a.wq, (uint32_t)((size_t)a.N * a.row_bytes));
+    const rsrc_t sr = make_rsrc(a.scales, (uint32_t)((size_t)a.N * a.gpr * 4));
+    const rsrc_t zr = make_rsrc(ZU ? a.scales : (const void*)a.zeros, ZU ? 0u : (uint32_t)((size_t)a.N * a.gpr * 4));
+    uint32_t xo[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int r = 2 * q + (lane >> 5);
+        xo[q] = (uint32_t)r * (uint32_t)a.K * 4u + 16u * (uint32_t)((lane & 31) ^ r);
+    }
+    const uint32_t wo = (uint32_t)n * (uint32_t)a.row_bytes + 16u * (uint32_t)g;
+    const uint32_t so = (uint32_t)n * (uint32_t)a.gpr * 4u;
+    uint8_t* const xb = lds + wid * 2 * kBuf;
+    struct W {
+        v4u q;
+        uint32_t s, z;
+    };
+    auto load = [&](W& w, int t, int buf) __attribute__((always_inline)) {
+        const bool ok = t < nt;
+        const uint32_t u = ok ? (uint32_t)(wid + 8 * t) : 0u, past = ok ? 0u : 0x80000000u;
+        w.q = __builtin_amdgcn_raw_buffer_load_b128(wr, wo, past + 64u * u, 0);
+        const uint32_t grp = a.group ? (4u * u + (uint32_t)g) >> gshift : 0u;
+        w.s = __builtin_amdgcn_raw_buffer_load_b32(sr, so + 4u * grp, past, 0);
+        if constexpr (!ZU) w.z = __builtin_amdgcn_raw_buffer_load_b32(zr, so + 4u * grp, past, 0);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) lds_dma16(xr, xb + buf * kBuf + 1024 * q, xo[q], past + 512u * u);
+    };
+    f4 acc[2] = {(f4){0.0f, 0.0f, 0.0f, 0.0f}, (f4){0.0f, 0.0f, 0.0f, 0.0f}};
+    W w[2];
+    load(w[0], 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
+    auto step = [&](int t, auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+        // the reads of step t - 1 have returned (its MFMAs used them), so its buffer is free
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        load(w[k ^ 1], t + 1, k ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<kLoads>();  // step t's loads have landed
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const float s = __builtin_bit_cast(float, w[k].s), z = ZU ? a.zero_value : __builtin_bit_cast(float, w[k].z);
+        const uint8_t* const x = xb + k * kBuf + 512 * c;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const uint32_t even = w[k].q[d] & 0x0F0F0F0Fu, odd = (w[k].q[d] >> 4) & 0x0F0F0F0Fu;
+            const f4 x0 = *reinterpret_cast<const f4*>(x + 16 * ((8 * g + 2 * d) ^ c));
+            const f4 x1 = *reinterpret_cast<const f4*>(x + 16 * ((8 * g + 2 * d + 1) ^ c));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float we = ((float)((even >> (8 * e)) & 255u) - z) * s, wq = ((float)((odd >> (8 * e)) & 255u) - z) * s;
+                const float xe = e < 2 ? x0[2 * e] : x1[2 * e - 4], xq = e < 2 ? x0[2 * e + 1] : x1[2 * e - 3];
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xe, we, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xq, wq, acc[1], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int t = 0; t < nt; t += 2) {
+        step(t, std::integral_constant<int, 0>{});
+        if (t + 1 < nt) step(t + 1, std::integral_constant<int, 1>{});
+    }
+    // every wave is done with its buffers and their direct loads have landed
+    wait_vmcnt<0>();
+    __syncthreads();
+    f4* const red = reinterpret_cast<f4*>(lds);
+    red[64 * wid + lane] = acc[0] + acc[1];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        f4 v = red[lane];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) v += red[64 * i + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = 4 * g + r;
+            if (m < a.M && n < a.N) store_any(a.y, a.y_dtype, (size_t)m * a.N + n, v[r]);
+        }
+    }
+}
+
 template <int FM>
 void launch_f32_q4_fm(const GemmArgs& a, dim3 grid) {
     if (a.zeros) launch("gemm_f32_q4", (gemm_f32_q4<FM, false>), grid, dim3(512), 0, a);
@@ -316,6 +412,16 @@ void launch_f32_q4_fm(const GemmArgs& a, dim3 grid) {
 // K splits: as many as leave one block per CU, each of at least two steps (K = N = 4096, M = 16, 4 / 8 /
 // 16 splits: 18.3 / 13.4 / 14.6 us).
 void launch_f32_q4(GemmArgs a) {
+    // Up to 16 rows on at most one 16-column block per CU (us, 128-column blocks with split K / this:
+    // K = N = 4096, M = 16 13.2 / 11.3, M = 4 11.8 / 10.0; K = 8192, N = 4096 18.8 / 16.9; K = 2048, N = 1000
+    // 8.4 / 6.3; K = 1024, N = 512 8.2 / 5.5; past it K = 4096, N = 6144, M = 9 17.4 / 18.4).
+    if (a.M <= 16 && (a.N + 15) / 16 <= compute_units() && env_int("BYHIP_Q4_SPLIT", 0) == 0) {
+        const dim3 grid((unsigned)((a.N + 15) / 16));
+        if (a.zeros) launch("gemm_f32_q4_cols", gemm_f32_q4_cols<false>, grid, dim3(512), 0, a);
+        else launch("gemm_f32_q4_cols", gemm_f32_q4_cols<true>, grid, dim3(512), 0, a);
+        BYHIP_LAUNCHED("gemm_f32_q4_cols");
+        return;
+    }
     const int row_tiles = (a.M + 63) / 64, fm = (a.M + 16 * row_tiles - 1) / (16 * row_tiles);
     const int rows = (a.M + 16 * fm - 1) / (16 * fm);
     const long tiles = (long)((a.N + 127) / 128) * rows;
