@@ -7,12 +7,12 @@
 //   FP4-KM with an E2M1 table and scales whose products with it are halves (checked per scale byte
 //          while it is used; a block that meets another scale, or a table that is not E2M1,
 //          computes its tile again in fp32 arithmetic as the reference does)
-//   F16
+//   F16    (gemm_planes_half, below, where both operands go through LDS)
 //   Q4     on the prefill copy: the codes less their zero (whole numbers) go through the MFMAs, and each
 //          32-value group's sums are scaled in fp32. Two MFMAs per product where weights as two fp16
 //          terms (the wide tile on fp32 activations) take three.
 //
-// Block: 16 FM rows x 128 columns, eight waves, two per SIMD. Waves w, w + 2, .. (p = w % 2) form K
+// gemm_planes. Block: 16 FM rows x 128 columns, eight waves, two per SIMD. Waves w, w + 2, .. (p = w % 2) form K
 // group p, which takes every other 128-value step of the block; wave h = w / 2 of the group owns
 // columns 32 h .. 32 h + 31 (2 fragments) and all rows: each decoded weight fragment feeds 2 FM
 // MFMAs (hi and lo), and each activation fragment read from LDS 2. Two K groups rather than four
@@ -22,7 +22,6 @@
 // slice of both planes moves straight into LDS by direct loads, 16-byte chunk k of row r at slot
 // k ^ x_swizzle(r), four buffers, loads three sub-steps ahead. Lane (c, g) = (lane % 16, lane / 16)
 // multiplies chunks 2 g and 2 g + 1 of the slice with its weights of column c:
-//   F16     16 halves of the weight row, in natural order
 //   Q4      chunks g and 4 + g instead: MFMA kk then covers one 32-value group, positions 32 kk + 8 g ..
 //           + 7 per lane, one dword of the prefill copy (a fragment's 64 dwords are 256 contiguous
 //           bytes). Its sums wait in registers of their own and are scaled and added during the next K
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     if (a.gate && *a.gate != a.gate_want) return;  // another route was chosen (whole grid)
     constexpr bool FP4 = F == BFormat::Fp4Km, Q4 = F == BFormat::Q4Fast;
     constexpr int FN = 2;
-    constexpr int WV = FP4 ? FN : Q4 ? 2 : 2 * FN;  // weight registers of a set, in 16-byte units
+    constexpr int WV = 2;  // weight registers of a set, in 16-byte units
     using S = PlaneShape<FM>;
     constexpr int BM = S::kBM, kXBuf = S::kXBuf;
     // One LDS array for everything, the eight waves' `bad` words at its end: beside a second array (a
@@ -169,12 +168,8 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     const rsrc_t xr = make_rsrc(h < 2 ? a.x : a.x_lo, (uint32_t)((size_t)a.M * K * 2));
     const uint32_t nsub = (uint32_t)K / kSub;
     const uint32_t wpf_bytes = ((uint32_t)a.N + 15) / 16 * nsub * 512, spf_bytes = ((uint32_t)a.N + 63) / 64 * nsub * 256;
-    const rsrc_t wr = FP4  ? make_rsrc(a.blob, (uint32_t)((size_t)a.N * (K >> 1)))
-                      : Q4 ? make_rsrc(a.wpf, wpf_bytes)
-                           : make_rsrc(a.w16, (uint32_t)((size_t)a.N * K * 2));
-    const rsrc_t sr = FP4  ? make_rsrc(a.blob + a.scale_base, (uint32_t)((size_t)a.N * (K >> 5)))
-                      : Q4 ? make_rsrc(a.spf, spf_bytes)
-                           : wr;
+    const rsrc_t wr = FP4 ? make_rsrc(a.blob, (uint32_t)((size_t)a.N * (K >> 1))) : make_rsrc(a.wpf, wpf_bytes);
+    const rsrc_t sr = FP4 ? make_rsrc(a.blob + a.scale_base, (uint32_t)((size_t)a.N * (K >> 5))) : make_rsrc(a.spf, spf_bytes);
     const rsrc_t zr = ZG ? make_rsrc(a.zpf, spf_bytes) : sr;
     // Direct load q (0 .. FM - 1) of wave h: stacked rows 8 FM h + 8 q + lane / 8 of the slice (the
     // high plane's BM rows, then the low plane's), LDS slot lane % 8.
@@ -190,9 +185,8 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     for (int j = 0; j < FN; ++j) {
         const int n = n0 + 32 * h + 16 * j + c;
         col_ok[j] = n < a.N;
-        wo[j] = FP4  ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g
-                : Q4 ? ((uint32_t)n >> 4) * nsub * 512u + 8u * c + 128u * (uint32_t)(g >> 1) + 4u * (uint32_t)(g & 1)
-                     : (uint32_t)n * (uint32_t)K * 2u + 32u * g;
+        wo[j] = FP4 ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g
+                    : ((uint32_t)n >> 4) * nsub * 512u + 8u * c + 128u * (uint32_t)(g >> 1) + 4u * (uint32_t)(g & 1);
         so[j] = (uint32_t)n * (uint32_t)(K >> 5) + 8u * g;
     }
     // Q4 scales (and zeros): the wave's 2 fragments are fragments 2 (h % 2) and the next of their quad
@@ -208,9 +202,8 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
 #pragma unroll
         for (int q = 0; q < FM; ++q) lds_dma16(xr, xgrp + buf * kXBuf + 1024 * (FM * h + q), xo[q], off);
     };
-    // FP4-KM: the 16 bytes per column of the group's step q (sub-steps 2 q and 2 q + 1); F16: the
-    // sub-step's 32 bytes; Q4: per MFMA kk a dword per fragment, w[kk][j], the fragments' scales
-    // w[kk][2] and zeros w[kk][3].
+    // FP4-KM: the 16 bytes per column of the group's step q (sub-steps 2 q and 2 q + 1); Q4: per MFMA
+    // kk a dword per fragment, w[kk][j], the fragments' scales w[kk][2] and zeros w[kk][3].
     v4u wv[kSets][WV];
     auto load_w = [&](v4u (&w)[WV], int t) __attribute__((always_inline)) {
         if constexpr (Q4) {
@@ -223,19 +216,11 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
                 w[kk][2] = __builtin_amdgcn_raw_buffer_load_b32(sr, sq, past + 256u * u + 128u * kk, 0);
                 if constexpr (ZG) w[kk][3] = __builtin_amdgcn_raw_buffer_load_b32(zr, sq, past + 256u * u + 128u * kk, 0);
             }
-        } else if constexpr (FP4) {
+        } else {
             const int s = p + 2 * t;
             const uint32_t off = s < steps ? 64u * (uint32_t)(step0 + s) : kPast;
 #pragma unroll
             for (int j = 0; j < FN; ++j) w[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off, 0);
-        } else {
-            const int sl = 2 * p + 4 * (t >> 1) + (t & 1);
-            const uint32_t off = sl < slices ? 128u * (uint32_t)(2 * step0 + sl) : kPast;
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                w[2 * j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off, 0);
-                w[2 * j + 1] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], off + 16u, 0);
-            }
         }
     };
     // FP4-KM scale bytes: the dword of lane (c, i) holds the four bytes (groups 0 .. 3) of column c in
@@ -291,7 +276,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
                 const uint4 u = make_uint4(h2_bits(bits_h2((d & 0x000F000Fu) | mag_lo) - z0), h2_bits(bits_h2((d & 0x00F000F0u) | mag_hi) - z1),
                                            h2_bits(bits_h2((d8 & 0x000F000Fu) | mag_lo) - z0), h2_bits(bits_h2((d8 & 0x00F000F0u) | mag_hi) - z1));
                 b[j] = *reinterpret_cast<const h8*>(&u);
-            } else if constexpr (FP4) {
+            } else {
                 const uint32_t d = w[j][2 * e + kk];
                 const h2 s2 = bits_h2(ss[j]);
                 const uint4 u = make_uint4(h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 0) * s2),
@@ -299,8 +284,6 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
                                            h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 2) * s2),
                                            h2_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 3) * s2));
                 b[j] = *reinterpret_cast<const h8*>(&u);
-            } else {
-                b[j] = __builtin_bit_cast(h8, w[2 * j + kk]);
             }
         }
     };
@@ -350,11 +333,11 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     };
 
     // Loads of a sub-step at position k of the unrolled loop (weights first, then activations): the
-    // activations of sub-step t + 3, the weights of t + 3 (F16) or, on even t, of step t / 2 + 3
+    // activations of sub-step t + 3, the weights of t + 3 (Q4) or, on even t, of step t / 2 + 3
     // (FP4-KM, with the next four steps' scale bytes at k = 0).
     constexpr int kXLoads = FM;
     auto issued = [](int k) constexpr {
-        return kXLoads + (FP4 ? ((k & 1) ? 0 : FN) + (k == 0 ? FN : 0) : Q4 ? 2 * (FN + 1 + ZG) : 2 * FN);
+        return kXLoads + (FP4 ? ((k & 1) ? 0 : FN) + (k == 0 ? FN : 0) : 2 * (FN + 1 + ZG));
     };
 
     h8 ax0[2][FM], ax1[2][FM], bw0[FN], bw1[FN];
@@ -378,7 +361,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         lut_h[0] = b[0] | (b[1] << 16);
         lut_h[1] = b[2] | (b[3] << 16);
     }
-    wait_vmcnt<2 * (kXLoads + (FP4 ? FN : Q4 ? 2 * (FN + 1 + ZG) : 2 * FN))>();
+    wait_vmcnt<2 * (kXLoads + (FP4 ? FN : 2 * (FN + 1 + ZG)))>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (FP4) scale_of(sb, 0, ss);
     read_x(0, 0, ax0);
@@ -386,7 +369,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
 
     constexpr int kMfmas = 2 * FM * FN;  // per K half
     // VALU operations beside each MFMA; Q4: the first half of the MFMAs beside the scaling
-    constexpr int kValuPerMfma = FP4 ? (FN * 9 + kMfmas - 1) / kMfmas : Q4 ? 4 : 1;
+    constexpr int kValuPerMfma = FP4 ? (FN * 9 + kMfmas - 1) / kMfmas : 4;
     // Sub-step t = base + k. Its loads, in `wait` order: at the mid-step wait those of this and of the
     // previous sub-step may stay in flight, which leaves t + 1's activations landed.
     auto step = [&](int t, auto kc, auto guard) __attribute__((always_inline)) {
@@ -396,7 +379,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         const bool live = !decltype(guard)::value || t < nt_all;
         uint32_t sn[FP4 ? FN : 1];
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!FP4) load_w(wv[(k + 3) % kSets], t + 3);
+        if constexpr (Q4) load_w(wv[(k + 3) % kSets], t + 3);
         if constexpr (FP4 && e == 0) load_w(wv[((k >> 1) + 3) % kSets], (t >> 1) + 3);
         if constexpr (FP4 && k == 0) load_sb(sbn, (t >> 3) + 1);
         load_x(t + 3, (k + 3) % kDepth);
@@ -497,6 +480,167 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
             v[e + 1] = __builtin_amdgcn_ldexpf(s0.y + s1.y, -sh);
             v[e + 2] = __builtin_amdgcn_ldexpf(s0.z + s1.z, -sh);
             v[e + 3] = __builtin_amdgcn_ldexpf(s0.w + s1.w, -sh);
+        }
+        store_out8<YT>(a, part, vec, m, n0 + col, v);
+    }
+}
+
+// gemm_planes_half: half weights, both operands through LDS. A fragment's 16 rows x 64 bytes of half
+// weights loaded straight into registers touch half a line per row, which costs the load unit as
+// much as whole lines: that alone took 18 of 42 us at M = 130, K = 4096, N = 6144. Here the weights'
+// 128 lines per 64-value sub-step go into LDS by direct loads beside the planes', and both are read as
+// fragments; one K group, so the buffers hold them.
+//   Block: 16 RP FR rows x 128 columns, RP x CP waves; wave w owns 128 / CP columns from part w % CP and
+//   16 FR rows from part w / CP. Loads run kDepth - 1 sub-steps ahead, each sub-step in two halves
+//   around one barrier as above. LDS bounds it: per sub-step a 64-row tile of 8 waves reads 96 KB of
+//   fragments and takes in 32 KB for 512 clocks of MFMAs per SIMD. A 128-row tile's waves (32 x 64
+//   outputs) read 2/3 of that per MFMA; four waves of that shape on 64 rows do too, but one wave
+//   per SIMD hides less: 39 us for 29 below.
+//   Time with split_planes and the splits' sum, against weights in registers:
+//     M = 130, K = 4096, N = 6144: 42.1 -> 29.2 us     M = 512, K = N = 4096: 48.7 -> 39.0
+//     M = 256, K = 4096, N = 14336: 86 (64 rows), 66 (128 rows)
+//     M = 16, K = 4096, N = 6144: 16.4 -> 15.2         M = 1: 15.3 -> 14.1
+template <int RP, int FR, int CP>
+struct HalfShape {
+    static constexpr int kWaves = RP * CP, kFN = kBN / 16 / CP, kBM = 16 * RP * FR;
+    static constexpr int kRows = 2 * kBM + kBN;                 // lines per buffer: planes, then weights
+    static constexpr int kBuf = kRows * 128, kDepth = kBM == 64 ? 4 : 3;
+    static constexpr int kLoads = kRows / 8 / kWaves;           // per wave and sub-step
+    static constexpr int kPlane = kBM / 8 / kWaves;             // of them a plane's
+    static constexpr int kRed = kBM * kPitch * 4;
+    static constexpr int kLds = kDepth * kBuf > kRed ? kDepth * kBuf : kRed;
+};
+
+template <int RP, int FR, int CP, int YT>
+__global__ __launch_bounds__(64 * RP * CP, RP * FR == 2 ? 4 : 2) void gemm_planes_half(GemmArgs a) {
+    using S = HalfShape<RP, FR, CP>;
+    constexpr int BM = S::kBM, D = S::kDepth, FN = S::kFN, NW = S::kWaves;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[S::kLds];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = wid % CP, rh = wid / CP, c = lane & 15, g = lane >> 4;
+    int bx = blockIdx.x, by = blockIdx.y;
+    {
+        // the wide tile's XCD-grouped tile order
+        const int gx = gridDim.x, gy = gridDim.y, tiles = gx * gy, id = bx + gx * by;
+        const int j = tiles % 8 == 0 ? (id % 8) * (tiles / 8) + id / 8 : id;
+        const int grp = j / (4 * gx), rows = min(4, gy - 4 * grp), r = j % (4 * gx);
+        by = 4 * grp + r % rows;
+        bx = r / rows;
+    }
+    const int n0 = bx * kBN, m0 = by * BM, K = a.K;
+    const int s_all = K / kSub, s_first = a.part ? (int)blockIdx.z * a.split_steps : 0;
+    const int nt = a.part ? min(a.split_steps, s_all - s_first) : s_all;
+
+    // Line groups NW i .. are one operand's each, except that 32 rows have both planes in the first NW.
+    const uint32_t plane = (uint32_t)((size_t)a.M * K * 2);
+    const rsrc_t xr = make_rsrc(S::kPlane == 0 && wid >= NW / 2 ? a.x_lo : a.x, plane), xlr = make_rsrc(a.x_lo, plane);
+    const rsrc_t wr = make_rsrc(a.w16, (uint32_t)((size_t)a.N * K * 2));
+    // Direct load i of wave w: line group w + NW i, rows 8 (w + NW i) + lane / 8 of the buffer (high plane,
+    // low plane, weights); rows past M or N read zeros.
+    uint32_t off[S::kLoads];
+#pragma unroll
+    for (int i = 0; i < S::kLoads; ++i) {
+        const int r = 8 * (wid + NW * i) + (lane >> 3);
+        const uint32_t row = r >= 2 * BM ? (uint32_t)(n0 + r - 2 * BM) : (uint32_t)(m0 + (r >= BM ? r - BM : r));
+        off[i] = row * (uint32_t)K * 2u + 16u * (uint32_t)((lane & 7) ^ x_swizzle(r & 15));
+    }
+    auto load = [&](int t, int buf) __attribute__((always_inline)) {
+        const uint32_t o = t < nt ? 128u * (uint32_t)(s_first + t) : kPast;
+        static_for<S::kLoads>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            uint8_t* const to = lds + buf * S::kBuf + 1024 * (wid + NW * i);
+            if constexpr (i >= (S::kPlane ? 2 * S::kPlane : 1)) lds_dma16(wr, to, off[i], o);
+            else if constexpr (S::kPlane && i >= S::kPlane) lds_dma16(xlr, to, off[i], o);
+            else lds_dma16(xr, to, off[i], o);
+        });
+    };
+    const int rd[2] = {128 * c + 16 * ((2 * g) ^ x_swizzle(c)), 128 * c + 16 * ((2 * g + 1) ^ x_swizzle(c))};
+
+    // Sums of their own for each plane and K half of a sub-step, added up at the end: in one chain of
+    // roundings the error against 64 bits was 5.8e-7 (M = 130, K = 4096), so it is 2.9e-7.
+    f4 acc[2][2][FR][FN];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < FR; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[s >> 1][s & 1][i][j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    auto read = [&](int buf, int kk, h8 (&x)[2][FR], h8 (&b)[FN]) __attribute__((always_inline)) {
+        const uint8_t* const s = lds + buf * S::kBuf + rd[kk];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b[j] = *reinterpret_cast<const h8*>(s + 128 * (2 * BM + 16 * FN * h + 16 * j));
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+            for (int i = 0; i < FR; ++i) x[pl][i] = *reinterpret_cast<const h8*>(s + 128 * (BM * pl + 16 * FR * rh + 16 * i));
+    };
+    auto mfmas = [&](const h8 (&x)[2][FR], const h8 (&b)[FN], f4 (&s)[2][FR][FN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+            for (int i = 0; i < FR; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    s[pl][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[pl][i], b[j], s[pl][i][j], 0, 0, 0);
+    };
+
+    h8 x0[2][FR], x1[2][FR], b0[FN], b1[FN];
+    static_for<D - 1>([&](auto kc) {
+        load(decltype(kc)::value, decltype(kc)::value);
+        __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
+    });
+    wait_vmcnt<(D - 2) * S::kLoads>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    read(0, 0, x0, b0);
+    auto step = [&](int t, auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        load(t + D - 1, (k + D - 1) % D);
+        mfmas(x0, b0, acc[0]);
+        read(k, 1, x1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<(D - 2) * S::kLoads>();  // t + 1's lines have landed
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        mfmas(x1, b1, acc[1]);
+        read((k + 1) % D, 0, x0, b0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int t = 0;
+    for (; t + D <= nt; t += D) static_for<D>([&](auto kc) { step(t + decltype(kc)::value, kc); });
+    static_for<D - 1>([&](auto kc) {
+        if (t + decltype(kc)::value < nt) step(t + decltype(kc)::value, kc);
+    });
+
+    // tiles -> LDS, once every load has landed and every wave is done with the buffers -> y or partials
+    wait_vmcnt<0>();
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int i = 0; i < FR; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                red[(16 * FR * rh + 16 * i + 4 * g + r) * kPitch + 16 * FN * h + 16 * j + c] =
+                    (acc[0][0][i][j][r] + acc[1][0][i][j][r]) + (acc[0][1][i][j][r] + acc[1][1][i][j][r]);
+    __syncthreads();
+    float* part = a.part ? a.part + (size_t)blockIdx.z * splitk_stride(a.M, a.N) : nullptr;
+    const bool vec = out8_vector_ok<YT>(a, part);
+#pragma unroll
+    for (int k = 0; k < BM * 16 / (64 * NW); ++k) {
+        const int u = tid + 64 * NW * k, row = u >> 4, col = (u & 15) * 8, m = m0 + row;
+        if (m >= a.M) continue;
+        const float* src = red + row * kPitch + col;
+        const int sh = a.row_shift[m];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const float4 q = *reinterpret_cast<const float4*>(src + e);
+            v[e] = __builtin_amdgcn_ldexpf(q.x, -sh);
+            v[e + 1] = __builtin_amdgcn_ldexpf(q.y, -sh);
+            v[e + 2] = __builtin_amdgcn_ldexpf(q.z, -sh);
+            v[e + 3] = __builtin_amdgcn_ldexpf(q.w, -sh);
         }
         store_out8<YT>(a, part, vec, m, n0 + col, v);
     }
@@ -619,6 +763,53 @@ int planes_splits(const GemmArgs& a, long tiles) {
     return best;
 }
 
+// The same for gemm_planes_half, in 64-value steps: 16 for a block's fixed cost, 12 for the sum's launch and
+// 1.5 per split for what it reads (M = 32, K = 4096, N = 6144: 4 splits 16.3 us, 6 splits,
+// a second block on some of the CUs, 17.9, 1 split 24.5).
+int half_splits(long tiles, int steps) {
+    const long cus = compute_units();
+    int best = 1;
+    double best_t = 1e300;
+    for (int s = 1; s <= std::max(1, steps / 8); ++s) {
+        const int per = (steps + s - 1) / s;
+        if ((steps + per - 1) / per != s) continue;
+        const double t = (double)((tiles * s + cus - 1) / cus) * (per + 16) + (s > 1 ? 12.0 + 1.5 * s : 0.0);
+        if (t < 0.97 * best_t) best = s, best_t = t;
+    }
+    return best;
+}
+
+template <int RP, int FR, int CP>
+void launch_half_y(const GemmArgs& a, int splits) {
+    using S = HalfShape<RP, FR, CP>;
+    const dim3 grid((a.N + kBN - 1) / kBN, (a.M + S::kBM - 1) / S::kBM, splits), block(64 * S::kWaves);
+    switch (a.y_dtype) {
+    case BYHIP_F32: launch("gemm_planes_half", (gemm_planes_half<RP, FR, CP, BYHIP_F32>), grid, block, 0, a); break;
+    case BYHIP_F16: launch("gemm_planes_half", (gemm_planes_half<RP, FR, CP, BYHIP_F16>), grid, block, 0, a); break;
+    default: launch("gemm_planes_half", (gemm_planes_half<RP, FR, CP, BYHIP_BF16>), grid, block, 0, a); break;
+    }
+    BYHIP_LAUNCHED("gemm_planes_half");
+}
+
+// Rows per tile: 32, two blocks per CU, for up to 32 rows (M = 8, K = N = 4096: 12.6 us, 64 rows
+// 13.1); else 64, or 128 where its rounds of blocks, each 1.6 times as long, take less time (M = 256, K =
+// 4096, N = 14336: one round for two, 66 us for 86; M = 512, K = N = 4096: one round either way, 45 for 39).
+void launch_half_rows(const GemmArgs& a0) {
+    GemmArgs a = a0;
+    const int cus = compute_units();
+    const long cols = (a.N + kBN - 1) / kBN, t64 = cols * ((a.M + 63) / 64), t128 = cols * ((a.M + 127) / 128);
+    const bool tall = (uint64_t)a.K * 256 < kPast / 2 && 8 * ((t128 + cus - 1) / cus) < 5 * ((t64 + cus - 1) / cus);
+    const long tiles = a.M <= 32 ? cols : tall ? t128 : t64;
+    const int steps = a.K / kSub;
+    const int forced = env_int("BYHIP_Q4_SPLIT", 0);
+    const int splits = choose_split(a, tiles, steps, 1, forced > 0 ? forced : half_splits(tiles, steps), 1);
+    if (splits == 1) a.part = nullptr;
+    if (a.M <= 32) launch_half_y<2, 1, 4>(a, splits);
+    else if (tall) launch_half_y<4, 2, 2>(a, splits);
+    else launch_half_y<2, 2, 4>(a, splits);
+    if (a.part) launch_splitk_sum(a, splits);
+}
+
 template <BFormat F>
 void launch_planes_rows(const GemmArgs& a0) {
     GemmArgs a = a0;
@@ -687,7 +878,7 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
         a.work_bytes = work_bytes - shift_bytes - 2 * plane;
         if (fmt == BFormat::Fp4Km) launch_planes_rows<BFormat::Fp4Km>(a);
         else if (fmt == BFormat::Q4Fast) launch_planes_rows<BFormat::Q4Fast>(a);
-        else launch_planes_rows<BFormat::F16>(a);
+        else launch_half_rows(a);
     }
 }
 

@@ -20,6 +20,7 @@ KERNELS = {
     "q4_gemm_wide": ("byhip_gemm.hip.o", lambda t: t[0] * (2 if t[3] == 2 else 1)),
     "q4_gemm_tall": ("byhip_gemm.hip.o", lambda t: 2),
     "gemm_planes": ("byhip_planes.hip.o", lambda t: t[1]),
+    "gemm_planes_half": ("byhip_planes.hip.o", lambda t: (4 * t[0] * t[1] + 16) // (t[0] * t[2])),
     "mxfp4_gemm_mid": ("byhip_mxfp4.hip.o", lambda t: 4),
     "gemm_f32_q4": ("byhip_exact.hip.o", lambda t: t[0]),
 }

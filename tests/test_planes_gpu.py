@@ -115,6 +115,30 @@ def test_f16_planes(hip, oracle, M, K, N):
     ref_check(y.read(np.float32), want)
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 4096, 257), (32, 448, 127), (33, 2112, 128), (65, 256, 640), (128, 1536, 300), (300, 64, 8200), (257, 320, 8193)])
+def test_f16_tiles(hip, oracle, M, K, N):
+    """Half weights at the edges of the 32-, 64- and 128-row tiles, fewer sub-steps than buffers, and with K
+    split; one row's infinity and one weight's NaN stay in their row and column."""
+    from bybylang_amd import synth
+    g = synth.rng(M + K + N)
+    x = synth.activations(g, M, K, np.float32)
+    w = (g.standard_normal((N, K)) * 0.05).astype(np.float16)
+    run = lambda: hip.f16_tile_gemm(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.DeviceBuffer.from_array(w.reshape(-1)), y, hip.F32,
+                                    M, K, N)
+    y = hip.DeviceBuffer(M * N * 4)
+    run()
+    want = np.asarray(oracle.tile_gemm(1, M, K, N, 0, 0, w.view(np.uint8).reshape(-1), None, x)).reshape(M, N)
+    ref_check(y.read(np.float32), want)
+    x[M - 1, K - 1] = np.inf
+    w[N - 1, 0] = np.nan
+    run()
+    got = y.read(np.float32).reshape(M, N)
+    assert np.isnan(got[:, N - 1]).all()
+    assert not np.isfinite(got[M - 1]).any()
+    if M > 1:
+        ref_check(got[:M - 1, :N - 1], want[:M - 1, :N - 1])
+
+
 @pytest.mark.parametrize("scales", ["ref", "mx", "edge"])
 @pytest.mark.parametrize("K,N", [(32, 1), (96, 9), (2048, 65), (2080, 16), (4096, 130), (6176, 7), (8224, 24), (15360, 17), (15392, 17)])
 def test_fp4km_decode_row(hip, oracle, K, N, scales):
