@@ -7,8 +7,9 @@
 //   F16     the half widened (cpu_vm.c:571-575)
 // Activations are used in fp32 (fp16 ones widened exactly); products and sums are fp32, in
 // v_mfma_f32_16x16x4_f32. This is the route for data the fp16 MFMA kernels cannot hold exactly:
-// Q4 weights outside fp16's range, FP4-KM tables whose products are not halves, and the micro-VM's
-// Q4 GEMV op (fp32 arithmetic in the reference) above the decode GEMV's rows. It differs from the
+// Q4 weights outside fp16's range, FP4-KM tables whose values are not E2M1 and whose products are not
+// halves, and the micro-VM's Q4 ops (fp32 arithmetic in the reference) above two rows; these take
+// gemm_f32_q4 (below), the pipelined form for Q4 rows and fp16 scales, where it fits. It differs from the
 // reference only in the order of the fp32 additions.
 //
 // Block: BM x 64 outputs, 4 waves; wave w owns columns 16w .. 16w+15 and all BM rows (BM / 16

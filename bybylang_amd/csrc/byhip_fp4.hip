@@ -3,8 +3,10 @@
 //
 // FP4-KM (cpu_vm.c:583-628): weight = lut[nibble] * lut[16 + scale byte] with the 272-float decode
 // table; nibble bytes [N, K/2] (byte j of a group: element j low, j + 16 high), scale bytes
-// [N, K/32] at scale_base. fp32/fp16 activations take the fp16 MFMA GEMM with the weights decoded
-// through the table in LDS; activations already in MXFP4 take the scaled MFMA when the table is
+// [N, K/32] at scale_base. fp32 activations and E2M1 values with any scale entries take one row on the
+// decode GEMV (byhip_fp4gemv.hip) and more on the two-plane GEMM (byhip_planes.hip); other tables whose
+// products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
+// the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
 // exactly E2M1 and 2^(e-127).
 #include <algorithm>
 #include <cmath>
