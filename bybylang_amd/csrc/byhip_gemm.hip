@@ -1632,7 +1632,11 @@ void launch_q4_big(const GemmArgs& a0, int split_choice = 0) {
 // K splits for the wide tile: the count that minimises the estimated time
 // ceil(tiles * s / CUs) x (sub-steps per split + 16), the 16 standing for a block's fixed cost (its
 // first loads' latency, the epilogue), with at least 8 sub-steps per split and each split a multiple
-// of 4 sub-steps (one per group and round); fewer splits win unless more save over 3 %.
+// of 4 sub-steps (one per group and round); fewer splits win unless more save over 3 %. Where the
+// tiles alone fill the CUs, a split only evens out the last round and each slice still writes and the sum
+// reads a whole output, so both count: 12 for the launch and 8 bytes per output and slice at 1.1 MB
+// per sub-step (0.22 us). K = 4096, fp16, unsplit / split 2 ways: M = 251, N = 11008 35.2 / 43.4 us, M = 520, N = 4096
+// 34.4 / 40.9; K = 14336: M = 256, N = 8448 100.6 / 93.2.
 int wide_splits(const GemmArgs& a, long tiles) {
     const int nsub = a.K / kWideSub;
     const long cus = compute_units();
@@ -1642,7 +1646,8 @@ int wide_splits(const GemmArgs& a, long tiles) {
         const int steps = ((nsub + s - 1) / s + 3) / 4 * 4;
         const int splits = (nsub + steps - 1) / steps;
         if (splits != s) continue;  // the same split as a smaller s
-        const double t = (double)((tiles * s + cus - 1) / cus) * (steps + 16);
+        const double sum = s > 1 && tiles >= cus ? 12.0 + 8.0 * a.M * a.N * s / 1.1e6 : 0.0;
+        const double t = (double)((tiles * s + cus - 1) / cus) * (steps + 16) + sum;
         if (t < 0.97 * best_t) {
             best = s;
             best_t = t;

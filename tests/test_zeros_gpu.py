@@ -68,3 +68,25 @@ def test_zero_per_group_equal_zeros_match_one_zero(hip):
         hip.q4_matmul(xd, hip.F16, w, yd, hip.F32, M)
         outs.append(yd.read(np.float32).view(np.uint32))
     assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("M,K,N", [(251, 512, 8320), (65, 8192, 16400)])
+def test_tiles_past_one_round(hip, oracle, monkeypatch, M, K, N):
+    """The wide tile with a few tiles more than CUs, unsplit (short K) and split (long K) by default: the
+    first and last rows against the oracle, every row against the same tile with K split three ways,
+    which differs by the order of the fp32 sums only."""
+    x, wq, sc, ze = case(M + K, M, K, N, 32, "codes")
+    w = hip.Q4Weights(wq, sc, ze, K, N, 32, K // 32)
+    xd = hip.DeviceBuffer.from_array(x.reshape(-1))
+    outs = []
+    monkeypatch.setenv("BYHIP_Q4_PREFILL", "3")
+    for split in (None, "3"):
+        if split:
+            monkeypatch.setenv("BYHIP_Q4_SPLIT", split)
+        yd = hip.DeviceBuffer(M * N * 4)
+        hip.q4_matmul(xd, hip.F16, w, yd, hip.F32, M)
+        outs.append(yd.read(np.float32).reshape(M, N))
+    ref_check(outs[0], outs[1])
+    rows = [0, M - 1]
+    want = oracle.matmul_q4(x[rows].astype(np.float32).reshape(-1), wq, sc, ze, 2, K, N, 32, K // 32)
+    tier_check(outs[0][rows].reshape(-1), np.asarray(want).reshape(-1), TIER_F32_ACC)
