@@ -250,9 +250,11 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
         for (int q = 0; q < FM; ++q) lds_dma16(xr, lds + buf * S::kBuf + 1024 * (FM * wid + q), xo[q], past + 512u * u);
     };
 
-    f4 acc[FM];
+    // Two sums per fragment, of even and odd products, added at the end: half the chain of roundings (one sum,
+    // M = 23, K = 7040, N = 1792: error against 64 bits 4.0e-7, two 2.9e-7).
+    f4 acc[FM], acc_odd[FM];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) acc[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < FM; ++i) acc[i] = acc_odd[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     W w[3];
     load(w[0], 0, 0);
     __builtin_amdgcn_sched_barrier(0);  // the first wait counts on this order
@@ -282,7 +284,10 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
                 const f4 x1 = *reinterpret_cast<const f4*>(x + 8192 * i + 16 * ((8 * g + 2 * d + 1) ^ c));
                 const float xv[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[e], wf[e], acc[i], 0, 0, 0);
+                for (int e = 0; e < 8; e += 2) {
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[e], wf[e], acc[i], 0, 0, 0);
+                    acc_odd[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[e + 1], wf[e + 1], acc_odd[i], 0, 0, 0);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -300,9 +305,10 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + 16 * i + 4 * g + r;
+            const float v = acc[i][r] + acc_odd[i][r];
             if (m < a.M && n < a.N) {
-                if (part) part[(size_t)m * a.N + n] = acc[i][r];
-                else store_any(a.y, a.y_dtype, (size_t)m * a.N + n, acc[i][r]);
+                if (part) part[(size_t)m * a.N + n] = v;
+                else store_any(a.y, a.y_dtype, (size_t)m * a.N + n, v);
             }
         }
 }
