@@ -5,16 +5,18 @@
 // lane l the 32-value groups l, l + 64, .. of each (one 16-byte load and one scale byte); every load
 // goes out before the first wait, activations, scale bytes, then weights.
 //
-// Activations: each 32-value group is brought onto fp16's range by an exact power of two and split
-// into fp16 hi + lo (about 23 bits of x over the whole fp32 range), staged once per block in LDS as
-// the pairs (x[j], x[j + 16]) that byte j of a group multiplies. v_cvt_scalef32_pk_f16_fp4 turns a
-// byte into its two values, two v_dot2_f32_f16 multiply them (exact products, fp32 sums), and the
-// group's sum is scaled in fp32 by lut[16 + byte] and the power of two. A scale that is not finite
-// multiplies element by element, as the reference does, so its NaNs and infinities come out alike.
+// Activations stay fp32, staged once per block in LDS as the runs of four that four bytes of a group
+// multiply: low nibbles x[4 t ..], high nibbles x[16 + 4 t ..]. v_cvt_scalef32_pk_f32_fp4 turns a byte into
+// twice its two values, whole numbers, so products with subnormal activations stay exact too; two
+// chains of fp32 FMAs sum a group, and half its scale multiplies the sum. Where that order differs from
+// the reference's x * (value * scale) by more than rounding, the group is computed element by element as
+// the reference does: a sum that is not finite (activations near fp32's largest, infinities, NaNs), a
+// scale whose product with 6 overflows or with 0.5 is not exact.
 //
-// What bounds it: K = 4096, N = 14336, 31.2 MB: 9.0 us against 6.4 for the bytes at the rate of a
-// large copy (16.0 us on gemm_planes, whose 16-row tiles and second launch one row cannot use); the
-// rest is each block's staging of x and a launch's ramp, as in the Q4 GEMV.
+// What bounds it: K = 4096, N = 14336, 31.2 MB: 6.9 us against 6.4 for the bytes at the rate of a
+// large copy (8.9 us with two fp16 terms per activation and v_dot2_f32_f16, which held 23 bits of them and
+// split the row in every block; 16.0 us on gemm_planes, whose 16-row tiles and second launch one row
+// cannot use).
 #include "byhip_gemm.h"
 #include "byhip_internal.h"
 #include "byhip_kernels.h"
@@ -25,6 +27,7 @@ namespace {
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kRows = 2;  // rows per wave, as the Q4 GEMV at one activation row
+constexpr float kScaleMax = 0x1p125f;  // products of scales up to here with 6 are finite
 
 template <int CPL, int YT>
 __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
@@ -34,12 +37,10 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int K = a.K, N = a.N, G = K >> 5;
-    // piece t (bytes 4 t .. 4 t + 3's pairs) of group i at uint4 index t G + i, hi then lo; the groups'
-    // back-scales; the scale table
-    uint4* const xh = reinterpret_cast<uint4*>(lds);
-    uint4* const xl = xh + 4 * G;
-    float* const back = reinterpret_cast<float*>(xl + 4 * G);
-    float* const table = back + G;
+    // half l (0: low nibbles, 1: high) of piece t (bytes 4 t .. 4 t + 3) of group i at float4 index
+    // (2 t + l) G + i; the table
+    f4* const xs = reinterpret_cast<f4*>(lds);
+    float* const table = reinterpret_cast<float*>(xs + 8 * G);
     const int n0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + (tid >> 6)) * R);
 
     const rsrc_t wr = make_rsrc(a.blob, (uint32_t)((size_t)N * (K >> 1)));
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
         for (int t = 0; t < 4; ++t)
             xv[i][t] = buf_load16(xr, off == kOutOfRange ? off : off + 16u * (t & 1) + 64u * (t >> 1));
     }
-    const float lut_v = a.lut[16 + tid];
+    const float lut_v = a.lut[16 + tid], lut_e = a.lut[tid & 15];
     // 2. scale bytes, 3. weights (streamed once: non-temporal); rows past N read zeros
     uint32_t sb[R][CPL];
     v4u wv[R][CPL];
@@ -74,41 +75,16 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
                                                              (uint32_t)min(n0 + r, N) * (uint32_t)(K >> 1), 2);
     __builtin_amdgcn_sched_barrier(0);  // every load is out before the first wait
 
-    // 4. stage: the two lanes of a group share its maximum
-    table[tid] = lut_v;
+    // 4. stage
+    table[16 + tid] = lut_v;
+    if (tid < 16) table[tid] = lut_e;
 #pragma unroll
     for (int i = 0; i < XC; ++i) {
         const int idx = (tid + 256 * i) >> 1, h = tid & 1;
         if (idx < G) {
-            float v[16];  // x[8 h + e] and x[16 + 8 h + e]
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                v[4 * t] = __builtin_bit_cast(float, xv[i][t].x);
-                v[4 * t + 1] = __builtin_bit_cast(float, xv[i][t].y);
-                v[4 * t + 2] = __builtin_bit_cast(float, xv[i][t].z);
-                v[4 * t + 3] = __builtin_bit_cast(float, xv[i][t].w);
-            }
-            float mx = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) mx = fmaxf(mx, fabsf(v[e]));
-            mx = fmaxf(mx, __shfl_xor(mx, 1, kWave));
-            const int sh = fp16_range_shift(mx);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                uint32_t hi[4], lo[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float u = __builtin_amdgcn_ldexpf(v[4 * j + q], sh), w = __builtin_amdgcn_ldexpf(v[8 + 4 * j + q], sh);
-                    const _Float16 hu = (_Float16)u, hw = (_Float16)w;
-                    const _Float16 lu = (_Float16)(__builtin_isinf(u) ? 0.0f : u - (float)hu);
-                    const _Float16 lw = (_Float16)(__builtin_isinf(w) ? 0.0f : w - (float)hw);
-                    hi[q] = (uint32_t)h_bits(hu) | ((uint32_t)h_bits(hw) << 16);
-                    lo[q] = (uint32_t)h_bits(lu) | ((uint32_t)h_bits(lw) << 16);
-                }
-                xh[(2 * h + j) * G + idx] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                xl[(2 * h + j) * G + idx] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            }
-            if (h == 0) back[idx] = __builtin_amdgcn_ldexpf(1.0f, -sh);
+            for (int t = 0; t < 4; ++t)
+                xs[(2 * (2 * h + (t & 1)) + (t >> 1)) * G + idx] = __builtin_bit_cast(f4, xv[i][t]);
         }
     }
     __syncthreads();
@@ -120,40 +96,40 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
         const int ci = lane + 64 * c, cc = min(ci, G - 1);
-        float p[R];
+        float pl[R], ph[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) p[r] = 0.0f;
+        for (int r = 0; r < R; ++r) pl[r] = ph[r] = 0.0f;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint4 hq = xh[t * G + cc], lq = xl[t * G + cc];
-            const uint32_t hp[4] = {hq.x, hq.y, hq.z, hq.w}, lp[4] = {lq.x, lq.y, lq.z, lq.w};
+            const f4 xl = xs[2 * t * G + cc], xh = xs[(2 * t + 1) * G + cc];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const uint32_t d = wv[r][c][t];
-                const h2 w[4] = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 1),
-                                 __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.0f, 3)};
+                const f32x2_t w[4] = {__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(d, 2.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(d, 2.0f, 1),
+                                      __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(d, 2.0f, 2), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(d, 2.0f, 3)};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    p[r] = __builtin_amdgcn_fdot2(bits_h2(hp[q]), w[q], p[r], false);
-                    p[r] = __builtin_amdgcn_fdot2(bits_h2(lp[q]), w[q], p[r], false);
+                    pl[r] = fmaf(xl[q], w[q][0], pl[r]);
+                    ph[r] = fmaf(xh[q], w[q][1], ph[r]);
                 }
             }
         }
-        const float b = back[cc];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const float s = table[sb[r][c] & 255u];
+            const float s = table[16 + (sb[r][c] & 255u)], hs = 0.5f * s, p = pl[r] + ph[r];
             if (ci < G) {
-                if (__builtin_isfinite(s)) {
-                    acc[r] = fmaf(s, p[r] * b, acc[r]);
+                if (fabsf(s) <= kScaleMax && hs + hs == s && __builtin_isfinite(p)) {
+                    acc[r] = fmaf(hs, p, acc[r]);
                 } else {
-                    const float* const x = static_cast<const float*>(a.x) + 32 * (size_t)ci;
-#pragma unroll 1
-                    for (int j = 0; j < 16; ++j) {
-                        const uint32_t w4 = j < 4 ? wv[r][c][0] : j < 8 ? wv[r][c][1] : j < 12 ? wv[r][c][2] : wv[r][c][3];
-                        const h2 w = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w4 >> (8 * (j & 3)), 1.0f, 0);
-                        acc[r] = fmaf(x[j], (float)w[0] * s, acc[r]);
-                        acc[r] = fmaf(x[j + 16], (float)w[1] * s, acc[r]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const f4 xl = xs[2 * t * G + cc], xh = xs[(2 * t + 1) * G + cc];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const uint32_t b = wv[r][c][t] >> (8 * q);
+                            acc[r] = fmaf(xl[q], table[b & 15u] * s, acc[r]);
+                            acc[r] = fmaf(xh[q], table[(b >> 4) & 15u] * s, acc[r]);
+                        }
                     }
                 }
             }
@@ -169,7 +145,7 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
 template <int CPL>
 void launch_cpl(const GemmArgs& a) {
     const int G = a.K / 32;
-    const size_t lds = (size_t)G * 128 + (size_t)G * 4 + 256 * 4;
+    const size_t lds = (size_t)G * 128 + 272 * 4;
     const dim3 grid((a.N + 4 * kRows - 1) / (4 * kRows));
     switch (a.y_dtype) {
     case BYHIP_F32: launch("fp4_gemv", (fp4_gemv<CPL, BYHIP_F32>), grid, dim3(256), lds, a); break;

@@ -1,0 +1,124 @@
+"""FP4-KM with fp32 activations: the reference forms value * scale in fp32 and multiplies the fp32
+activation with it (cpu_vm.c:583-628), so every bit of an activation counts, whatever its size beside its
+neighbours', and no product leaves fp32's range that the reference's does not.
+
+Bar: against the result in 64 bits, the roundings of an fp32 sum. Each of the K products and additions
+may round once (2^-24 of what it holds), in any order at most |error| <= K 2^-24 sum |x w|, and sums
+formed as trees or chains of a few dozen stay far below: 64 2^-24 sum |x w| (3.8e-6) is the bar.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BAR = 64 * 2.0 ** -24
+
+
+def mx_table():
+    from bybylang_amd import synth
+    t = np.zeros(272, np.float32)
+    t[:16] = synth.E2M1
+    with np.errstate(over="ignore"):
+        t[16:] = np.ldexp(np.float32(1), np.arange(256) - 127)
+    return t
+
+
+def run(hip, x, codes, sb, t):
+    from bybylang_amd import synth
+    M, K = x.shape
+    N = codes.shape[0]
+    blob = np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.astype(np.uint8).reshape(-1)])
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.fp4km_tile_gemm(hip.DeviceBuffer.from_array(np.ascontiguousarray(x, np.float32).reshape(-1)), hip.F32,
+                        hip.DeviceBuffer.from_array(blob), N * (K // 2), hip.DeviceBuffer.from_array(t), 0, y, hip.F32, M, K, N)
+    return y.read(np.float32).reshape(M, N)
+
+
+def exact(x, codes, sb, t):
+    """(x . W^T, |x| . |W|^T) in 64 bits, the weights rounded to fp32 as the reference forms them."""
+    with np.errstate(over="ignore", invalid="ignore"):
+        w = (t[codes] * np.repeat(t[16 + sb.astype(np.int64)], 32, axis=1)).astype(np.float64)
+        return x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T
+
+
+def check(got, x, codes, sb, t):
+    want, size = exact(x, codes, sb, t)
+    assert np.all(np.isfinite(want)) and np.all(np.isfinite(got))
+    err = np.abs(got - want) / np.maximum(size, 2.0 ** -126)
+    assert err.max() <= BAR, f"{err.max():.3g} of sum |x w| at {np.unravel_index(err.argmax(), err.shape)}"
+
+
+@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("lead", [-10, -20, -30])
+def test_small_activations_beside_large_ones(hip, M, lead):
+    """The first activations of each 32-value group are 2^-lead times the others, and their codes zero:
+    the results are sums of the small ones alone."""
+    from bybylang_amd import synth
+    g = synth.rng(100 * M - lead)
+    K, N = 512, 40
+    x = synth.activations(g, M, K, np.float32)
+    codes = g.integers(1, 8, size=(N, K), dtype=np.uint8) | (g.integers(0, 2, size=(N, K), dtype=np.uint8) << 3)
+    big = np.arange(K) % 32 < 3
+    x[:, ~big] *= np.float32(2.0 ** lead)
+    codes[:, big] = 0
+    sb = g.integers(120, 130, size=(N, K // 32))
+    check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
+
+
+@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("spread,byte", [(8, 127), (26, 113), (60, 127)])
+def test_groups_of_small_activations_on_large_weights(hip, M, spread, byte):
+    """Group i of a row holds activations of about 2^-e, e up to `spread`, each column's scale there is 2^(e +
+    byte - 127): every group counts alike. (26, 113) keeps every product within fp16's range."""
+    from bybylang_amd import synth
+    g = synth.rng(7 * M + spread)
+    K, N = 1024, 70
+    e = g.integers(0, spread + 1, size=K // 32)
+    x = synth.activations(g, M, K, np.float32) * np.repeat(2.0 ** -e, 32).astype(np.float32)
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    sb = np.broadcast_to(byte + e, (N, K // 32)) + g.integers(-1, 2, size=(N, K // 32))
+    check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
+
+
+@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("size,byte", [(1.5 * 2.0 ** 126, 117), (2.0 ** 120, 100), (2.0 ** 126, 60), (2.0 ** -126, 180), (2.0 ** -140, 230)])
+def test_activations_at_the_ends_of_fp32(hip, M, size, byte):
+    """Activations up to 1.5 2^126, whose sums with codes alone pass 2^128, on scales that bring them back,
+    and subnormal ones on large scales."""
+    from bybylang_amd import synth
+    g = synth.rng(M + byte)
+    K, N = 256, 33
+    x = (g.uniform(0.5, 1.0, (M, K)) * size).astype(np.float32)
+    codes = g.integers(1, 8, size=(N, K), dtype=np.uint8)
+    codes[:, :4] = 7
+    sb = np.full((N, K // 32), byte)
+    check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
+
+
+@pytest.mark.parametrize("M", [1])
+def test_products_that_overflow_or_vanish(hip, oracle, M):
+    """Scale entries of zero, 2^126 and 2^127 (value * scale overflows for the larger codes), subnormal
+    ones, and a huge activation beside them: infinities and NaNs where the reference has them."""
+    from bybylang_amd import synth
+    g = synth.rng(900 + M)
+    K, N = 256, 64
+    t = mx_table()
+    t[16 + 10] = 0.0
+    t[16 + 11] = 2.0 ** -149
+    t[16 + 12] = 3 * 2.0 ** -149
+    x = synth.activations(g, M, K, np.float32)
+    x[:, 5] = 2.0 ** 127
+    x[:, 70] = 0.0
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    sb = np.full((N, K // 32), 100)
+    sb[:, 0] = np.array([10, 11, 12, 0, 1, 90])[np.arange(N) % 6]
+    sb[:32, 2] = np.array([253, 254, 255, 252])[np.arange(32) % 4]
+    got = run(hip, x, codes, sb, t)
+    blob = np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.astype(np.uint8).reshape(-1)])
+    want = np.asarray(oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x.reshape(-1))).reshape(M, N)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+    fin = np.isfinite(want)
+    _, size = exact(x, codes, sb, t)
+    assert np.all(np.abs(got[fin] - want[fin]) <= 2 * BAR * size[fin])
