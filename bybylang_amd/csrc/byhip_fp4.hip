@@ -3,8 +3,8 @@
 //
 // FP4-KM (cpu_vm.c:583-628): weight = lut[nibble] * lut[16 + scale byte] with the 272-float decode
 // table; nibble bytes [N, K/2] (byte j of a group: element j low, j + 16 high), scale bytes
-// [N, K/32] at scale_base. fp32 activations and E2M1 values with any scale entries take one row on the
-// decode GEMV (byhip_fp4gemv.hip) and more on the two-plane GEMM (byhip_planes.hip); other tables whose
+// [N, K/32] at scale_base. One row of fp32 activations takes the decode GEMV (byhip_fp4gemv.hip), more
+// on E2M1 values with any scale entries the two-plane GEMM (byhip_planes.hip); other tables whose
 // products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
 // the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
 // exactly E2M1 and 2^(e-127).
@@ -135,7 +135,8 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
     GemmArgs a;
     a.x = x; a.x_dtype = x_dtype; a.y = y; a.y_dtype = y_dtype; a.M = M; a.K = K; a.N = N;
     a.blob = blob; a.scale_base = scale_base; a.lut = lut + lut_base;
-    // fp32 activations and an E2M1 table: the decode GEMV for one row, else the two-plane kernel. Else the general fp16 MFMA kernel when
+    // One row of fp32 activations: the decode GEMV, which takes any table. More and an E2M1 table: the
+    // two-plane kernel. Else the general fp16 MFMA kernel when
     // every decoded weight is a half, otherwise the exact fp32 GEMM. The table is classified on the
     // host from its host copy, outside recordings; otherwise on the device, by a kernel that writes
     // the choice to a flag, with all routes queued behind it and each gated on the flag, so that a
@@ -143,15 +144,15 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
     // waits for the device to read the table.
     const bool aligned = reinterpret_cast<uintptr_t>(blob) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
     if (aligned && env_int("BYHIP_TILE_EXACT", 0) == 0) {
-        const bool gemv = fp4_gemv_ok(a), e2m1 = gemv || gemm_planes_ok(BFormat::Fp4Km, a);
-        auto launch_e2m1 = [&](const GemmArgs& g) {
-            if (gemv) launch_fp4_gemv(g);
-            else launch_gemm_planes(BFormat::Fp4Km, g);
-        };
+        if (fp4_gemv_ok(a)) {
+            launch_fp4_gemv(a);
+            return;
+        }
+        const bool e2m1 = gemm_planes_ok(BFormat::Fp4Km, a);
         float t[272];
         if (!session_recording() && mirror_read(lut, lut_base * 4, t, sizeof t)) {
             if (e2m1 && table_is_e2m1(t)) {
-                launch_e2m1(a);
+                launch_gemm_planes(BFormat::Fp4Km, a);
                 return;
             }
             if (table_products_are_halves(t)) {
@@ -166,7 +167,7 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
             g.gate = flag;
             if (e2m1) {
                 g.gate_want = kTableE2m1;
-                launch_e2m1(g);
+                launch_gemm_planes(BFormat::Fp4Km, g);
             }
             g.gate_want = kTableHalves;
             launch_gemm(BFormat::Fp4Km, g);

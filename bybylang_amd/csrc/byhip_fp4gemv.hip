@@ -1,17 +1,20 @@
 // byhip_fp4gemv.hip - the FP4-KM decode GEMV (one row of fp32 activations, gfx950).
 //
-// y[n] = sum_k x[k] * lut[code] * lut[16 + scale byte] for tables whose 16 values are E2M1's. Work
-// split and arithmetic follow the Q4 decode GEMV (byhip_gemv.hip): a wave owns kRows weight rows,
+// y[n] = sum_k x[k] * lut[code] * lut[16 + scale byte] for any decode table. The work is split as in the Q4
+// decode GEMV (byhip_gemv.hip): a wave owns kRows weight rows,
 // lane l the 32-value groups l, l + 64, .. of each (one 16-byte load and one scale byte); every load
 // goes out before the first wait, activations, scale bytes, then weights.
 //
 // Activations stay fp32, staged once per block in LDS as the runs of four that four bytes of a group
-// multiply: low nibbles x[4 t ..], high nibbles x[16 + 4 t ..]. v_cvt_scalef32_pk_f32_fp4 turns a byte into
+// multiply: low nibbles x[4 t ..], high nibbles x[16 + 4 t ..]. Where the table's 16 values are E2M1's, which
+// each wave sees for itself, v_cvt_scalef32_pk_f32_fp4 turns a byte into
 // twice its two values, whole numbers, so products with subnormal activations stay exact too; two
 // chains of fp32 FMAs sum a group, and half its scale multiplies the sum. Where that order differs from
 // the reference's x * (value * scale) by more than rounding, the group is computed element by element as
 // the reference does: a sum that is not finite (activations near fp32's largest, infinities, NaNs), a
-// scale whose product with 6 overflows or with 0.5 is not exact.
+// scale whose product with 6 overflows or with 0.5 is not exact. Other tables take that form throughout,
+// their values looked up in LDS (11.4 us, 51 on the general GEMM; recorded calls, which had queued every route
+// behind a look at the table, 7.0 us for 19.7 with E2M1 values and 10.4 for 57.9 with others).
 //
 // What bounds it: K = 4096, N = 14336, 31.2 MB: 6.9 us against 6.4 for the bytes at the rate of a
 // large copy (8.9 us with two fp16 terms per activation and v_dot2_f32_f16, which held 23 bits of them and
@@ -29,9 +32,13 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 constexpr int kRows = 2;  // rows per wave, as the Q4 GEMV at one activation row
 constexpr float kScaleMax = 0x1p125f;  // products of scales up to here with 6 are finite
 
+__device__ constexpr uint32_t e2m1_bits(int i) {  // fp32 bits of the E2M1 value of code i
+    constexpr uint32_t v[8] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u, 0x40C00000u};
+    return v[i & 7] | (i & 8 ? 0x80000000u : 0u);
+}
+
 template <int CPL, int YT>
 __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
-    if (a.gate && *a.gate != a.gate_want) return;  // another route was chosen (whole grid)
     constexpr int R = kRows;
     constexpr int XC = (CPL + 1) / 2;  // half groups a thread stages: 2 G <= 128 CPL over 256 threads
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
@@ -89,6 +96,7 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
     }
     __syncthreads();
     if (n0 >= N) return;
+    const bool e2m1 = __all(__builtin_bit_cast(uint32_t, lut_e) == e2m1_bits(lane & 15));
 
     float acc[R];
 #pragma unroll
@@ -100,7 +108,7 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
 #pragma unroll
         for (int r = 0; r < R; ++r) pl[r] = ph[r] = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < (e2m1 ? 4 : 0); ++t) {
             const f4 xl = xs[2 * t * G + cc], xh = xs[(2 * t + 1) * G + cc];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
@@ -118,7 +126,7 @@ __global__ __launch_bounds__(256) void fp4_gemv(GemmArgs a) {
         for (int r = 0; r < R; ++r) {
             const float s = table[16 + (sb[r][c] & 255u)], hs = 0.5f * s, p = pl[r] + ph[r];
             if (ci < G) {
-                if (fabsf(s) <= kScaleMax && hs + hs == s && __builtin_isfinite(p)) {
+                if (e2m1 && fabsf(s) <= kScaleMax && hs + hs == s && __builtin_isfinite(p)) {
                     acc[r] = fmaf(hs, p, acc[r]);
                 } else {
 #pragma unroll

@@ -193,13 +193,8 @@ void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
 
-// The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, a table with E2M1's values
-// and any scales, K % 32 == 0 up to 15,360.
-bool fp4_gemv_ok(const GemmArgs& a);
-void launch_fp4_gemv(const GemmArgs& a);
-
-// The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, a table with E2M1's values
-// and any scales, K % 32 == 0 up to 15,360.
+// The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, any decode table, K % 32 == 0
+// up to 15,360, 16-byte aligned operands. It reads no gate.
 bool fp4_gemv_ok(const GemmArgs& a);
 void launch_fp4_gemv(const GemmArgs& a);
 

@@ -122,3 +122,45 @@ def test_products_that_overflow_or_vanish(hip, oracle, M):
     fin = np.isfinite(want)
     _, size = exact(x, codes, sb, t)
     assert np.all(np.abs(got[fin] - want[fin]) <= 2 * BAR * size[fin])
+
+
+@pytest.mark.parametrize("K,N", [(32, 3), (2080, 33), (4096, 130), (15360, 9)])
+@pytest.mark.parametrize("recorded", [False, True])
+def test_one_row_takes_any_table(hip, oracle, recorded, K, N):
+    """One row on E2M1 with E8M0 scales, on values that are not E2M1's, on scales that are not halves: the
+    same recording follows the table the buffer holds at each replay."""
+    from bybylang_amd import _abi, synth
+    from bybylang_amd import gpubackend as gb
+    g = synth.rng(K + N)
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    sb = g.integers(118, 136, size=(N, K // 32), dtype=np.uint8)
+    x = synth.activations(g, 1, K, np.float32)
+    mx = mx_table()
+    values = mx.copy()
+    values[:16] = g.standard_normal(16)
+    scales = mx.copy()
+    scales[16:] = np.exp(g.normal(0, 2, 256))
+    minus = mx.copy()
+    minus[8] = 0.0  # E2M1 but for the sign of its second zero
+    if not recorded:
+        for t in (mx, values, scales, minus):
+            check(run(hip, x, codes, sb, t), x, codes, sb, t)
+        return
+    blob = np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.reshape(-1)])
+    words = np.zeros((blob.size + 3) // 4, np.float32)
+    words.view(np.uint8)[: blob.size] = blob
+    assert gb.sessionBegin(gb.gbHip)
+    hx, hw, ht = (gb.sessionUpload(gb.gbHip, v) for v in (x.reshape(-1), words, mx))
+    ho = gb.sessionAllocScratch(gb.gbHip, N)
+    assert gb.sessionEnd(gb.gbHip)
+    assert gb.sessionBeginRecording(gb.gbHip)
+    assert gb.sessionFp4GemmTensorCore(gb.gbHip, hx, hw, ht, ho, 1, K, N)
+    assert gb.sessionEnd(gb.gbHip), gb.sessionGetLastError(gb.gbHip)
+    rid = gb.sessionLastRecording(gb.gbHip)
+    for t in (mx, values, scales, minus, mx):
+        _abi.check(_abi.load().byhip_upload(ht.hipHandle, 0, t.ctypes.data, t.nbytes))
+        assert gb.sessionReplay(gb.gbHip, rid, 1), gb.sessionGetLastError(gb.gbHip)
+        check(np.asarray(gb.sessionRead(gb.gbHip, ho, N)).reshape(1, N), x, codes, sb, t)
+    gb.sessionFreeRecording(gb.gbHip, rid)
+    for h in (hx, hw, ht, ho):
+        gb.sessionFree(gb.gbHip, h)
