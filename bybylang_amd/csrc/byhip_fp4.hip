@@ -4,8 +4,8 @@
 // FP4-KM (cpu_vm.c:583-628): weight = lut[nibble] * lut[16 + scale byte] with the 272-float decode
 // table; nibble bytes [N, K/2] (byte j of a group: element j low, j + 16 high), scale bytes
 // [N, K/32] at scale_base. One row of fp32 activations takes the decode GEMV (byhip_fp4gemv.hip), more
-// on E2M1 values with any scale entries the two-plane GEMM (byhip_planes.hip); other tables whose
-// products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
+// on E2M1 / E8M0 tables or E2M1 values whose products are halves gemm_planes (byhip_planes.hip); other
+// tables whose products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
 // the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
 // exactly E2M1 and 2^(e-127).
 #include <algorithm>
@@ -80,29 +80,40 @@ bool table_products_are_halves(const float* t) {
     return ok;
 }
 
-// The route of a decode table: kTableE2m1 when its 16 values are E2M1's bit for bit (gemm_planes, fp4_gemv),
-// else kTableHalves when every product is a half, else kTableAny.
-enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2 };
+// The class of a decode table, which the route of fp32 activations goes by:
+//   kTableMx      E2M1's 16 values bit for bit and the scales 2^(b - 127) up to byte 252 (a larger one's
+//                 products may overflow; the kernel looks out for those bytes)
+//   kTableE2m1    E2M1's values, and every product a half
+//   kTableHalves  every product a half
+//   kTableAny     any other
+enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2, kTableMx = 3 };
 
-bool table_is_e2m1(const float* t) { return memcmp(t, kE2M1, sizeof kE2M1) == 0; }
+int table_class(const float* t) {
+    const bool e2m1 = memcmp(t, kE2M1, sizeof kE2M1) == 0;
+    bool mx = e2m1;
+    for (int b = 0; b < 253 && mx; ++b) mx = t[16 + b] == std::ldexp(1.0f, b - 127);
+    if (mx) return kTableMx;
+    return !table_products_are_halves(t) ? kTableAny : e2m1 ? kTableE2m1 : kTableHalves;
+}
 
-// Device-side form of the choice: thread b checks the 16 products with scale entry b (finite, and
-// exact in fp16), and the block's AND goes to *flag; `e2m1_route`: whether a kernel for E2M1's values
-// takes the call.
-__global__ __launch_bounds__(256) void fp4km_classify(const float* __restrict__ t, int e2m1_route, int* flag) {
-    constexpr uint32_t e2m1[16] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u,
+// The same on the device, for the routes that are queued: `mx` and `e2m1` say whether those classes'
+// kernels are, otherwise such tables count as the next class. Thread b checks scale entry b.
+__global__ __launch_bounds__(256) void fp4km_classify(const float* __restrict__ t, int mx, int e2m1, int* flag) {
+    constexpr uint32_t bits[16] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u,
                                    0x40C00000u, 0x80000000u, 0xBF000000u, 0xBF800000u, 0xBFC00000u, 0xC0000000u,
                                    0xC0400000u, 0xC0800000u, 0xC0C00000u};
-    const float s = t[16 + threadIdx.x];
-    bool ok = true, same = e2m1_route != 0;
+    const uint32_t b = threadIdx.x;
+    const float s = t[16 + b];
+    bool halves = true, same = true;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const float p = t[i] * s;
-        ok = ok && __builtin_isfinite(p) && (float)(_Float16)p == p;
-        same = same && __builtin_bit_cast(uint32_t, t[i]) == e2m1[i];
+        halves = halves && __builtin_isfinite(p) && (float)(_Float16)p == p;
+        same = same && __builtin_bit_cast(uint32_t, t[i]) == bits[i];
     }
-    ok = __syncthreads_and(ok);
-    if (threadIdx.x == 0) *flag = same ? kTableE2m1 : ok ? kTableHalves : kTableAny;
+    halves = __syncthreads_and(halves);
+    const bool e8m0 = __syncthreads_and(b >= 253u || __builtin_bit_cast(uint32_t, s) == (b ? b << 23 : 0x00400000u));
+    if (b == 0) *flag = same && e8m0 && mx ? kTableMx : !halves ? kTableAny : same && e2m1 ? kTableE2m1 : kTableHalves;
 }
 
 void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_bytes, size_t scale_base,
@@ -135,12 +146,12 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
     GemmArgs a;
     a.x = x; a.x_dtype = x_dtype; a.y = y; a.y_dtype = y_dtype; a.M = M; a.K = K; a.N = N;
     a.blob = blob; a.scale_base = scale_base; a.lut = lut + lut_base;
-    // One row of fp32 activations: the decode GEMV, which takes any table. More and an E2M1 table: the
-    // two-plane kernel. Else the general fp16 MFMA kernel when
-    // every decoded weight is a half, otherwise the exact fp32 GEMM. The table is classified on the
-    // host from its host copy, outside recordings; otherwise on the device, by a kernel that writes
-    // the choice to a flag, with all routes queued behind it and each gated on the flag, so that a
-    // recording replays the right route for whatever table the buffer holds at replay, and no call
+    // One row of fp32 activations: the decode GEMV, which takes any table. More: the three-term kernel for
+    // an E8M0 table, the two-plane kernel for E2M1 values whose products are halves. Else the general fp16
+    // MFMA kernel when every decoded weight is a half, otherwise the exact fp32 GEMM. The table is
+    // classified on the host from its host copy, outside recordings; otherwise on the device, by a kernel
+    // that writes the choice to a flag, with all routes queued behind it and each gated on the flag, so
+    // that a recording replays the right route for whatever table the buffer holds at replay, and no call
     // waits for the device to read the table.
     const bool aligned = reinterpret_cast<uintptr_t>(blob) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
     if (aligned && env_int("BYHIP_TILE_EXACT", 0) == 0) {
@@ -148,23 +159,32 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
             launch_fp4_gemv(a);
             return;
         }
-        const bool e2m1 = gemm_planes_ok(BFormat::Fp4Km, a);
+        const bool mx = fp4_mx_ok(a), e2m1 = gemm_planes_ok(BFormat::Fp4Km, a);
         float t[272];
         if (!session_recording() && mirror_read(lut, lut_base * 4, t, sizeof t)) {
-            if (e2m1 && table_is_e2m1(t)) {
+            const int cls = table_class(t);
+            if (cls == kTableMx && mx) {
+                launch_fp4_mx(a);
+                return;
+            }
+            if (cls == kTableE2m1 && e2m1) {
                 launch_gemm_planes(BFormat::Fp4Km, a);
                 return;
             }
-            if (table_products_are_halves(t)) {
+            if (cls == kTableE2m1 || cls == kTableHalves) {
                 launch_gemm(BFormat::Fp4Km, a);
                 return;
             }
         } else {
             int* flag = device_flags();
             launch("fp4km_classify", fp4km_classify, dim3(1), dim3(256), 0, static_cast<const float*>(lut + lut_base),
-                   (int)e2m1, flag);
+                   (int)mx, (int)e2m1, flag);
             GemmArgs g = a;
             g.gate = flag;
+            if (mx) {
+                g.gate_want = kTableMx;
+                launch_fp4_mx(g);
+            }
             if (e2m1) {
                 g.gate_want = kTableE2m1;
                 launch_gemm_planes(BFormat::Fp4Km, g);

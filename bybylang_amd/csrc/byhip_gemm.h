@@ -60,8 +60,6 @@ struct GemmArgs {
     // The wide tile on fp32 activations: x holds the high fp16 plane of the shifted activations and
     // x_lo the low one (x * 2^t = hi + lo, t per row in row_shift).
     const void* x_lo = nullptr;
-    // gemm_planes: the fp32 activations themselves (x and x_lo hold their planes).
-    const void* x_raw = nullptr;
     // A device-side route choice: when gate is set, the general fp16 MFMA GEMM, the exact GEMM and
     // their split-K sum do nothing unless *gate == gate_want (the flag a classification kernel
     // earlier on the stream wrote), so two routes can be queued and only the chosen one runs.
@@ -186,12 +184,17 @@ int stream_fn(const GemmArgs& a, int row_blocks);
 int stream_row_blocks(const GemmArgs& a);
 void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 
-// fp32 activations as two fp16 planes against FP4-KM weights with an E2M1 table, or half weights
-// (byhip_planes.hip): whether the kernel takes the call (K % 128 == 0 for FP4-KM, K % 64 == 0 for F16,
-// 16-byte aligned operands, offsets below 2^31), and the launch. FP4-KM tables other than E2M1 give
-// the same results, slowly.
+// fp32 activations as two fp16 planes (byhip_planes.hip) against FP4-KM weights with an E2M1 table whose
+// products are all halves, half weights, or the prefill copy of Q4 weights: whether the kernel takes the
+// call (K % 128 == 0 for FP4-KM, else K % 64 == 0, 16-byte aligned operands, offsets below 2^31), and the launch.
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
+
+// fp32 activations as three bf16 terms (byhip_fp4mx.hip) against FP4-KM weights with E2M1's values and the
+// scales 2^(b - 127); entries 253 to 255 may hold anything. K % 128 == 0, 16-byte aligned operands,
+// offsets below 2^31.
+bool fp4_mx_ok(const GemmArgs& a);
+void launch_fp4_mx(const GemmArgs& a);
 
 // The FP4-KM decode GEMV (byhip_fp4gemv.hip): one row of fp32 activations, any decode table, K % 32 == 0
 // up to 15,360, 16-byte aligned operands. It reads no gate.

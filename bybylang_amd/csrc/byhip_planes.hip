@@ -4,9 +4,7 @@
 // (undone on the output) and split into hi = fp16(x) and lo = fp16(x - hi), about 23 bits of x
 // (split_planes); hi . w + lo . w in v_mfma_f32_16x16x32_f16 with fp32 accumulation then keeps
 // them, for weights that are exact in fp16:
-//   FP4-KM with an E2M1 table and scales whose products with it are halves (checked per scale byte
-//          while it is used; a block that meets another scale, or a table that is not E2M1,
-//          computes its tile again in fp32 arithmetic as the reference does)
+//   FP4-KM with E2M1 values and scales whose products with them are all halves
 //   F16    (gemm_planes_half, below, where both operands go through LDS)
 //   Q4     on the prefill copy: the codes less their zero (whole numbers) go through the MFMAs, and each
 //          32-value group's sums are scaled in fp32. Two MFMAs per product where weights as two fp16
@@ -49,7 +47,6 @@ constexpr int kDepth = 4;             // activation buffers per K group
 constexpr int kSets = 4;              // weight register sets
 constexpr int kUnroll = 8;            // sub-steps per loop iteration
 constexpr int kPitch = kBN + 4;       // floats per row of a staged partial tile
-constexpr uint32_t kUnsafe = 0xFFFFu;      // (a NaN) a scale whose products with E2M1 are not all halves
 constexpr uint32_t kPast = 0x80000000u;    // added to an offset: every resource here rejects it
 
 template <int FM>
@@ -61,64 +58,6 @@ struct PlaneShape {
     static constexpr int kLds = kLdsX > kLdsRed ? kLdsX : kLdsRed;
 };
 
-__device__ constexpr uint32_t e2m1_bits(int i) {  // fp32 bits of the E2M1 value of code i
-    constexpr uint32_t v[8] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u, 0x40C00000u};
-    return v[i & 7] | (i & 8 ? 0x80000000u : 0u);
-}
-
-// The block's tile in fp32 arithmetic, each weight lut[code] * lut[16 + scale byte] as the
-// reference forms it, x in fp32, v_mfma_f32_16x16x4_f32: wave w computes columns 16 w .. + 15 over
-// 32-value groups g0 .. g1 - 1 and leaves its sums in `red`.
-template <int FM>
-__device__ __forceinline__ void fp4_tile_exact(const GemmArgs& a, int m0, int n0, int g0, int g1,
-                                               float* red) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-    const int n = n0 + 16 * wid + c;
-    const float* const x = static_cast<const float*>(a.x_raw);
-    const float* const lut = a.lut;
-    f4 acc[FM];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) acc[i] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-    for (int G = g0; G < g1; ++G) {
-        uint32_t w = 0;
-        float s = 0.0f;
-        if (n < a.N) {
-            w = *reinterpret_cast<const uint32_t*>(a.blob + (size_t)n * (a.K >> 1) + 16 * (size_t)G + 4 * g);
-            s = lut[16 + a.blob[a.scale_base + (size_t)n * (a.K >> 5) + G]];
-        }
-        float wl[4], wh[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            wl[j] = n < a.N ? lut[(w >> (8 * j)) & 15u] * s : 0.0f;
-            wh[j] = n < a.N ? lut[(w >> (8 * j + 4)) & 15u] * s : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const int m = m0 + 16 * i + c;
-            float4 xl = make_float4(0.0f, 0.0f, 0.0f, 0.0f), xh = xl;
-            if (m < a.M) {
-                const float* r = x + (size_t)m * a.K + 32 * (size_t)G + 4 * g;
-                xl = *reinterpret_cast<const float4*>(r);
-                xh = *reinterpret_cast<const float4*>(r + 16);
-            }
-            const float al[4] = {xl.x, xl.y, xl.z, xl.w}, ah[4] = {xh.x, xh.y, xh.z, xh.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(al[j], wl[j], acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[j], wh[j], acc[i], 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int at = (16 * i + 4 * g + r) * kPitch + 16 * wid + c;
-            red[at] = acc[i][r];
-            red[16 * FM * kPitch + at] = 0.0f;  // the second K group's partial tile
-        }
-}
-
 template <BFormat F, int FM, int YT, bool ZG = false>
 __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 4 : 2) void gemm_planes(GemmArgs a) {
     if (a.gate && *a.gate != a.gate_want) return;  // another route was chosen (whole grid)
@@ -127,11 +66,10 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     constexpr int WV = 2;  // weight registers of a set, in 16-byte units
     using S = PlaneShape<FM>;
     constexpr int BM = S::kBM, kXBuf = S::kXBuf;
-    // One LDS array for everything, the eight waves' `bad` words at its end: beside a second array (a
-    // table of its own, or the one inside __syncthreads_or) the compiler no longer told the direct
-    // loads from the fragment reads apart and waited for every load in flight before each read: 47 us
-    // instead of 43 at M = 512, K = N = 4096.
-    __shared__ __attribute__((aligned(16))) uint8_t lds[S::kLds + 32];
+    // One LDS array for everything: beside a second one (a table, or the one inside __syncthreads_or) the
+    // compiler no longer told the direct loads from the fragment reads apart and waited for every load
+    // in flight before each read: 47 us instead of 43 at M = 512, K = N = 4096.
+    __shared__ __attribute__((aligned(16))) uint8_t lds[S::kLds];
 
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int p = wid & 1, h = wid >> 1;
@@ -154,15 +92,12 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     const int slices = min(2 * steps, K / kSub - 2 * step0);
     const int pairs_all = (steps + 1) / 2, nt_all = 2 * pairs_all;  // per K group: its steps, sub-steps
 
-    // The table lives in registers: lane l holds scale entries 4 l .. 4 l + 3 as halves (kUnsafe: its
-    // products with E2M1 are not all halves), looked up across lanes.
+    // The scales live in registers as halves, entries 4 l .. 4 l + 3 in lane l, looked up across lanes.
     float lut_v[FP4 ? 4 : 1];
     uint32_t lut_h[FP4 ? 2 : 1];
-    bool bad = false;
     if constexpr (FP4) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) lut_v[i] = a.lut[16 + 4 * lane + i];
-        bad = lane < 16 && __builtin_bit_cast(uint32_t, a.lut[lane & 15]) != e2m1_bits(lane & 15);
     }
 
     const rsrc_t xr = make_rsrc(h < 2 ? a.x : a.x_lo, (uint32_t)((size_t)a.M * K * 2));
@@ -180,11 +115,9 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         xo[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + 16u * chunk;
     }
     uint32_t wo[FN], so[FN];
-    bool col_ok[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
         const int n = n0 + 32 * h + 16 * j + c;
-        col_ok[j] = n < a.N;
         wo[j] = FP4 ? (uint32_t)n * (uint32_t)(K >> 1) + 16u * g
                     : ((uint32_t)n >> 4) * nsub * 512u + 8u * c + 128u * (uint32_t)(g >> 1) + 4u * (uint32_t)(g & 1);
         so[j] = (uint32_t)n * (uint32_t)(K >> 5) + 8u * g;
@@ -235,16 +168,13 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
             d[j] = __builtin_amdgcn_raw_buffer_load_b32(sr, so[j] | past, 4u * (uint32_t)(step0 + s0), 0);
     };
     auto scale_of = [&](const uint32_t (&d)[FP4 ? FN : 1], int q, uint32_t (&s)[FP4 ? FN : 1]) __attribute__((always_inline)) {
-        const bool live = p + 2 * q < steps;
 #pragma unroll
         for (int j = 0; j < (FP4 ? FN : 0); ++j) {
             const uint32_t b = ((uint32_t)__builtin_amdgcn_ds_bpermute(4 * (16 * (q & 3) + c), (int)d[j]) >> (8 * g)) & 255u;
             const uint32_t v0 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(b & 252u), (int)lut_h[0]);
             const uint32_t v1 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(b & 252u), (int)lut_h[FP4 ? 1 : 0]);
             const uint32_t v = (((b & 2u) ? v1 : v0) >> (16 * (b & 1u))) & 0xFFFFu;
-            const bool use = live && col_ok[j];
-            bad = bad || (use && v == kUnsafe);
-            s[j] = use ? v | (v << 16) : 0u;
+            s[j] = v | (v << 16);  // columns past N and steps past the last: weights of zero
         }
     };
 
@@ -352,12 +282,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     if constexpr (FP4) {
         uint32_t b[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            // every product with E2M1 is a half when 0.5 v and 1.5 v are and 6 v is in range
-            const float v = lut_v[i], v1 = 0.5f * v, v3 = 1.5f * v;
-            const bool ok = fabsf(6.0f * v) <= 65504.0f && (float)(_Float16)v1 == v1 && (float)(_Float16)v3 == v3;
-            b[i] = ok ? h_bits((_Float16)v) : kUnsafe;
-        }
+        for (int i = 0; i < 4; ++i) b[i] = h_bits((_Float16)lut_v[i]);
         lut_h[0] = b[0] | (b[1] << 16);
         lut_h[1] = b[2] | (b[3] << 16);
     }
@@ -436,29 +361,15 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
     // Partial tiles -> LDS, once every wave's loads have landed and every wave is done with the
     // buffers -> the two groups' sums -> y or the split-K partials.
     wait_vmcnt<0>();
-    uint32_t* const bads = reinterpret_cast<uint32_t*>(lds + S::kLds);
-    if constexpr (FP4) {
-        const bool any = __any(bad);
-        if (lane == 0) bads[wid] = any ? 1u : 0u;
-    }
     __syncthreads();
-    bool redo = false;
-    if constexpr (FP4) {
-        const uint4 b0 = reinterpret_cast<const uint4*>(bads)[0], b1 = reinterpret_cast<const uint4*>(bads)[1];
-        redo = (b0.x | b0.y | b0.z | b0.w | b1.x | b1.y | b1.z | b1.w) != 0u;
-    }
     float* red = reinterpret_cast<float*>(lds);  // [2 groups][BM rows][kPitch]
-    if (redo) {
-        fp4_tile_exact<FM>(a, m0, n0, 4 * step0, min(4 * (step0 + steps), K / 32), red);
-    } else {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    red[(p * BM + 16 * i + 4 * g + r) * kPitch + 32 * h + 16 * j + c] = acc[i][j][r];
-    }
+            for (int r = 0; r < 4; ++r)
+                red[(p * BM + 16 * i + 4 * g + r) * kPitch + 32 * h + 16 * j + c] = acc[i][j][r];
     __syncthreads();
     float* part = a.part ? a.part + (size_t)blockIdx.z * splitk_stride(a.M, a.N) : nullptr;
     const bool vec = out8_vector_ok<YT>(a, part);
@@ -470,7 +381,7 @@ __global__ __launch_bounds__(512, FM == 1 || (FM == 2 && F == BFormat::Fp4Km) ? 
         const int m = m0 + row;
         if (m >= a.M) continue;
         const float* src = red + row * kPitch + col;
-        const int sh = redo ? 0 : a.row_shift[m];
+        const int sh = a.row_shift[m];
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; e += 4) {
@@ -857,7 +768,7 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
     for (size_t m = 0; m < (size_t)a0.M; m += rows) {
         GemmArgs a = a0;
         a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);
-        a.x_raw = static_cast<const float*>(a0.x) + m * a0.K;
+        const float* const x = static_cast<const float*>(a0.x) + m * a0.K;
         a.y = static_cast<uint8_t*>(a0.y) + m * a0.N * es;
         const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256;
         const size_t plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
@@ -866,10 +777,10 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
         uint8_t* const lo = hi + plane;
         if (fmt == BFormat::Fp4Km)
             launch("split_planes", split_planes<true>, dim3((unsigned)a.M), dim3(256), 0,
-                   static_cast<const float*>(a.x_raw), a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
+                   x, a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
         else
             launch("split_planes", split_planes<false>, dim3((unsigned)a.M), dim3(256), 0,
-                   static_cast<const float*>(a.x_raw), a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
+                   x, a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
         BYHIP_LAUNCHED("split_planes");
         a.x = hi;
         a.x_lo = lo;

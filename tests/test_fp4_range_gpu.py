@@ -48,7 +48,7 @@ def check(got, x, codes, sb, t):
     assert err.max() <= BAR, f"{err.max():.3g} of sum |x w| at {np.unravel_index(err.argmax(), err.shape)}"
 
 
-@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("M", [1, 2, 17, 70])
 @pytest.mark.parametrize("lead", [-10, -20, -30])
 def test_small_activations_beside_large_ones(hip, M, lead):
     """The first activations of each 32-value group are 2^-lead times the others, and their codes zero:
@@ -65,7 +65,7 @@ def test_small_activations_beside_large_ones(hip, M, lead):
     check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
 
 
-@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("M", [1, 2, 17, 70])
 @pytest.mark.parametrize("spread,byte", [(8, 127), (26, 113), (60, 127)])
 def test_groups_of_small_activations_on_large_weights(hip, M, spread, byte):
     """Group i of a row holds activations of about 2^-e, e up to `spread`, each column's scale there is 2^(e +
@@ -80,7 +80,7 @@ def test_groups_of_small_activations_on_large_weights(hip, M, spread, byte):
     check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
 
 
-@pytest.mark.parametrize("M", [1])
+@pytest.mark.parametrize("M", [1, 5, 40])
 @pytest.mark.parametrize("size,byte", [(1.5 * 2.0 ** 126, 117), (2.0 ** 120, 100), (2.0 ** 126, 60), (2.0 ** -126, 180), (2.0 ** -140, 230)])
 def test_activations_at_the_ends_of_fp32(hip, M, size, byte):
     """Activations up to 1.5 2^126, whose sums with codes alone pass 2^128, on scales that bring them back,
@@ -95,18 +95,23 @@ def test_activations_at_the_ends_of_fp32(hip, M, size, byte):
     check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
 
 
-@pytest.mark.parametrize("M", [1])
-def test_products_that_overflow_or_vanish(hip, oracle, M):
-    """Scale entries of zero, 2^126 and 2^127 (value * scale overflows for the larger codes), subnormal
-    ones, and a huge activation beside them: infinities and NaNs where the reference has them."""
+@pytest.mark.parametrize("table", ["mx", "other"])
+@pytest.mark.parametrize("M", [1, 40])
+def test_products_that_overflow_or_vanish(hip, oracle, M, table):
+    """Scale entries of 2^126 and 2^127 (value * scale overflows for the larger codes), infinity, zero and
+    subnormals, and a huge activation beside them: infinities and NaNs where the reference has them.
+    The activations on the largest scales are about 2^-8, so that no finite sum passes 2^128 in any
+    order of its additions."""
     from bybylang_amd import synth
     g = synth.rng(900 + M)
     K, N = 256, 64
     t = mx_table()
-    t[16 + 10] = 0.0
-    t[16 + 11] = 2.0 ** -149
-    t[16 + 12] = 3 * 2.0 ** -149
+    if table == "other":
+        t[16 + 10] = 0.0
+        t[16 + 11] = 2.0 ** -149
+        t[16 + 12] = 3 * 2.0 ** -149
     x = synth.activations(g, M, K, np.float32)
+    x[:, 64:96] *= np.float32(2.0 ** -8)
     x[:, 5] = 2.0 ** 127
     x[:, 70] = 0.0
     codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
@@ -164,3 +169,24 @@ def test_one_row_takes_any_table(hip, oracle, recorded, K, N):
     gb.sessionFreeRecording(gb.gbHip, rid)
     for h in (hx, hw, ht, ho):
         gb.sessionFree(gb.gbHip, h)
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("M,K,N", [(2, 128, 1), (16, 2432, 129), (17, 2176, 128), (40, 1152, 200), (63, 640, 127), (64, 2304, 130), (65, 4224, 40), (129, 256, 300)])
+def test_three_term_tiles(hip, monkeypatch, M, K, N, splits):
+    """E8M0 tables at the edges of the 16- to 64-row tiles, even and odd steps per K group, one to 17 of them,
+    and K split: the scales up to byte 252, one zero-filled group with byte 0."""
+    from bybylang_amd import synth
+    g = synth.rng(M + K + N)
+    if splits:
+        monkeypatch.setenv("BYHIP_Q4_SPLIT", str(splits))
+    x = synth.activations(g, M, K, np.float32)
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    sb = g.integers(120, 134, size=(N, K // 32))
+    codes[N // 2, 32:64] = 0
+    sb[N // 2, 1] = 0
+    x[:, :4] *= np.float32(2.0 ** -8)  # no sum of the last column's passes 2^128 in any order
+    codes[N - 1, :] = 0     # a column whose only weights are at the ends of the scales
+    codes[N - 1, :4] = [1, 7, 9, 15]
+    sb[N - 1, 0] = 252 if M % 2 else 1
+    check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())

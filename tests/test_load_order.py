@@ -23,6 +23,7 @@ KERNELS = {
     "gemm_planes_half": ("byhip_planes.hip.o", lambda t: (4 * t[0] * t[1] + 16) // (t[0] * t[2])),
     "mxfp4_gemm_mid": ("byhip_mxfp4.hip.o", lambda t: 4),
     "gemm_f32_q4": ("byhip_exact.hip.o", lambda t: t[0]),
+    "gemm_fp4_mx": ("byhip_fp4mx.hip.o", lambda t: 2 * t[0]),
 }
 
 
