@@ -186,7 +186,8 @@ void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 
 // fp32 activations as two fp16 planes (byhip_planes.hip) against FP4-KM weights with an E2M1 table whose
 // products are all halves, half weights, or the prefill copy of Q4 weights: whether the kernel takes the
-// call (K % 128 == 0 for FP4-KM, else K % 64 == 0, 16-byte aligned operands, offsets below 2^31), and the launch.
+// call (K % 128 == 0 for FP4-KM, else K % 64 == 0, 16-byte aligned operands, offsets below 2^31, room for a
+// row's planes in half the scratch), and the launch.
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
 

@@ -738,12 +738,18 @@ void launch_planes_rows(const GemmArgs& a0) {
     if (a.part) launch_splitk_sum(a, splits);
 }
 
+// Rows whose planes fit half the scratch (the rest holds split-K partials) and whose offsets stay below 2^31.
+size_t plane_rows(const GemmArgs& a) {
+    const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
+    return std::min<size_t>({work_bytes / 2 / ((size_t)a.K * 4 + sizeof(int)), ((size_t)kPast / 2) / ((size_t)a.K * 2), 65535 * 16});
+}
+
 }  // namespace
 
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a) {
     constexpr uint64_t kLim = kPast;  // offsets stay below 2^31 (loads past the end)
     if (a.x_dtype != BYHIP_F32 || reinterpret_cast<uintptr_t>(a.x) % 16 != 0) return false;
-    if ((uint64_t)(a.K) * 2 * 128 >= kLim) return false;
+    if ((uint64_t)(a.K) * 2 * 128 >= kLim || plane_rows(a) == 0) return false;
     if (fmt == BFormat::Fp4Km)
         return a.K % 128 == 0 && reinterpret_cast<uintptr_t>(a.blob) % 16 == 0 && a.scale_base % 4 == 0 &&
                (uint64_t)(a.N + kBN) * (a.K / 2) < kLim;
@@ -758,13 +764,8 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
     uint8_t* const work = static_cast<uint8_t*>(a0.work ? a0.work : workspace());
     const size_t work_bytes = a0.work ? a0.work_bytes : kWorkspaceBytes;
     const size_t es = dtype_bytes(a0.y_dtype);
-    // Row blocks whose planes fit half the scratch (the rest holds split-K partials) and whose
-    // offsets stay below 2^31.
-    const size_t row_planes = (size_t)a0.K * 4;
-    size_t rows = std::min<size_t>(work_bytes / 2 / (row_planes + sizeof(int)), ((size_t)kPast / 2) / ((size_t)a0.K * 2));
-    rows = std::min<size_t>(rows, 65535 * 16);
+    size_t rows = plane_rows(a0);
     if (rows > 64) rows = rows / 64 * 64;
-    if (rows == 0) fail("byhip: K=%d rows of fp32 activations exceed the scratch", a0.K);
     for (size_t m = 0; m < (size_t)a0.M; m += rows) {
         GemmArgs a = a0;
         a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);

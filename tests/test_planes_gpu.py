@@ -190,3 +190,29 @@ def test_q4_planes(hip, oracle, monkeypatch, M, K, N, group, zeros, splits):
         ref_check(outs[hip.F32][m] / scale, want[m] / scale)
     from parity import f32_to_bf16_rne
     assert np.array_equal(outs[hip.BF16], (f32_to_bf16_rne(outs[hip.F32]).view(np.uint32) >> 16).astype(np.uint16))
+
+
+@pytest.mark.parametrize("fmt", ["f16", "fp4km"])
+@pytest.mark.parametrize("K", [4194304 - 128, 4194304])
+def test_rows_longer_than_the_scratch(hip, fmt, K):
+    """Rows whose planes do not fit the scratch (from K = 4,194,304 on) run on the other kernels. Whole numbers
+    few enough for exact sums."""
+    from bybylang_amd import synth
+    M, N = 2, 3
+    g = synth.rng(K)
+    x = np.zeros((M, K), np.float32)
+    x[:, :: K // 512] = g.integers(-8, 9, size=x[:, :: K // 512].shape)
+    x[:, K - 1] = 5
+    y = hip.DeviceBuffer(M * N * 4)
+    if fmt == "f16":
+        w = g.integers(-4, 5, size=(N, K)).astype(np.float16)
+        hip.f16_tile_gemm(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.DeviceBuffer.from_array(w.reshape(-1)), y, hip.F32, M, K, N)
+    else:
+        codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+        t = np.concatenate([synth.E2M1, np.full(256, 2.0)]).astype(np.float32)
+        w = 2 * np.asarray(synth.E2M1)[codes]
+        blob = np.concatenate([synth.fp4km_pack(codes).reshape(-1), np.zeros(N * (K // 32), np.uint8)])
+        hip.fp4km_tile_gemm(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.DeviceBuffer.from_array(blob), N * (K // 2),
+                            hip.DeviceBuffer.from_array(t), 0, y, hip.F32, M, K, N)
+    k = np.nonzero(x.any(axis=0))[0]
+    assert np.array_equal(y.read(np.float32).reshape(M, N), x[:, k].astype(np.float64) @ w[:, k].astype(np.float64).T)
