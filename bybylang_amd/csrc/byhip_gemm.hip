@@ -1907,7 +1907,6 @@ void launch_gemm(BFormat fmt, const GemmArgs& a) {
     if (a.M > 65535 * BM) fail("byhip: M=%d too large for one launch", a.M);
     switch (fmt) {
     case BFormat::Q4Fast:
-        // fp32 activations: the wide tile on two fp16 planes where the scratch holds them
         // fp32 activations: the two-plane kernel (two MFMAs per product) when its 64 x 128 tiles fill half
         // the CUs, else the 16- or 32-row wide tile (three, but twice the blocks) where the scratch holds
         // its planes. us, wide / planes: K = N = 4096, M = 64 18.3 / 22.7, 128 24.3 / 25.0, 256 32.2 / 32.2,

@@ -658,18 +658,28 @@ int planes_fm(int M) {
     return (M + 16 * row_tiles - 1) / (16 * row_tiles);
 }
 
+long planes_tiles(int M, int N) {
+    const int rows = 16 * planes_fm(M);
+    return (long)((N + kBN - 1) / kBN) * ((M + rows - 1) / rows);
+}
+
+// A number of K splits and the time a pass is expected to take, in steps.
+struct Pass {
+    int splits;
+    double time;
+};
+
 // K splits, in 128-value steps: the count that minimises rounds of blocks x (steps per split + 12)
 // (12 for a block's fixed cost: first loads, epilogue), plus 6 steps for the sum's launch.
-int planes_splits(const GemmArgs& a, long tiles) {
-    const int steps = (a.K + 127) / 128;
+Pass planes_pass(int K, long tiles) {
+    const int steps = (K + 127) / 128;
     const long cus = compute_units();
-    int best = 1;
-    double best_t = 1e300;
+    Pass best = {1, 1e300};
     for (int s = 1; s <= std::max(1, steps / 4); ++s) {
         const int per = (steps + s - 1) / s;
         if ((steps + per - 1) / per != s) continue;  // the same split as a smaller s
         const double t = (double)((tiles * s + cus - 1) / cus) * (per + 12) + (s > 1 ? 6.0 : 0.0);
-        if (t < 0.97 * best_t) best = s, best_t = t;
+        if (t < 0.97 * best.time) best = {s, t};
     }
     return best;
 }
@@ -677,15 +687,14 @@ int planes_splits(const GemmArgs& a, long tiles) {
 // The same for gemm_planes_half, in 64-value steps: 16 for a block's fixed cost, 12 for the sum's launch and
 // 1.5 per split for what it reads (M = 32, K = 4096, N = 6144: 4 splits 16.3 us, 6 splits,
 // a second block on some of the CUs, 17.9, 1 split 24.5).
-int half_splits(long tiles, int steps) {
+Pass half_pass(long tiles, int steps) {
     const long cus = compute_units();
-    int best = 1;
-    double best_t = 1e300;
+    Pass best = {1, 1e300};
     for (int s = 1; s <= std::max(1, steps / 8); ++s) {
         const int per = (steps + s - 1) / s;
         if ((steps + per - 1) / per != s) continue;
         const double t = (double)((tiles * s + cus - 1) / cus) * (per + 16) + (s > 1 ? 12.0 + 1.5 * s : 0.0);
-        if (t < 0.97 * best_t) best = s, best_t = t;
+        if (t < 0.97 * best.time) best = {s, t};
     }
     return best;
 }
@@ -705,18 +714,26 @@ void launch_half_y(const GemmArgs& a, int splits) {
 // Rows per tile: 32, two blocks per CU, for up to 32 rows (M = 8, K = N = 4096: 12.6 us, 64 rows
 // 13.1); else 64, or 128 where its rounds of blocks, each 1.6 times as long, take less time (M = 256, K =
 // 4096, N = 14336: one round for two, 66 us for 86; M = 512, K = N = 4096: one round either way, 45 for 39).
+struct HalfTiles {
+    int rows;
+    long tiles;
+};
+HalfTiles half_tiles(int M, int K, int N) {
+    const int cus = compute_units();
+    const long cols = (N + kBN - 1) / kBN, t64 = cols * ((M + 63) / 64), t128 = cols * ((M + 127) / 128);
+    if (M <= 32) return {32, cols};
+    if ((uint64_t)K * 256 < kPast / 2 && 8 * ((t128 + cus - 1) / cus) < 5 * ((t64 + cus - 1) / cus)) return {128, t128};
+    return {64, t64};
+}
+
 void launch_half_rows(const GemmArgs& a0) {
     GemmArgs a = a0;
-    const int cus = compute_units();
-    const long cols = (a.N + kBN - 1) / kBN, t64 = cols * ((a.M + 63) / 64), t128 = cols * ((a.M + 127) / 128);
-    const bool tall = (uint64_t)a.K * 256 < kPast / 2 && 8 * ((t128 + cus - 1) / cus) < 5 * ((t64 + cus - 1) / cus);
-    const long tiles = a.M <= 32 ? cols : tall ? t128 : t64;
-    const int steps = a.K / kSub;
-    const int forced = env_int("BYHIP_Q4_SPLIT", 0);
-    const int splits = choose_split(a, tiles, steps, 1, forced > 0 ? forced : half_splits(tiles, steps), 1);
+    const HalfTiles h = half_tiles(a.M, a.K, a.N);
+    const int steps = a.K / kSub, forced = env_int("BYHIP_Q4_SPLIT", 0);
+    const int splits = choose_split(a, h.tiles, steps, 1, forced > 0 ? forced : half_pass(h.tiles, steps).splits, 1);
     if (splits == 1) a.part = nullptr;
-    if (a.M <= 32) launch_half_y<2, 1, 4>(a, splits);
-    else if (tall) launch_half_y<4, 2, 2>(a, splits);
+    if (h.rows == 32) launch_half_y<2, 1, 4>(a, splits);
+    else if (h.rows == 128) launch_half_y<4, 2, 2>(a, splits);
     else launch_half_y<2, 2, 4>(a, splits);
     if (a.part) launch_splitk_sum(a, splits);
 }
@@ -725,9 +742,9 @@ template <BFormat F>
 void launch_planes_rows(const GemmArgs& a0) {
     GemmArgs a = a0;
     const int fm = planes_fm(a.M);
-    const long tiles = (long)((a.N + kBN - 1) / kBN) * ((a.M + 16 * fm - 1) / (16 * fm));
+    const long tiles = planes_tiles(a.M, a.N);
     const int forced = env_int("BYHIP_Q4_SPLIT", 0);
-    const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : planes_splits(a, tiles), 1);
+    const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : planes_pass(a.K, tiles).splits, 1);
     if (splits == 1) a.part = nullptr;
     if constexpr (F == BFormat::Q4Fast) {
         if (a.zeros) launch_planes_fm<F, true>(a, fm, splits);
@@ -742,6 +759,24 @@ void launch_planes_rows(const GemmArgs& a0) {
 size_t plane_rows(const GemmArgs& a) {
     const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
     return std::min<size_t>({work_bytes / 2 / ((size_t)a.K * 4 + sizeof(int)), ((size_t)kPast / 2) / ((size_t)a.K * 2), 65535 * 16});
+}
+
+// Rows of a pass over the weights: all of them where they fit (K = N = 4096, M = 970 in one pass 87 us,
+// 960 + 10 94), else as many whole 64-row tiles as fit or even shares of those, whichever passes' rounds of
+// blocks take less time (us, K = N = 4096, M = 1024: 960 + 64 rows 105, 2 x 512 94; M = 2048: 2 x 960 + 128 191, 3 x 704
+// 227; K = 14336, N = 4096, M = 300: 256 + 44 103, 192 + 108 113).
+int planes_pass_rows(BFormat fmt, const GemmArgs& a) {
+    const int most = (int)std::min<size_t>(plane_rows(a), (size_t)a.M);
+    if (most == a.M || most < 64) return most;
+    auto time_of = [&](int rows) {
+        if (rows == 0) return 0.0;
+        if (fmt != BFormat::F16) return planes_pass(a.K, planes_tiles(rows, a.N)).time;
+        const HalfTiles h = half_tiles(rows, a.K, a.N);
+        return half_pass(h.tiles, a.K / kSub).time * (h.rows == 128 ? 1.6 : 1.0);
+    };
+    auto total = [&](int rows) { return (double)(a.M / rows) * time_of(rows) + time_of(a.M % rows); };
+    const int full = most / 64 * 64, blocks = (a.M + full - 1) / full, even = (a.M + 64 * blocks - 1) / (64 * blocks) * 64;
+    return total(even) < 0.97 * total(full) ? even : full;
 }
 
 }  // namespace
@@ -764,8 +799,7 @@ void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
     uint8_t* const work = static_cast<uint8_t*>(a0.work ? a0.work : workspace());
     const size_t work_bytes = a0.work ? a0.work_bytes : kWorkspaceBytes;
     const size_t es = dtype_bytes(a0.y_dtype);
-    size_t rows = plane_rows(a0);
-    if (rows > 64) rows = rows / 64 * 64;
+    const size_t rows = (size_t)planes_pass_rows(fmt, a0);
     for (size_t m = 0; m < (size_t)a0.M; m += rows) {
         GemmArgs a = a0;
         a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);

@@ -216,3 +216,27 @@ def test_rows_longer_than_the_scratch(hip, fmt, K):
                             hip.DeviceBuffer.from_array(t), 0, y, hip.F32, M, K, N)
     k = np.nonzero(x.any(axis=0))[0]
     assert np.array_equal(y.read(np.float32).reshape(M, N), x[:, k].astype(np.float64) @ w[:, k].astype(np.float64).T)
+
+
+@pytest.mark.parametrize("fmt", ["f16", "q4"])
+@pytest.mark.parametrize("M", [257, 292, 293, 600])
+def test_rows_about_what_the_scratch_holds(hip, oracle, monkeypatch, fmt, M):
+    """K = 14336, where half the scratch holds the planes of 292 rows: all of them in one pass, also where
+    that is no whole number of 64-row tiles, or in blocks."""
+    from bybylang_amd import synth
+    K, N = 14336, 24
+    g = synth.rng(M)
+    x = synth.activations(g, M, K, np.float32)
+    y = hip.DeviceBuffer(M * N * 4)
+    xd = hip.DeviceBuffer.from_array(x.reshape(-1))
+    rows = sorted({0, 63, 64, 127, 128, 191, 192, 255, 256, M // 2, M - 65, M - 1})
+    if fmt == "f16":
+        w = (g.standard_normal((N, K)) * 0.05).astype(np.float16)
+        hip.f16_tile_gemm(xd, hip.F32, hip.DeviceBuffer.from_array(w.reshape(-1)), y, hip.F32, M, K, N)
+        want = oracle.tile_gemm(1, len(rows), K, N, 0, 0, w.view(np.uint8).reshape(-1), None, x[rows])
+    else:
+        wq, sc, ze, _ = synth.q4_weights(g, N, K, 32)
+        monkeypatch.setenv("BYHIP_Q4_PLANES", "1")
+        hip.q4_matmul(xd, hip.F32, hip.Q4Weights(wq, sc, ze, K, N, 32, K // 32), y, hip.F32, M)
+        want = oracle.matmul_q4(x[rows].reshape(-1), wq, sc, ze, len(rows), K, N, 32, K // 32)
+    ref_check(y.read(np.float32).reshape(M, N)[rows], np.asarray(want).reshape(len(rows), N))
