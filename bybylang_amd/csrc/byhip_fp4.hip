@@ -4,8 +4,8 @@
 // FP4-KM (cpu_vm.c:583-628): weight = lut[nibble] * lut[16 + scale byte] with the 272-float decode
 // table; nibble bytes [N, K/2] (byte j of a group: element j low, j + 16 high), scale bytes
 // [N, K/32] at scale_base. One row of fp32 activations takes the decode GEMV (byhip_fp4gemv.hip), more
-// on E2M1 / E8M0 tables or E2M1 values whose products are halves gemm_planes (byhip_planes.hip); other
-// tables whose products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
+// on E2M1 / E8M0 tables gemm_fp4_mx (byhip_fp4mx.hip), on E2M1 values whose products are halves
+// gemm_planes (byhip_planes.hip); other tables whose products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
 // the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
 // exactly E2M1 and 2^(e-127).
 #include <algorithm>
@@ -80,40 +80,13 @@ bool table_products_are_halves(const float* t) {
     return ok;
 }
 
-// The class of a decode table, which the route of fp32 activations goes by:
-//   kTableMx      E2M1's 16 values bit for bit and the scales 2^(b - 127) up to byte 252 (a larger one's
-//                 products may overflow; the kernel looks out for those bytes)
-//   kTableE2m1    E2M1's values, and every product a half
-//   kTableHalves  every product a half
-//   kTableAny     any other
-enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2, kTableMx = 3 };
-
+// The class of a decode table from its host copy.
 int table_class(const float* t) {
     const bool e2m1 = memcmp(t, kE2M1, sizeof kE2M1) == 0;
     bool mx = e2m1;
     for (int b = 0; b < 253 && mx; ++b) mx = t[16 + b] == std::ldexp(1.0f, b - 127);
     if (mx) return kTableMx;
     return !table_products_are_halves(t) ? kTableAny : e2m1 ? kTableE2m1 : kTableHalves;
-}
-
-// The same on the device, for the routes that are queued: `mx` and `e2m1` say whether those classes'
-// kernels are, otherwise such tables count as the next class. Thread b checks scale entry b.
-__global__ __launch_bounds__(256) void fp4km_classify(const float* __restrict__ t, int mx, int e2m1, int* flag) {
-    constexpr uint32_t bits[16] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u,
-                                   0x40C00000u, 0x80000000u, 0xBF000000u, 0xBF800000u, 0xBFC00000u, 0xC0000000u,
-                                   0xC0400000u, 0xC0800000u, 0xC0C00000u};
-    const uint32_t b = threadIdx.x;
-    const float s = t[16 + b];
-    bool halves = true, same = true;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float p = t[i] * s;
-        halves = halves && __builtin_isfinite(p) && (float)(_Float16)p == p;
-        same = same && __builtin_bit_cast(uint32_t, t[i]) == bits[i];
-    }
-    halves = __syncthreads_and(halves);
-    const bool e8m0 = __syncthreads_and(b >= 253u || __builtin_bit_cast(uint32_t, s) == (b ? b << 23 : 0x00400000u));
-    if (b == 0) *flag = same && e8m0 && mx ? kTableMx : !halves ? kTableAny : same && e2m1 ? kTableE2m1 : kTableHalves;
 }
 
 void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_bytes, size_t scale_base,
@@ -177,10 +150,13 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
             }
         } else {
             int* flag = device_flags();
-            launch("fp4km_classify", fp4km_classify, dim3(1), dim3(256), 0, static_cast<const float*>(lut + lut_base),
-                   (int)mx, (int)e2m1, flag);
+            RouteSums sums;
             GemmArgs g = a;
             g.gate = flag;
+            if (launch_fp4km_prepare(a, mx, e2m1, flag)) {  // a single pass on each route
+                g.prepared = true;
+                g.sums = &sums;
+            }
             if (mx) {
                 g.gate_want = kTableMx;
                 launch_fp4_mx(g);
@@ -193,6 +169,7 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
             launch_gemm(BFormat::Fp4Km, g);
             g.gate_want = kTableAny;
             launch_gemm_exact(BFormat::Fp4Km, g);
+            launch_route_sums(g, sums);
             return;
         }
     }

@@ -60,11 +60,29 @@ struct GemmArgs {
     // The wide tile on fp32 activations: x holds the high fp16 plane of the shifted activations and
     // x_lo the low one (x * 2^t = hi + lo, t per row in row_shift).
     const void* x_lo = nullptr;
-    // A device-side route choice: when gate is set, the general fp16 MFMA GEMM, the exact GEMM and
-    // their split-K sum do nothing unless *gate == gate_want (the flag a classification kernel
-    // earlier on the stream wrote), so two routes can be queued and only the chosen one runs.
+    // A device-side route choice: when gate is set, the FP4-KM kernels above one row and their split-K sums
+    // do nothing unless *gate == gate_want (the class of the decode table, which fp4km_prepare wrote earlier
+    // on the stream), so every route can be queued and only the chosen one runs.
     const int* gate = nullptr;
     int gate_want = 0;
+    // Queued routes only: fp4km_prepare has left the row shifts and planes in the scratch; the routes' split-K
+    // sums are collected here (on the host) for one launch behind them all.
+    bool prepared = false;
+    struct RouteSums* sums = nullptr;
+};
+
+// The class of a decode table, which the route of fp32 activations goes by:
+//   kTableMx      E2M1's 16 values bit for bit and the scales 2^(b - 127) up to byte 252 (a larger one's
+//                 products may overflow; the kernel looks out for those bytes)
+//   kTableE2m1    E2M1's values, and every product a half
+//   kTableHalves  every product a half
+//   kTableAny     any other
+enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2, kTableMx = 3, kTableClasses = 4 };
+
+// The split-K sum of each class's route: none where splits is 0. Without a gate entry 0 counts.
+struct RouteSums {
+    const float* part[kTableClasses] = {};
+    int splits[kTableClasses] = {};
 };
 
 // Whether 8-output chunks may leave as 16-byte stores: every row of y (or of the split-K
@@ -138,6 +156,7 @@ __host__ __device__ __forceinline__ size_t splitk_stride(int M, int N) { return 
 int choose_split(GemmArgs& a, long tiles, int nsteps, int min_steps, int forced, int per_cu = 2);
 // y = the sum of the split-K partials in slice order.
 void launch_splitk_sum(const GemmArgs& a, int splits);
+void launch_route_sums(const GemmArgs& a, const RouteSums& s);
 
 // Queues the GEMM on the library stream; K % 32 == 0 is required (callers check). fp16 MFMA: the
 // weights are rounded once to fp16 (exact for F16 weights and for FP4-KM tables whose products
@@ -190,6 +209,11 @@ void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 // row's planes in half the scratch), and the launch.
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
+
+// Classifies the decode table on the device into *flag (`mx`, `e2m1`: whether those classes' kernels take the
+// call; otherwise such tables count as the next class) and prepares fp32 activations for it. False when
+// their planes do not fit the scratch at once: then it has only classified.
+bool launch_fp4km_prepare(const GemmArgs& a, bool mx, bool e2m1, int* flag);
 
 // fp32 activations as three bf16 terms (byhip_fp4mx.hip) against FP4-KM weights with E2M1's values and the
 // scales 2^(b - 127); entries 253 to 255 may hold anything. K % 128 == 0, 16-byte aligned operands,

@@ -305,7 +305,9 @@ __global__ __launch_bounds__(256) void gemm_f16_mfma(GemmArgs a) {
 // Per-row shift t of fp32 activations: the row's largest magnitude brought into [2^14, 2^15) (one
 // block per row), so the fp16 hi + lo split of x * 2^t neither overflows nor loses the row's large
 // values to fp16 subnormals.
-__global__ __launch_bounds__(256) void row_range_shift(const float* __restrict__ x, int K, int* __restrict__ out) {
+__global__ __launch_bounds__(256) void row_range_shift(const float* __restrict__ x, int K, int* __restrict__ out,
+                                                      const int* gate, int gate_want) {
+    if (gate && *gate != gate_want) return;  // another route was chosen (whole grid)
     __shared__ float part[4];
     const float* r = x + (size_t)blockIdx.x * K;
     float mx = 0.0f;
@@ -559,14 +561,27 @@ __global__ __launch_bounds__(256) void q4_gemm_pipe(GemmArgs a) {
         }
 }
 
+// The partials and splits of the route that ran (splits 0: it wrote y itself).
+__device__ __forceinline__ int pick_route(const RouteSums& s, const int* gate, const float*& part) {
+    int splits = s.splits[0];
+    part = s.part[0];
+    if (gate) {
+        const int c = *gate;
+#pragma unroll
+        for (int i = 1; i < kTableClasses; ++i)
+            if (c == i) splits = s.splits[i], part = s.part[i];
+    }
+    return splits;
+}
+
 // y = sum over z of part[z] (z in order, so the result does not depend on block timing), four
-// consecutive outputs per thread; nothing when `gate` is set and *gate != want (GemmArgs::gate).
-// The same sum, one output per thread: four times the blocks, for outputs too few to fill the CUs
-// four to a thread.
+// consecutive outputs per thread (splitk_sum), or one: four times the blocks, for outputs too few to fill
+// the CUs four to a thread. With a gate, of the route it names.
 template <int YT>
-__global__ __launch_bounds__(256) void splitk_sum1(const float* __restrict__ part, int splits, int M, int N,
-                                                   void* y, const int* gate, int want) {
-    if (gate && *gate != want) return;
+__global__ __launch_bounds__(256) void splitk_sum1(RouteSums s, int M, int N, void* y, const int* gate) {
+    const float* part;
+    const int splits = pick_route(s, gate, part);
+    if (splits == 0) return;
     const size_t mn = (size_t)M * N, stride = splitk_stride(M, N);
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
@@ -584,9 +599,10 @@ __global__ __launch_bounds__(256) void splitk_sum1(const float* __restrict__ par
 }
 
 template <int YT>
-__global__ __launch_bounds__(256) void splitk_sum(const float* __restrict__ part, int splits, int M, int N,
-                                                  void* y, const int* gate, int want) {
-    if (gate && *gate != want) return;
+__global__ __launch_bounds__(256) void splitk_sum(RouteSums s, int M, int N, void* y, const int* gate) {
+    const float* part;
+    const int splits = pick_route(s, gate, part);
+    if (splits == 0) return;
     const size_t mn = (size_t)M * N, stride = splitk_stride(M, N);
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= mn) return;
@@ -1537,22 +1553,31 @@ int choose_split(GemmArgs& a, long tiles, int nsteps, int min_steps, int forced,
 }
 
 void launch_splitk_sum(const GemmArgs& a, int splits) {
+    RouteSums s, &to = a.sums ? *a.sums : s;
+    const int c = a.gate ? a.gate_want : 0;
+    to.part[c] = a.part;
+    to.splits[c] = splits;
+    if (!a.sums) launch_route_sums(a, s);
+}
+
+void launch_route_sums(const GemmArgs& a, const RouteSums& s) {
+    if (std::all_of(s.splits, s.splits + kTableClasses, [](int n) { return n == 0; })) return;
     const size_t quads = ((size_t)a.M * a.N + 3) / 4;
     const dim3 grid((unsigned)((quads + 255) / 256));
     if (grid.x < (unsigned)compute_units()) {  // fp32 route M = 9 .. 32: 0.2-0.4 us faster
         const dim3 g1((unsigned)(((size_t)a.M * a.N + 255) / 256));
         switch (a.y_dtype) {
-        case BYHIP_F32: launch("splitk_sum1", splitk_sum1<BYHIP_F32>, g1, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
-        case BYHIP_F16: launch("splitk_sum1", splitk_sum1<BYHIP_F16>, g1, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
-        default: launch("splitk_sum1", splitk_sum1<BYHIP_BF16>, g1, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
+        case BYHIP_F32: launch("splitk_sum1", splitk_sum1<BYHIP_F32>, g1, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
+        case BYHIP_F16: launch("splitk_sum1", splitk_sum1<BYHIP_F16>, g1, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
+        default: launch("splitk_sum1", splitk_sum1<BYHIP_BF16>, g1, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
         }
         BYHIP_LAUNCHED("splitk_sum1");
         return;
     }
     switch (a.y_dtype) {
-    case BYHIP_F32: launch("splitk_sum", splitk_sum<BYHIP_F32>, grid, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
-    case BYHIP_F16: launch("splitk_sum", splitk_sum<BYHIP_F16>, grid, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
-    default: launch("splitk_sum", splitk_sum<BYHIP_BF16>, grid, dim3(256), 0, a.part, splits, a.M, a.N, a.y, a.gate, a.gate_want); break;
+    case BYHIP_F32: launch("splitk_sum", splitk_sum<BYHIP_F32>, grid, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
+    case BYHIP_F16: launch("splitk_sum", splitk_sum<BYHIP_F16>, grid, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
+    default: launch("splitk_sum", splitk_sum<BYHIP_BF16>, grid, dim3(256), 0, s, a.M, a.N, a.y, a.gate); break;
     }
     BYHIP_LAUNCHED("splitk_sum");
 }
@@ -1825,9 +1850,11 @@ void launch_f(const GemmArgs& a0) {
     const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
     if ((size_t)a.M * sizeof(int) > work_bytes) fail("byhip: M=%d rows of fp32 activations exceed the scratch", a.M);
     int* shifts = static_cast<int*>(work);
-    launch("row_range_shift", row_range_shift, dim3((unsigned)a.M), dim3(256), 0, static_cast<const float*>(a.x), a.K,
-                       shifts);
-    BYHIP_LAUNCHED("row_range_shift");
+    if (!a.prepared) {
+        launch("row_range_shift", row_range_shift, dim3((unsigned)a.M), dim3(256), 0, static_cast<const float*>(a.x), a.K,
+               shifts, a.gate, a.gate_want);
+        BYHIP_LAUNCHED("row_range_shift");
+    }
     a.row_shift = shifts;
     // the split-K partial sums, if any, go after the shifts
     const size_t used = ((size_t)a.M * sizeof(int) + 255) / 256 * 256;

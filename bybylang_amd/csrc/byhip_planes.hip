@@ -565,8 +565,8 @@ __global__ __launch_bounds__(64 * RP * CP, RP * FR == 2 ? 4 : 2) void gemm_plane
 // first kHeld chunks of a thread stay in registers between the maximum and the split.
 constexpr int kHeld = 4;
 template <bool FP4>
-__global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x, int K, int* __restrict__ shifts,
-                                                   uint4* __restrict__ hi, uint4* __restrict__ lo) {
+__device__ __forceinline__ void split_row(const float* __restrict__ x, int K, bool planes, int* __restrict__ shifts,
+                                          uint4* __restrict__ hi, uint4* __restrict__ lo) {
     __shared__ float part[4];
     const size_t row = (size_t)blockIdx.x * K;
     const float4* r = reinterpret_cast<const float4*>(x + row);
@@ -599,6 +599,7 @@ __global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x,
     __syncthreads();
     const int t = fp16_range_shift(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
     if (threadIdx.x == 0) shifts[blockIdx.x] = t;
+    if (!planes) return;
     auto split = [&](int i, const float4& va, const float4& vb) {
         const float s[8] = {va.x, FP4 ? vb.x : va.y, FP4 ? va.y : va.z, FP4 ? vb.y : va.w,
                             FP4 ? va.z : vb.x, FP4 ? vb.z : vb.y, FP4 ? va.w : vb.z, vb.w};
@@ -627,6 +628,41 @@ __global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x,
         if (i < nc) split(i, ha[u], hb[u]);
     }
     for (int i = (int)threadIdx.x + 256 * kHeld; i < nc; i += 256) split(i, r[first(i)], r[first(i) + second]);
+}
+
+template <bool FP4>
+__global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x, int K, int* __restrict__ shifts,
+                                                   uint4* __restrict__ hi, uint4* __restrict__ lo, const int* gate, int gate_want) {
+    if (gate && *gate != gate_want) return;  // another route was chosen (whole grid)
+    split_row<FP4>(x, K, true, shifts, hi, lo);
+}
+
+// Calls whose route the device chooses (recorded ones, tables without a host copy): each block classifies the
+// decode table (thread b: scale entry b), the first one writes the class to *flag, and each then brings its
+// row of x (null: none) into the form that the class's kernel takes: planes, or the shift alone. One launch
+// for the three that would take, as the routes' split-K sums share one (launch_route_sums): a launch that
+// does nothing still costs 1.5 to 2 us. Recorded, us, each of ten launches by itself / these six: K = N = 4096,
+// M = 16 E8M0 26.5 / 19.2, E2M1 on halves 26.9 / 19.5, other halves 39.4 / 30.9, any values 32.5 / 25.3; K = 4096,
+// N = 6144, M = 47 39.6 / 32.5, 34.0 / 26.6, 52.0 / 43.1, 78.4 / 71.1.
+__global__ __launch_bounds__(256) void fp4km_prepare(const float* __restrict__ t, int mx, int e2m1, int* flag, const float* __restrict__ x,
+                                                     int K, int* __restrict__ shifts, uint4* __restrict__ hi, uint4* __restrict__ lo) {
+    constexpr uint32_t bits[16] = {0u, 0x3F000000u, 0x3F800000u, 0x3FC00000u, 0x40000000u, 0x40400000u, 0x40800000u,
+                                   0x40C00000u, 0x80000000u, 0xBF000000u, 0xBF800000u, 0xBFC00000u, 0xC0000000u,
+                                   0xC0400000u, 0xC0800000u, 0xC0C00000u};
+    const uint32_t b = threadIdx.x;
+    const float s = t[16 + b];
+    bool halves = true, same = true;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float p = t[i] * s;
+        halves = halves && __builtin_isfinite(p) && (float)(_Float16)p == p;
+        same = same && __builtin_bit_cast(uint32_t, t[i]) == bits[i];
+    }
+    halves = __syncthreads_and(halves);
+    const bool e8m0 = __syncthreads_and(b >= 253u || __builtin_bit_cast(uint32_t, s) == (b ? b << 23 : 0x00400000u));
+    const int cls = same && e8m0 && mx ? kTableMx : !halves ? kTableAny : same && e2m1 ? kTableE2m1 : kTableHalves;
+    if (b == 0 && blockIdx.x == 0) *flag = cls;
+    if (x && (cls == kTableE2m1 || cls == kTableHalves)) split_row<true>(x, K, cls == kTableE2m1, shifts, hi, lo);
 }
 
 template <BFormat F, int FM, bool ZG>
@@ -795,33 +831,53 @@ bool gemm_planes_ok(BFormat fmt, const GemmArgs& a) {
     return false;
 }
 
+namespace {
+
+// Where the row shifts and planes of M rows go, and what of the scratch is left.
+struct PlaneScratch {
+    int* shifts;
+    uint8_t *hi, *lo, *rest;
+    size_t rest_bytes;
+};
+
+PlaneScratch plane_scratch(const GemmArgs& a) {
+    uint8_t* const work = static_cast<uint8_t*>(a.work ? a.work : workspace());
+    const size_t bytes = a.work ? a.work_bytes : kWorkspaceBytes;
+    const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256, plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
+    return {reinterpret_cast<int*>(work), work + shift_bytes, work + shift_bytes + plane, work + shift_bytes + 2 * plane,
+            bytes - shift_bytes - 2 * plane};
+}
+
+}  // namespace
+
+bool launch_fp4km_prepare(const GemmArgs& a, bool mx, bool e2m1, int* flag) {
+    const bool f32 = a.x_dtype == BYHIP_F32, fits = !f32 || (size_t)a.M <= plane_rows(a);
+    PlaneScratch p = {};
+    if (f32 && fits) p = plane_scratch(a);
+    launch("fp4km_prepare", fp4km_prepare, dim3(f32 && fits ? (unsigned)a.M : 1u), dim3(256), 0, a.lut, (int)mx, (int)e2m1, flag,
+           f32 && fits ? static_cast<const float*>(a.x) : nullptr, a.K, p.shifts, reinterpret_cast<uint4*>(p.hi), reinterpret_cast<uint4*>(p.lo));
+    BYHIP_LAUNCHED("fp4km_prepare");
+    return fits;
+}
+
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
-    uint8_t* const work = static_cast<uint8_t*>(a0.work ? a0.work : workspace());
-    const size_t work_bytes = a0.work ? a0.work_bytes : kWorkspaceBytes;
-    const size_t es = dtype_bytes(a0.y_dtype);
     const size_t rows = (size_t)planes_pass_rows(fmt, a0);
     for (size_t m = 0; m < (size_t)a0.M; m += rows) {
         GemmArgs a = a0;
         a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);
         const float* const x = static_cast<const float*>(a0.x) + m * a0.K;
-        a.y = static_cast<uint8_t*>(a0.y) + m * a0.N * es;
-        const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256;
-        const size_t plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
-        int* const shifts = reinterpret_cast<int*>(work);
-        uint8_t* const hi = work + shift_bytes;
-        uint8_t* const lo = hi + plane;
-        if (fmt == BFormat::Fp4Km)
-            launch("split_planes", split_planes<true>, dim3((unsigned)a.M), dim3(256), 0,
-                   x, a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
-        else
-            launch("split_planes", split_planes<false>, dim3((unsigned)a.M), dim3(256), 0,
-                   x, a.K, shifts, reinterpret_cast<uint4*>(hi), reinterpret_cast<uint4*>(lo));
-        BYHIP_LAUNCHED("split_planes");
-        a.x = hi;
-        a.x_lo = lo;
-        a.row_shift = shifts;
-        a.work = lo + plane;
-        a.work_bytes = work_bytes - shift_bytes - 2 * plane;
+        a.y = static_cast<uint8_t*>(a0.y) + m * a0.N * dtype_bytes(a0.y_dtype);
+        const PlaneScratch p = plane_scratch(a);
+        if (!a.prepared) {
+            launch("split_planes", fmt == BFormat::Fp4Km ? split_planes<true> : split_planes<false>, dim3((unsigned)a.M), dim3(256), 0, x, a.K,
+                   p.shifts, reinterpret_cast<uint4*>(p.hi), reinterpret_cast<uint4*>(p.lo), a.gate, a.gate_want);
+            BYHIP_LAUNCHED("split_planes");
+        }
+        a.x = p.hi;
+        a.x_lo = p.lo;
+        a.row_shift = p.shifts;
+        a.work = p.rest;
+        a.work_bytes = p.rest_bytes;
         if (fmt == BFormat::Fp4Km) launch_planes_rows<BFormat::Fp4Km>(a);
         else if (fmt == BFormat::Q4Fast) launch_planes_rows<BFormat::Q4Fast>(a);
         else launch_half_rows(a);

@@ -190,3 +190,40 @@ def test_three_term_tiles(hip, monkeypatch, M, K, N, splits):
     codes[N - 1, :4] = [1, 7, 9, 15]
     sb[N - 1, 0] = 252 if M % 2 else 1
     check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 128, 40), (40, 1152, 130), (130, 640, 72)])
+def test_recorded_rows_follow_the_table(hip, M, K, N):
+    """A recording of more than one row queues every route and runs the one for the table the buffer holds at each
+    replay: E8M0 scales, scales whose products are halves, other values with halves, any values."""
+    from bybylang_amd import _abi, synth
+    from bybylang_amd import gpubackend as gb
+    g = synth.rng(M + N)
+    codes = g.integers(0, 16, size=(N, K), dtype=np.uint8)
+    sb = g.integers(118, 136, size=(N, K // 32), dtype=np.uint8)
+    x = synth.activations(g, M, K, np.float32)
+    mx = mx_table()
+    halves = mx.copy()
+    halves[16:] = (1 + np.arange(256) % 13) / 64
+    values = halves.copy()
+    values[1] = 0.75
+    other = mx.copy()
+    other[:16] = g.standard_normal(16)
+    blob = np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.reshape(-1)])
+    words = np.zeros((blob.size + 3) // 4, np.float32)
+    words.view(np.uint8)[: blob.size] = blob
+    assert gb.sessionBegin(gb.gbHip)
+    hx, hw, ht = (gb.sessionUpload(gb.gbHip, v) for v in (x.reshape(-1), words, mx))
+    ho = gb.sessionAllocScratch(gb.gbHip, M * N)
+    assert gb.sessionEnd(gb.gbHip)
+    assert gb.sessionBeginRecording(gb.gbHip)
+    assert gb.sessionFp4GemmTensorCore(gb.gbHip, hx, hw, ht, ho, M, K, N)
+    assert gb.sessionEnd(gb.gbHip), gb.sessionGetLastError(gb.gbHip)
+    rid = gb.sessionLastRecording(gb.gbHip)
+    for t in (mx, halves, other, values, mx, values, halves):
+        _abi.check(_abi.load().byhip_upload(ht.hipHandle, 0, t.ctypes.data, t.nbytes))
+        assert gb.sessionReplay(gb.gbHip, rid, 1), gb.sessionGetLastError(gb.gbHip)
+        check(np.asarray(gb.sessionRead(gb.gbHip, ho, M * N)).reshape(M, N), x, codes, sb, t)
+    gb.sessionFreeRecording(gb.gbHip, rid)
+    for h in (hx, hw, ht, ho):
+        gb.sessionFree(gb.gbHip, h)
