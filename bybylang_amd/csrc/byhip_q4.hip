@@ -408,6 +408,23 @@ bool q4_fast(const byhip_q4w* w) {
     return w->scale_f16 && (zeros_integral(w) || w->zpf) && (w->group == 0 || w->group % 32 == 0);
 }
 
+// Three or four rows of fp32 activations on fp32 scales. The fp32 GEMM's time barely moves with the rows, the
+// GEMV's grows with them and with its launches. Up to one 16-column block per CU the GEMM adds up K inside a
+// block and wins throughout; with more columns it splits K over the grid, and the GEMV wins while it takes the
+// rows in one launch (K up to 2048; four rows of K = 1024 excepted), or three rows in two launches with more than
+// twice the columns. GEMV / GEMM, us, recorded:
+//   M = 3  K = 1024, N = 4096 8.5 / 6.4, N = 8192 8.9 / 9.5, N = 14336 11.7 / 12.5; K = 2048, N = 4096 10.5 / 7.7, N = 6144
+//          10.6 / 12.2, N = 14336 14.0 / 18.8; K = 4096, N = 6144 17.3 / 17.2, N = 11008 25.4 / 29.7, N = 14336 27.4 / 30.0;
+//          K = 6144, N = 4224 30.3 / 17.4, N = 11008 49.2 / 40.9; K = 8192, N = 14336 63.1 / 52.3
+//   M = 4  K = 1024, N = 8192 10.2 / 9.5; K = 2048, N = 5120 11.4 / 10.8, N = 8192 11.5 / 12.7, N = 14336 15.8 / 18.8;
+//          K = 4096, N = 8192 20.8 / 19.1, N = 14336 31.0 / 30.1
+bool gemv_beats_f32_gemm(const byhip_q4w* w, int M) {
+    const int cus = compute_units();
+    if (M > 4 || w->N <= 16 * cus) return false;
+    const bool one = gemv_rows_per_launch(w->K, M, BYHIP_F32) >= M;
+    return M == 3 ? one || (w->K <= 4096 && w->N > 32 * cus) : one && w->K > 1024;
+}
+
 // Routes y = x . W^T. Decode shapes (M <= 8) take the GEMV, whose arithmetic is exact (fp32 scales,
 // zeros and sums; fp32 activations kept to ~22 bits over their whole range), or the per-element
 // kernel when the GEMV does not take the shape. Exception: fp32 activations on weights with the
@@ -461,9 +478,8 @@ void q4_matmul_impl(const void* x, int x_dtype, const byhip_q4w* w, void* y, int
             return;
     }
     // fp32 scales (micro-VM slots, weights outside fp16's range) have no wide tile: from three rows on the
-    // pipelined fp32 GEMM, whose time barely moves with the rows, where the GEMV's grows (K = N = 4096,
-    // M = 1 / 2 / 4 / 8: GEMV 6.0 / 8.7 / 17.3 / 34.6 us, GEMM 11.6 / 12.0 / 12.1 / 12.4).
-    if (mode == 0 && M > 2 && M <= 8 && aligned && gemm_f32_q4_ok(ga)) return launch_gemm_exact(BFormat::Q4Generic, ga);
+    // pipelined fp32 GEMM, but for what gemv_beats_f32_gemm leaves to the GEMV.
+    if (mode == 0 && M > 2 && M <= 8 && aligned && gemm_f32_q4_ok(ga) && !(gemv && gemv_beats_f32_gemm(w, M))) return launch_gemm_exact(BFormat::Q4Generic, ga);
     if (gemv && (mode == 1 || (mode == 0 && M <= 8)))
         return launch_q4_gemv(x, x_dtype, w, y, y_dtype, M, work, work_bytes);
     // Decode shapes the GEMV does not take (K or the group not a multiple of 32, unaligned rows or

@@ -52,3 +52,14 @@ def test_f32_q4_resident(hip, oracle, M, K, N, group, zeros):
     hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, w, y, hip.F32, M)
     want = oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, K // group if group else 1)
     ref_check(y.read(np.float32), want)
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 1024, 4104), (3, 2048, 4097), (4, 1024, 4104), (4, 2048, 4100), (3, 4096, 8200), (3, 4096, 8192), (4, 4096, 4104)])
+def test_few_rows_on_many_columns(hip, oracle, M, K, N):
+    """Three and four rows with more columns than one 16-column block per CU, on either side of the GEMV's lines."""
+    group = 64
+    x, wq, sc, ze = slots(K + M, M, K, N, group, True)
+    w = hip.Q4Weights(wq, sc, ze, K, N, group, K // group)
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, w, y, hip.F32, M)
+    ref_check(y.read(np.float32), oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, K // group))
