@@ -54,6 +54,35 @@ def test_f32_q4_resident(hip, oracle, M, K, N, group, zeros):
     ref_check(y.read(np.float32), want)
 
 
+@pytest.mark.parametrize("zeros", ["one", "group"])
+@pytest.mark.parametrize("M,K,N,group", [(3, 896, 16, 32), (9, 1024, 130, 128), (16, 1152, 600, 64), (11, 2176, 40, 0), (16, 4096, 72, 256),
+                                         (5, 4224, 1000, 32)])
+def test_f32_q4_columns(hip, oracle, M, K, N, group, zeros):
+    """Up to 16 rows on few columns, K split over a block's eight waves: waves without a step, one step
+    for each, one more for the first, up to five for some."""
+    x, wq, sc, ze = slots(M + N, M, K, N, group or K, True)
+    if zeros == "one":
+        ze[:] = 7.5
+    gpr = K // group if group else 1
+    w = hip.Q4Weights(wq, sc, ze, K, N, group, gpr)
+    assert not w.info()["f16_safe"]
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, w, y, hip.F32, M)
+    ref_check(y.read(np.float32), oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, gpr))
+
+
+@pytest.mark.parametrize("M,K", [(13, 2176), (30, 1152), (48, 1280), (60, 2304)])
+def test_f32_q4_unsplit(hip, oracle, monkeypatch, M, K):
+    """All of K in one block of 16 to 64 rows: several rounds of the three buffers, and each remainder."""
+    N, group = 130, 64
+    x, wq, sc, ze = slots(M, M, K, N, group, True)
+    monkeypatch.setenv("BYHIP_Q4_SPLIT", "1")
+    w = hip.Q4Weights(wq, sc, ze, K, N, group, K // group)
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, w, y, hip.F32, M)
+    ref_check(y.read(np.float32), oracle.matmul_q4(x.reshape(-1), wq, sc, ze, M, K, N, group, K // group))
+
+
 @pytest.mark.parametrize("M,K,N", [(3, 1024, 4104), (3, 2048, 4097), (4, 1024, 4104), (4, 2048, 4100), (3, 4096, 8200), (3, 4096, 8192), (4, 4096, 4104)])
 def test_few_rows_on_many_columns(hip, oracle, M, K, N):
     """Three and four rows with more columns than one 16-column block per CU, on either side of the GEMV's lines."""

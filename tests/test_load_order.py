@@ -27,16 +27,21 @@ KERNELS = {
 }
 
 
-def prologues(obj, tmp):
-    """{mangled name: (string of 'D' for direct loads and 'r' for register loads before the first barrier,
-    the vmcnt of the last wait before it)}"""
+def listing(obj, tmp):
+    """The disassembly of an object's gfx950 code, line by line."""
     fb, co = str(tmp / "fatbin"), str(tmp / "code")
     subprocess.run(["objcopy", "--dump-section", ".hip_fatbin=" + fb, obj, os.devnull], check=True, capture_output=True)
     subprocess.run([LLVM + "/clang-offload-bundler", "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
                     "--input=" + fb, "--output=" + co], check=True, capture_output=True)
     text = subprocess.run([LLVM + "/llvm-objdump", "-d", "--no-show-raw-insn", co], check=True, capture_output=True, text=True).stdout
+    return text.splitlines()
+
+
+def prologues(obj, tmp):
+    """{mangled name: (string of 'D' for direct loads and 'r' for register loads before the first barrier,
+    the vmcnt of the last wait before it)}"""
     out, name, seq, wait = {}, None, "", None
-    for line in text.splitlines():
+    for line in listing(obj, tmp):
         m = re.match(r"[0-9a-f]+ <(.*)>:", line)
         if m:
             name, seq, wait = m.group(1), "", None
@@ -69,3 +74,34 @@ def test_first_loads_precede_the_ones_left_in_flight(kernel, tmp_path):
         landed = seq[:max(0, len(seq) - wait)]
         assert landed.count("D") >= direct(args), f"{name}: {seq} with {wait} left in flight"
     assert seen >= 3
+
+
+def test_column_kernel_leaves_one_step_in_flight(tmp_path):
+    """gemm_f32_q4_cols has no barrier in its loop: each wave waits for step t by leaving the loads of step
+    t + 1 in flight, so those must be the newest at every such wait, all of them issued since the branch
+    before it, and the first step's must stand before the first branch."""
+    path = os.path.join(BUILD, "byhip_exact.hip.o")
+    if not (os.path.exists(path) and shutil.which("objcopy") and os.path.exists(LLVM + "/llvm-objdump")):
+        pytest.skip("the build's objects or binutils are not there")
+    seen, name = 0, None
+    for line in listing(path, tmp_path):
+        m = re.match(r"[0-9a-f]+ <(.*)>:", line)
+        if m:
+            m = re.search(r"16gemm_f32_q4_colsILb([01])EEEv", m.group(1))
+            name, seq, first, waits = m, "", True, 0
+            loads = 8 + 2 + (m.group(1) == "0") if m else 0  # activations, weights and scales, zeros per group
+        if not name:
+            continue
+        if re.search(r"\b(buffer|global)_load", line):
+            seq += "D" if " lds" in line else "r"
+        elif re.search(r"\bs_c?branch", line):
+            if first:
+                assert seq.count("D") == 8 and len(seq) == loads, seq
+            first, seq = False, ""
+        elif re.search(r"s_waitcnt vmcnt\(%d\)" % loads, line):
+            assert seq.count("D") == 8 and len(seq) == loads, f"{seq} before a wait that leaves {loads} in flight"
+            waits += 1
+        elif "s_endpgm" in line:
+            assert waits == 2, waits
+            seen, name = seen + 1, None
+    assert seen == 2

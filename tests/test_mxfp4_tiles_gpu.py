@@ -56,3 +56,19 @@ def test_mxfp4_nan_scales_stay_in_their_rows(hip, M, K, N):
     want[M // 2, :] = True
     want[:, N // 2] = True
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("mid", ["1", "2", "3", "4"])
+@pytest.mark.parametrize("K", [3072, 3200, 5888, 6272])
+def test_mxfp4_small_tiles_long_k(hip, oracle, monkeypatch, K, mid):
+    """12, 13, 23 and 25 pairs of steps in one block: the loop over 12 pairs run once and twice, then a tail,
+    with even and odd counts of steps."""
+    from bybylang_amd import synth
+    M, N = 16 * int(mid) - 3, 130
+    xb, xf, wb, _, _ = operands(M, K, N, M + K)
+    monkeypatch.setenv("BYHIP_MX_MID", mid)
+    monkeypatch.setenv("BYHIP_MX_SPLIT", "1")
+    want = np.asarray(oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, wb, synth.mx_table(), xf)).reshape(M, N)
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.mxfp4_gemm(hip.DeviceBuffer.from_array(xb), hip.DeviceBuffer.from_array(wb), y, hip.F32, M, K, N)
+    assert max_abs_rel(y.read(np.float32).reshape(M, N), want) < 1e-5

@@ -1,8 +1,9 @@
-"""fp32 activations as two fp16 planes (FP4-KM with an E2M1 table, half weights) on the MI355X against
-the oracle, at the edges of the tiles and of the table's scales.
+"""fp32 activations on FP4-KM weights with E2M1 values (two fp16 planes where the products are halves, three
+bf16 terms on E8M0 scales), half weights and Q4 weights (two planes) on the MI355X against the oracle, at
+the edges of the tiles and of the table's scales.
 
-Bar: the reference test's tolerance (max|diff| <= 1e-4 * max(1, peak)); a tile that meets a scale
-whose products are not halves is computed in fp32 arithmetic, inf and NaN included.
+Bar: the reference test's tolerance (max|diff| <= 1e-4 * max(1, peak)); infinities and NaNs where the
+oracle has them.
 """
 import numpy as np
 import pytest
@@ -27,7 +28,7 @@ def fp4_case(M, K, N, scales, seed):
     sb = {"ref": g.integers(0, 256, (N, K // 32)), "mx": g.integers(104, 141, (N, K // 32)),
           "edge": g.integers(100, 150, (N, K // 32)), "one": g.integers(120, 130, (N, K // 32))}[scales].astype(np.uint8)
     if scales == "one":
-        sb[N // 2, (K // 32) // 2] = 150  # one scale past the halves: one tile takes fp32 arithmetic
+        sb[N // 2, (K // 32) // 2] = 150  # one scale past the halves
     x = synth.activations(g, M, K, np.float32)
     return x, np.concatenate([synth.fp4km_pack(codes).reshape(-1), sb.reshape(-1)]), t
 
@@ -216,6 +217,18 @@ def test_rows_longer_than_the_scratch(hip, fmt, K):
                             hip.DeviceBuffer.from_array(t), 0, y, hip.F32, M, K, N)
     k = np.nonzero(x.any(axis=0))[0]
     assert np.array_equal(y.read(np.float32).reshape(M, N), x[:, k].astype(np.float64) @ w[:, k].astype(np.float64).T)
+
+
+@pytest.mark.parametrize("scales", ["ref", "one"])
+@pytest.mark.parametrize("K", [2304, 4224])
+@pytest.mark.parametrize("M", [16, 32, 48, 64, 128])
+def test_fp4km_long_k(hip, oracle, monkeypatch, M, K, scales):
+    """All of K in one block, at each tile height: 18 and 33 steps, so that the loop over eight sub-steps runs
+    twice and more, its scale bytes are handed over each time, and a guarded tail follows."""
+    N = 130
+    x, blob, t = fp4_case(M, K, N, scales, M + K)
+    monkeypatch.setenv("BYHIP_Q4_SPLIT", "1")
+    ref_check(run_fp4(hip, x, blob, t, M, K, N, True), oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x))
 
 
 @pytest.mark.parametrize("fmt", ["f16", "q4"])
