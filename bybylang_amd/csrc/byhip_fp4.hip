@@ -84,7 +84,10 @@ bool table_products_are_halves(const float* t) {
 int table_class(const float* t) {
     const bool e2m1 = memcmp(t, kE2M1, sizeof kE2M1) == 0;
     bool mx = e2m1;
-    for (int b = 0; b < 253 && mx; ++b) mx = t[16 + b] == std::ldexp(1.0f, b - 127);
+    for (uint32_t b = 0; b < 253 && mx; ++b) {
+        const uint32_t power = b ? b << 23 : 0x00400000u;  // 2^(b - 127)
+        mx = memcmp(&t[16 + b], &power, 4) == 0;
+    }
     if (mx) return kTableMx;
     return !table_products_are_halves(t) ? kTableAny : e2m1 ? kTableE2m1 : kTableHalves;
 }
