@@ -7,10 +7,10 @@
 //   F16     the half widened (cpu_vm.c:571-575)
 // Activations are used in fp32 (fp16 ones widened exactly); products and sums are fp32, in
 // v_mfma_f32_16x16x4_f32. This is the route for data the fp16 MFMA kernels cannot hold exactly:
-// Q4 weights outside fp16's range, FP4-KM tables whose values are not E2M1 and whose products are not
-// halves, and the micro-VM's Q4 ops (fp32 arithmetic in the reference) above two rows; these take
-// gemm_f32_q4 (below), the pipelined form for Q4 rows and fp16 scales, where it fits. It differs from the
-// reference only in the order of the fp32 additions.
+// Q4 weights outside fp16's range, the micro-VM's Q4 ops (fp32 arithmetic in the reference) above two
+// rows, and FP4-KM tables above one row that are neither E2M1 with E8M0 scales nor all halves in their
+// products. Q4 rows with fp32 scales take gemm_f32_q4 (below), the pipelined form, where it fits. It differs
+// from the reference only in the order of the fp32 additions.
 //
 // Block: BM x 64 outputs, 4 waves; wave w owns columns 16w .. 16w+15 and all BM rows (BM / 16
 // fragments). K steps of 64: each thread stages BM / 4 activations and 16 weights of one column
@@ -197,8 +197,9 @@ __global__ __launch_bounds__(256) void gemm_f32_exact(GemmArgs a) {
 //   chunk k of row r at slot k ^ (r % 16), so the 16 rows of a fragment read hit distinct banks),
 //   three buffers, loads two steps ahead, one barrier per step.
 //   What bounds it: a launch's ramp and the split-K sum at few rows, the fp32 MFMAs with more.
-//   Group 32, fp32 scales and zeros (us with the sum, gemm_f32_exact / here): K = N = 4096 M = 16
-//   26.7 / 13.3, M = 64 60.0 / 28.1; K = N = 8192, M = 64 204.8 / 77.4; K = 2048, N = 600, M = 33 19.5 / 13.0.
+//   Group 32, fp32 scales and zeros (us with the sum, gemm_f32_exact on one copy of the weights / here on three
+//   in turn): K = N = 4096 M = 16 26.7 / 14.6, M = 64 60.0 / 29.6; K = N = 8192, M = 64 204.8 / 79.8; K = 2048,
+//   N = 600, M = 33 19.5 / 13.8.
 constexpr int kRStep = 128;
 
 template <int FM>
@@ -316,8 +317,9 @@ __global__ __launch_bounds__(512, FM <= 2 ? 4 : 2) void gemm_f32_q4(GemmArgs a) 
 // The same for up to 16 rows and so few columns that 128-column blocks would need K split over the grid:
 // a block owns 16 columns over all of K and its eight waves split K (wave w takes steps w, w + 8, ..), each
 // with two activation buffers of its own and no barrier; the partial tiles are added in wave order
-// through LDS, so there is no second launch. K = N = 4096, M = 16: 11.3 us against 13.2 with 8 K
-// splits and their sum; the fp32 MFMAs and the weights' decoding take 5.6 of it per 4,096 of K.
+// through LDS, so there is no second launch. K = N = 4096, M = 16, three copies of the weights in turn: 12.8 us
+// against 14.6 with 8 K splits and their sum; the fp32 MFMAs and the weights' decoding take 5.6 of it per
+// 4,096 of K.
 template <bool ZU>
 __global__ __launch_bounds__(512, 2) void gemm_f32_q4_cols(GemmArgs a) {
     constexpr int kBuf = 16 * kRStep * 4, kLoads = 8 + 2 + (ZU ? 0 : 1);  // per wave and step
@@ -419,9 +421,10 @@ void launch_f32_q4_fm(const GemmArgs& a, dim3 grid) {
 // K splits: as many as leave one block per CU, each of at least two steps (K = N = 4096, M = 16, 4 / 8 /
 // 16 splits: 18.3 / 13.4 / 14.6 us).
 void launch_f32_q4(GemmArgs a) {
-    // Up to 16 rows on at most one 16-column block per CU (us, 128-column blocks with split K / this:
-    // K = N = 4096, M = 16 13.2 / 11.3, M = 4 11.8 / 10.0; K = 8192, N = 4096 18.8 / 16.9; K = 2048, N = 1000
-    // 8.4 / 6.3; K = 1024, N = 512 8.2 / 5.5; past it K = 4096, N = 6144, M = 9 17.4 / 18.4).
+    // Up to 16 rows on at most one 16-column block per CU (us, 128-column blocks with split K / this, three
+    // copies of the weights in turn: K = N = 4096, M = 16 14.6 / 12.8, M = 4 13.5 / 12.0; K = 8192, N = 4096 20.5 / 19.6;
+    // K = 2048, N = 1000 9.6 / 8.4; K = 1024, N = 512 9.4 / 6.3; past it, one copy, K = 4096, N = 6144, M = 9
+    // 17.4 / 18.4).
     if (a.M <= 16 && (a.N + 15) / 16 <= compute_units() && env_int("BYHIP_Q4_SPLIT", 0) == 0) {
         const dim3 grid((unsigned)((a.N + 15) / 16));
         if (a.zeros) launch("gemm_f32_q4_cols", gemm_f32_q4_cols<false>, grid, dim3(512), 0, a);

@@ -5,8 +5,8 @@
 // table; nibble bytes [N, K/2] (byte j of a group: element j low, j + 16 high), scale bytes
 // [N, K/32] at scale_base. One row of fp32 activations takes the decode GEMV (byhip_fp4gemv.hip), more
 // on E2M1 / E8M0 tables gemm_fp4_mx (byhip_fp4mx.hip), on E2M1 values whose products are halves
-// gemm_planes (byhip_planes.hip); other tables whose products are all halves take the fp16 MFMA GEMM with the weights decoded through the table in LDS,
-// the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
+// gemm_planes (byhip_planes.hip); other tables whose products are all halves take the fp16 MFMA GEMM
+// with the weights decoded through the table in LDS, the rest the exact fp32 GEMM. Activations already in MXFP4 take the scaled MFMA when the table is
 // exactly E2M1 and 2^(e-127).
 #include <algorithm>
 #include <cmath>

@@ -945,7 +945,7 @@ struct WideStep {
 // ZG: a zero per group, in fp16 beside the scales (zpf): one more 8-byte load per sub-step and, per
 // fragment and K half, two packed additions that form the zeros' exponent-word terms. Everything
 // else is as with one zero. K = 4096, N = 11008, group 128, M = 251, fp16: 169 us on the general
-// kernel (gemm_f16_mfma), 43 here.
+// kernel (gemm_f16_mfma), 35 here.
 template <int FM, int YT, int D = wide_depth(FM), int V = kWideHalf, bool ZG = false>
 __global__ __launch_bounds__(512, 1) void q4_gemm_wide(GemmArgs a) {
     static_assert(FM == 1 || FM == 2 || FM == 4, "q4_gemm_wide: 16, 32 or 64 rows");

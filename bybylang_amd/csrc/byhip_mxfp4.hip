@@ -554,7 +554,7 @@ void launch_mxfp4_mid(MxArgs a, GemmArgs out) {
     a.tiles_m = (a.M + 16 * FM - 1) / (16 * FM);
     a.tiles = a.tiles_m * ((a.N + 127) / 128);
     a.per_xcd = (a.tiles + kXcds - 1) / kXcds;
-    // K split, in units of four steps, so that the grid holds up to two blocks per CU
+    // K split in units of four steps
     const int units = (a.K / KSTEP + 3) / 4;
     const int splits = choose_split(out, a.tiles, units, 1, env_int("BYHIP_MX_SPLIT", mx_mid_splits(a.tiles, units)), 1);
     if (splits == 1) out.part = nullptr;
