@@ -305,9 +305,7 @@ __global__ __launch_bounds__(256) void gemm_f16_mfma(GemmArgs a) {
 // Per-row shift t of fp32 activations: the row's largest magnitude brought into [2^14, 2^15) (one
 // block per row), so the fp16 hi + lo split of x * 2^t neither overflows nor loses the row's large
 // values to fp16 subnormals.
-__global__ __launch_bounds__(256) void row_range_shift(const float* __restrict__ x, int K, int* __restrict__ out,
-                                                      const int* gate, int gate_want) {
-    if (gate && *gate != gate_want) return;  // another route was chosen (whole grid)
+__global__ __launch_bounds__(256) void row_range_shift(const float* __restrict__ x, int K, int* __restrict__ out) {
     __shared__ float part[4];
     const float* r = x + (size_t)blockIdx.x * K;
     float mx = 0.0f;
@@ -1852,7 +1850,7 @@ void launch_f(const GemmArgs& a0) {
     int* shifts = static_cast<int*>(work);
     if (!a.prepared) {
         launch("row_range_shift", row_range_shift, dim3((unsigned)a.M), dim3(256), 0, static_cast<const float*>(a.x), a.K,
-               shifts, a.gate, a.gate_want);
+               shifts);
         BYHIP_LAUNCHED("row_range_shift");
     }
     a.row_shift = shifts;
