@@ -209,6 +209,9 @@ void launch_q4_stream(const GemmArgs& a, int split_choice = 0);
 // row's planes in half the scratch), and the launch.
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a);
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a);
+// Whether it takes all rows in one pass over the weights, and the time of Q4's passes without split_planes.
+bool gemm_planes_one_pass(BFormat fmt, const GemmArgs& a);
+double gemm_planes_q4_us(const GemmArgs& a);
 
 // Classifies the decode table on the device into *flag (`mx`, `e2m1`: whether those classes' kernels take the
 // call; otherwise such tables count as the next class) and prepares fp32 activations for it. False when

@@ -1660,7 +1660,7 @@ void launch_q4_big(const GemmArgs& a0, int split_choice = 0) {
 // reads a whole output, so both count: 12 for the launch and 8 bytes per output and slice at 1.1 MB
 // per sub-step (0.22 us). K = 4096, fp16, unsplit / split 2 ways: M = 251, N = 11008 35.2 / 43.4 us, M = 520, N = 4096
 // 34.4 / 40.9; K = 14336: M = 256, N = 8448 100.6 / 93.2.
-int wide_splits(const GemmArgs& a, long tiles) {
+int wide_splits(const GemmArgs& a, long tiles, double* time = nullptr) {
     const int nsub = a.K / kWideSub;
     const long cus = compute_units();
     int best = 1;
@@ -1676,6 +1676,7 @@ int wide_splits(const GemmArgs& a, long tiles) {
             best_t = t;
         }
     }
+    if (time) *time = best_t;
     return best;
 }
 
@@ -1744,17 +1745,23 @@ void launch_q4_wide_planes(GemmArgs a, int split_choice) {
     if (a.part) launch_splitk_sum(a, splits);
 }
 
+// Whether the scratch holds the planes of all rows.
+bool q4_wide_f32_fits(const GemmArgs& a) {
+    const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
+    return ((size_t)a.M * sizeof(int) + 255) / 256 * 256 + 2 * (((size_t)a.M * a.K * 2 + 255) / 256 * 256) <= work_bytes;
+}
+
 // The wide tile on fp32 activations: per row a power-of-two shift onto fp16's range and the shifted
 // row as two fp16 planes (split_rows_f16, into the scratch), then the 16- or 32-row tile with three
 // MFMAs per product (hi . w_hi + lo . w_hi + hi . w_lo), every fp32 weight and about 22 bits of
 // each activation kept. False, queueing nothing, when the planes do not fit the scratch.
 bool launch_q4_wide_f32(const GemmArgs& a0, int split_choice = 0) {
+    if (!q4_wide_f32_fits(a0)) return false;
     GemmArgs a = a0;
     uint8_t* const work = static_cast<uint8_t*>(a.work ? a.work : workspace());
     const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
     const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256;
     const size_t plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
-    if (shift_bytes + 2 * plane > work_bytes) return false;
     int* const shifts = reinterpret_cast<int*>(work);
     _Float16* const hi = reinterpret_cast<_Float16*>(work + shift_bytes);
     _Float16* const lo = reinterpret_cast<_Float16*>(work + shift_bytes + plane);
@@ -1909,6 +1916,24 @@ bool launch_q4_choice(BFormat fmt, const GemmArgs& a, int kind, int tile, int sp
 
 bool q4_f32_wide_takes(const GemmArgs& a) { return q4_wide_f32_ok(a) && env_int("BYHIP_Q4_F32_WIDE", 1) != 0; }
 
+// Whether a call with fp32 activations takes the two-plane kernel (two MFMAs per product, 23 bits of x) rather than
+// the 16- or 32-row wide tile (three, 22 bits, but twice the blocks): when its 64 x 128 tiles fill half the CUs;
+// with more rows than one pass takes, also only if its passes take less time than the wide tile's rounds of
+// blocks, 0.30 us per 64-value sub-step. us, wide / planes:
+//   K = N = 4096, M = 64 18.3 / 22.7, 128 24.3 / 25.0, 256 32.2 / 32.2, 300 45.5 / 33.3, 512 58.1 / 44.9
+//   K = 4096, N = 14336, M = 64 25.3 / 26.4, 128 46.6 / 37.2, 509 176.7 / 147; K = 14336, N = 4096, M = 256 82.4 / 69.0;
+//   K = N = 1024, M = 700 13.5 / 17.2
+//   more than one pass: K = 14336, N = 4096, M = 300 125 / 100; K = 9344, N = 1856, M = 1085 221 / 132; K = 6272, N = 1280,
+//   M = 780 49 / 62
+bool q4_planes_take(const GemmArgs& a) {
+    const long cols = (a.N + 127) / 128;
+    if (2 * cols * ((a.M + 63) / 64) < compute_units()) return false;
+    if (gemm_planes_one_pass(BFormat::Q4Fast, a) || !q4_wide_f32_fits(a)) return true;
+    double wide;
+    wide_splits(a, cols * ((a.M + 31) / 32), &wide);
+    return gemm_planes_q4_us(a) < 0.30 * wide;
+}
+
 // Whether a call takes the small-M streaming GEMM: fp16 activations, up to 32 rows (or the lower
 // limit BYHIP_Q4_SKINNY_MAX_M sets for the small-M kernels), weights with the prefill copy, at most
 // two column fragments per 32-row block and K up to 8192, where it beats the split-K kernels (it
@@ -1932,16 +1957,12 @@ void launch_gemm(BFormat fmt, const GemmArgs& a) {
     if (a.M > 65535 * BM) fail("byhip: M=%d too large for one launch", a.M);
     switch (fmt) {
     case BFormat::Q4Fast:
-        // fp32 activations: the two-plane kernel (two MFMAs per product) when its 64 x 128 tiles fill half
-        // the CUs, else the 16- or 32-row wide tile (three, but twice the blocks) where the scratch holds
-        // its planes. us, wide / planes: K = N = 4096, M = 64 18.3 / 22.7, 128 24.3 / 25.0, 256 32.2 / 32.2,
-        // 300 45.5 / 33.3, 512 58.1 / 44.9; K = 4096, N = 14336, M = 64 25.3 / 26.4, 128 46.6 / 37.2, 509
-        // 176.7 / 152.4; K = 14336, N = 4096, M = 256 82.4 / 69.0; K = N = 1024, M = 700 13.5 / 17.2.
-        // BYHIP_Q4_PLANES=0 / 1 leaves every call to the wide tile / gives the planes every call.
+        // fp32 activations: the two-plane kernel (q4_planes_take), else the 16- or 32-row wide tile where the
+        // scratch holds its planes. BYHIP_Q4_PLANES=0 / 1 leaves every call to the wide tile / gives the planes
+        // every call.
         if (q4_f32_wide_takes(a) && gemm_planes_ok(fmt, a)) {
             const int forced = env_int("BYHIP_Q4_PLANES", -1);
-            const long tiles = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
-            if (forced == 1 || (forced < 0 && 2 * tiles >= compute_units())) {
+            if (forced == 1 || (forced < 0 && q4_planes_take(a))) {
                 launch_gemm_planes(fmt, a);
                 break;
             }

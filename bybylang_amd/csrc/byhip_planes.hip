@@ -687,9 +687,7 @@ void launch_planes_fm(const GemmArgs& a, int fm, int splits) {
     }
 }
 
-// Row fragments per tile: the fewest tiles of up to 64 rows, cut to the rows there are (a tile's time
-// hangs on its K more than on its rows: Q4, M = 100, K = 4096, N = 14336, 336 tiles of 48 rows 54.8 us, 224
-// of 64 rows 36.5).
+// FP4-KM: row fragments per tile, the fewest tiles of up to 64 rows, cut to the rows there are.
 int planes_fm(int M) {
     const int row_tiles = (M + 63) / 64;
     return (M + 16 * row_tiles - 1) / (16 * row_tiles);
@@ -706,7 +704,7 @@ struct Pass {
     double time;
 };
 
-// K splits, in 128-value steps: the count that minimises rounds of blocks x (steps per split + 12)
+// FP4-KM: K splits, in 128-value steps: the count that minimises rounds of blocks x (steps per split + 12)
 // (12 for a block's fixed cost: first loads, epilogue), plus 6 steps for the sum's launch.
 Pass planes_pass(int K, long tiles) {
     const int steps = (K + 127) / 128;
@@ -717,6 +715,38 @@ Pass planes_pass(int K, long tiles) {
         if ((steps + per - 1) / per != s) continue;  // the same split as a smaller s
         const double t = (double)((tiles * s + cus - 1) / cus) * (per + 12) + (s > 1 ? 6.0 : 0.0);
         if (t < 0.97 * best.time) best = {s, t};
+    }
+    return best;
+}
+
+// Q4: row fragments per tile and K splits together, by the time of their rounds of blocks in us. A block of 2 / 3 / 4
+// fragments takes 5.9 / 6.7 / 7.7 us and 0.75 / 0.72 / 0.86 per 128-value step, a sum 3.1 us and 1.6 per 1e6 partial
+// values. Fitted to 112 calls of M = 49 .. 1082, K = 128 .. 14336, N = 1088 .. 14336 at every height with 1 to 6
+// splits: the choice is on average 0.2% from the fastest of those, the fewest 64-row tiles were 7.6%; it is never
+// the slower of the two. us, fewest tiles / this: M = 496, K = 1920, N = 1984 25.9 (64 rows, 2 splits) / 19.6 (32 rows);
+// M = 343, K = 1792, N = 5632 40.6 / 30.9 (32); M = 198, K = 3264, N = 4224 33.6 / 26.2 (32); M = 391, K = 6144, N = 10240 149 / 126
+// (48); M = 567, K = 3712, N = 8128 106 / 93 (48); M = 509, K = 4096, N = 14336 147 either way (64).
+struct Q4Tile {
+    int fm;
+    Pass pass;
+};
+Q4Tile q4_tile(int M, int K, int N, size_t room) {  // room: scratch for the partials
+    const int steps = (K + 127) / 128;
+    const int most = std::max(1, std::min<int>(steps / 4, (int)(room / (splitk_stride(M, N) * sizeof(float)))));
+    const long cus = compute_units(), cols = (N + kBN - 1) / kBN;
+    if (M <= 16) return {1, planes_pass(K, cols)};
+    constexpr double kBlock[3] = {5.9, 6.7, 7.7}, kStepUs[3] = {0.75, 0.72, 0.86};
+    Q4Tile best = {4, {1, 1e300}};
+    for (int fm = 4; fm >= 2; --fm) {
+        if (16 * fm >= M + 16) continue;  // a fragment of rows past M
+        const long tiles = cols * ((M + 16 * fm - 1) / (16 * fm));
+        for (int s = 1; s <= most; ++s) {
+            const int per = (steps + s - 1) / s;
+            if ((steps + per - 1) / per != s) continue;  // the same split as a smaller s
+            const double t = (double)((tiles * s + cus - 1) / cus) * (kBlock[fm - 2] + per * kStepUs[fm - 2]) +
+                             (s > 1 ? 3.1 + 1.6e-6 * M * N * s : 0.0);
+            if (t < best.pass.time) best = {fm, {s, t}};
+        }
     }
     return best;
 }
@@ -778,10 +808,12 @@ void launch_half_rows(const GemmArgs& a0) {
 template <BFormat F>
 void launch_planes_rows(const GemmArgs& a0) {
     GemmArgs a = a0;
-    const int fm = planes_fm(a.M);
-    const long tiles = planes_tiles(a.M, a.N);
-    const int forced = env_int("BYHIP_Q4_SPLIT", 0);
-    const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : planes_pass(a.K, tiles).splits, 1);
+    Q4Tile tile = {planes_fm(a.M), {}};
+    if constexpr (F == BFormat::Q4Fast) tile = q4_tile(a.M, a.K, a.N, a.work_bytes);
+    else tile.pass = planes_pass(a.K, planes_tiles(a.M, a.N));
+    const int fm = tile.fm, forced = env_int("BYHIP_Q4_SPLIT", 0);
+    const long tiles = (long)((a.N + kBN - 1) / kBN) * ((a.M + 16 * fm - 1) / (16 * fm));
+    const int splits = choose_split(a, tiles, (a.K + 127) / 128, 1, forced > 0 ? forced : tile.pass.splits, 1);
     if (splits == 1) a.part = nullptr;
     if constexpr (F == BFormat::Q4Fast) {
         if (a.zeros) launch_planes_fm<F, true>(a, fm, splits);
@@ -792,31 +824,52 @@ void launch_planes_rows(const GemmArgs& a0) {
     if (a.part) launch_splitk_sum(a, splits);
 }
 
+// The row shifts and both planes.
+size_t plane_bytes(int M, int K) {
+    return ((size_t)M * sizeof(int) + 255) / 256 * 256 + 2 * (((size_t)M * K * 2 + 255) / 256 * 256);
+}
+
 // Rows whose planes fit half the scratch (the rest holds split-K partials) and whose offsets stay below 2^31.
 size_t plane_rows(const GemmArgs& a) {
     const size_t work_bytes = a.work ? a.work_bytes : kWorkspaceBytes;
     return std::min<size_t>({work_bytes / 2 / ((size_t)a.K * 4 + sizeof(int)), ((size_t)kPast / 2) / ((size_t)a.K * 2), 65535 * 16});
 }
 
-// Rows of a pass over the weights: all of them where they fit (K = N = 4096, M = 970 in one pass 87 us,
-// 960 + 10 94), else as many whole 64-row tiles as fit or even shares of those, whichever passes' rounds of
-// blocks take less time (us, K = N = 4096, M = 1024: 960 + 64 rows 105, 2 x 512 94; M = 2048: 2 x 960 + 128 191, 3 x 704
-// 227; K = 14336, N = 4096, M = 300: 256 + 44 103, 192 + 108 113).
-int planes_pass_rows(BFormat fmt, const GemmArgs& a) {
-    const int most = (int)std::min<size_t>(plane_rows(a), (size_t)a.M);
-    if (most == a.M || most < 64) return most;
-    auto time_of = [&](int rows) {
-        if (rows == 0) return 0.0;
-        if (fmt != BFormat::F16) return planes_pass(a.K, planes_tiles(rows, a.N)).time;
-        const HalfTiles h = half_tiles(rows, a.K, a.N);
+// The time of passes of `rows` rows each and one of what is left.
+double passes_time(BFormat fmt, const GemmArgs& a, int rows) {
+    auto pass = [&](int m) {
+        if (m == 0) return 0.0;
+        if (fmt == BFormat::Q4Fast) return q4_tile(m, a.K, a.N, (a.work ? a.work_bytes : kWorkspaceBytes) - plane_bytes(m, a.K)).pass.time;
+        if (fmt == BFormat::Fp4Km) return planes_pass(a.K, planes_tiles(m, a.N)).time;
+        const HalfTiles h = half_tiles(m, a.K, a.N);
         return half_pass(h.tiles, a.K / kSub).time * (h.rows == 128 ? 1.6 : 1.0);
     };
-    auto total = [&](int rows) { return (double)(a.M / rows) * time_of(rows) + time_of(a.M % rows); };
-    const int full = most / 64 * 64, blocks = (a.M + full - 1) / full, even = (a.M + 64 * blocks - 1) / (64 * blocks) * 64;
-    return total(even) < 0.97 * total(full) ? even : full;
+    return (double)(a.M / rows) * pass(rows) + pass(a.M % rows);
+}
+
+// Rows of a pass over the weights: all of them up to the whole 64-row tiles that fit the scratch. Past that, all
+// of them where they fit, those whole tiles, or even shares of them, by the time of the passes' rounds of blocks
+// (us, K = N = 4096, M = 970: all 85, 960 + 10 94; M = 1024: 960 + 64 rows 105, 2 x 512 92; M = 2048: 2 x 960 + 128 185, 3 x 704
+// 227; K = 14336, N = 4096, M = 300: 256 + 44 100, 192 + 108 113; K = 11328, N = 6016, M = 361: all 147, 320 + 41 130).
+int planes_pass_rows(BFormat fmt, const GemmArgs& a) {
+    const int most = (int)plane_rows(a), full = most / 64 * 64;
+    if (a.M <= std::max(full, std::min(most, 63))) return a.M;
+    if (full == 0) return most;
+    const int blocks = (a.M + full - 1) / full, even = (a.M + 64 * blocks - 1) / (64 * blocks) * 64;
+    int best = full;
+    double best_t = passes_time(fmt, a, full);
+    for (const int rows : {even, a.M <= most ? a.M : even}) {
+        const double t = passes_time(fmt, a, rows);
+        if (t < (rows == a.M ? 1.03 : 0.97) * best_t) best = rows, best_t = t;
+    }
+    return best;
 }
 
 }  // namespace
+
+bool gemm_planes_one_pass(BFormat fmt, const GemmArgs& a) { return planes_pass_rows(fmt, a) >= a.M; }
+
+double gemm_planes_q4_us(const GemmArgs& a) { return passes_time(BFormat::Q4Fast, a, planes_pass_rows(BFormat::Q4Fast, a)); }
 
 bool gemm_planes_ok(BFormat fmt, const GemmArgs& a) {
     constexpr uint64_t kLim = kPast;  // offsets stay below 2^31 (loads past the end)
@@ -845,8 +898,8 @@ PlaneScratch plane_scratch(const GemmArgs& a) {
     uint8_t* const work = static_cast<uint8_t*>(a.work ? a.work : workspace());
     const size_t bytes = a.work ? a.work_bytes : kWorkspaceBytes;
     const size_t shift_bytes = ((size_t)a.M * sizeof(int) + 255) / 256 * 256, plane = ((size_t)a.M * a.K * 2 + 255) / 256 * 256;
-    return {reinterpret_cast<int*>(work), work + shift_bytes, work + shift_bytes + plane, work + shift_bytes + 2 * plane,
-            bytes - shift_bytes - 2 * plane};
+    const size_t used = plane_bytes(a.M, a.K);
+    return {reinterpret_cast<int*>(work), work + shift_bytes, work + shift_bytes + plane, work + used, bytes - used};
 }
 
 }  // namespace

@@ -231,6 +231,26 @@ def test_fp4km_long_k(hip, oracle, monkeypatch, M, K, scales):
     ref_check(run_fp4(hip, x, blob, t, M, K, N, True), oracle.tile_gemm(0, M, K, N, N * (K // 2), 0, blob, t, x))
 
 
+@pytest.mark.parametrize("M,K,N", [(33, 256, 16400), (49, 1088, 9000), (67, 64, 8320), (331, 896, 5696), (392, 576, 2368), (391, 1024, 5000),
+                                   (448, 384, 3776), (70, 4096, 8256), (361, 8192, 2100)])
+@pytest.mark.parametrize("zeros", ["one", "group"])
+def test_q4_tile_heights(hip, oracle, monkeypatch, M, K, N, zeros):
+    """Calls that the times of the blocks' rounds give to tiles of 32, 48 and 64 rows, whole and with K split: rows at
+    the tiles' edges against the oracle."""
+    from bybylang_amd import synth
+    g = synth.rng(M + K)
+    wq, sc, ze, _ = synth.q4_weights(g, N, K, 32)
+    if zeros == "group":
+        ze = g.integers(0, 16, ze.size).astype(np.float32)
+    monkeypatch.setenv("BYHIP_Q4_PLANES", "1")
+    x = synth.activations(g, M, K, np.float32)
+    y = hip.DeviceBuffer(M * N * 4)
+    hip.q4_matmul(hip.DeviceBuffer.from_array(x.reshape(-1)), hip.F32, hip.Q4Weights(wq, sc, ze, K, N, 32, K // 32), y, hip.F32, M)
+    rows = sorted({0, 31, 32, min(47, M - 1), min(48, M - 1), min(64, M - 1), M - 1})
+    want = oracle.matmul_q4(x[rows].reshape(-1), wq, sc, ze, len(rows), K, N, 32, K // 32)
+    ref_check(y.read(np.float32).reshape(M, N)[rows], np.asarray(want).reshape(len(rows), N))
+
+
 @pytest.mark.parametrize("fmt", ["f16", "q4"])
 @pytest.mark.parametrize("M", [257, 292, 293, 600])
 def test_rows_about_what_the_scratch_holds(hip, oracle, monkeypatch, fmt, M):
