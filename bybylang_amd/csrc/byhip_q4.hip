@@ -410,9 +410,10 @@ bool q4_fast(const byhip_q4w* w) {
 
 // Three or four rows of fp32 activations on fp32 scales. The fp32 GEMM's time barely moves with the rows, the
 // GEMV's grows with them and with its launches. Up to one 16-column block per CU the GEMM adds up K inside a
-// block and wins throughout; with more columns it splits K over the grid, and the GEMV wins while it takes the
-// rows in one launch (K up to 2048; four rows of K = 1024 excepted), or three rows in two launches with more than
-// twice the columns. GEMV / GEMM, us, recorded:
+// block and wins throughout; with more columns it splits K over the grid, and from K = 1024 on the GEMV wins
+// while it takes the rows in one launch (K up to 2048), or three rows in two launches with more than twice the
+// columns. Errors against 64 bits there are alike (K = 2048 2.9e-7 / 2.8e-7, K = 4096 2.7e-7 / 4.6e-7; at K = 1024
+// 3.0e-7 / 2.1e-7 and 6% in time, which stays on the GEMM). GEMV / GEMM, us, recorded:
 //   M = 3  K = 1024, N = 4096 8.5 / 6.4, N = 8192 8.9 / 9.5, N = 14336 11.7 / 12.5; K = 2048, N = 4096 10.5 / 7.7, N = 6144
 //          10.6 / 12.2, N = 14336 14.0 / 18.8; K = 4096, N = 6144 17.3 / 17.2, N = 11008 25.4 / 29.7, N = 14336 27.4 / 30.0;
 //          K = 6144, N = 4224 30.3 / 17.4, N = 11008 49.2 / 40.9; K = 8192, N = 14336 63.1 / 52.3
@@ -420,9 +421,9 @@ bool q4_fast(const byhip_q4w* w) {
 //          K = 4096, N = 8192 20.8 / 19.1, N = 14336 31.0 / 30.1
 bool gemv_beats_f32_gemm(const byhip_q4w* w, int M) {
     const int cus = compute_units();
-    if (M > 4 || w->N <= 16 * cus) return false;
+    if (M > 4 || w->K <= 1024 || w->N <= 16 * cus) return false;
     const bool one = gemv_rows_per_launch(w->K, M, BYHIP_F32) >= M;
-    return M == 3 ? one || (w->K <= 4096 && w->N > 32 * cus) : one && w->K > 1024;
+    return one || (M == 3 && w->K <= 4096 && w->N > 32 * cus);
 }
 
 // Routes y = x . W^T. Decode shapes (M <= 8) take the GEMV, whose arithmetic is exact (fp32 scales,
@@ -432,7 +433,9 @@ bool gemv_beats_f32_gemm(const byhip_q4w* w, int M) {
 // bits of x) from M = 3, and at M = 2 when one GEMV launch does not hold both rows. The GEMV's time
 // grows with its rows while the tile's barely moves (fp32, K x N = 4096 x 14336, M = 1 / 2 / 3 /
 // 4 / 8: GEMV 11.6 / 14.0 / 25.6 / 27.6 / 54.2 us, tile 15.6 / 15.8 / 15.9 / 16.1 / 16.6;
-// 14336 x 4096: GEMV 13.7 / 27.2 / 40.6 / 53.9 / 107.0, tile 18.6 / 19.2 / 19.3 / 19.5 / 20.7).
+// 14336 x 4096: GEMV 13.7 / 27.2 / 40.6 / 53.9 / 107.0, tile 18.6 / 19.2 / 19.3 / 19.5 / 20.7). Three and four
+// rows of K up to 2048 on up to 8192 columns would take less time on the GEMV (K = 1024, N = 4096, M = 3 / 4 7.2 / 8.6 us,
+// tile 10.2 / 10.2), at twice the error against 64 bits (2.9e-7, tile 1.5e-7): they stay on the tile.
 // fp16 activations take the wide tile with each weight as two fp16 terms that add up to it (the
 // weights exact, as in the GEMV) past 4 rows, or past the rows one GEMV launch holds (fp16,
 // M = 2 / 4 / 5 / 8: 4096 x 14336 GEMV 9.9 / 13.8 / 21.1 / 27.2 us, tile 12.6 / 12.6 / 12.7 /
