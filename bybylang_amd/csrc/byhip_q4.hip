@@ -410,7 +410,7 @@ bool q4_fast(const byhip_q4w* w) {
 
 // Three or four rows of fp32 activations on fp32 scales. The fp32 GEMM's time barely moves with the rows, the
 // GEMV's grows with them and with its launches. Up to one 16-column block per CU the GEMM adds up K inside a
-// block and wins throughout; with more columns it splits K over the grid, and from K = 1024 on the GEMV wins
+// block and wins throughout; with more columns it splits K over the grid, and above K = 1024 the GEMV wins
 // while it takes the rows in one launch (K up to 2048), or three rows in two launches with more than twice the
 // columns. Errors against 64 bits there are alike (K = 2048 2.9e-7 / 2.8e-7, K = 4096 2.7e-7 / 4.6e-7; at K = 1024
 // 3.0e-7 / 2.1e-7 and 6% in time, which stays on the GEMM). GEMV / GEMM, us, recorded:
