@@ -159,6 +159,7 @@ void fp4km_run(const void* x, int x_dtype, const uint8_t* blob, size_t blob_byte
             if (launch_fp4km_prepare(a, mx, e2m1, flag)) {  // a single pass on each route
                 g.prepared = true;
                 g.sums = &sums;
+                sums.rows = M;
             }
             if (mx) {
                 g.gate_want = kTableMx;

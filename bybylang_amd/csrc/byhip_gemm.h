@@ -65,8 +65,9 @@ struct GemmArgs {
     // on the stream), so every route can be queued and only the chosen one runs.
     const int* gate = nullptr;
     int gate_want = 0;
-    // Queued routes only: fp4km_prepare has left the row shifts and planes in the scratch; the routes' split-K
-    // sums are collected here (on the host) for one launch behind them all.
+    // Queued routes only: fp4km_prepare has left the row shifts and planes of all rows in the scratch, so each
+    // route takes them in one pass; the routes' split-K sums are collected here (on the host) for one launch
+    // behind them all.
     bool prepared = false;
     struct RouteSums* sums = nullptr;
 };
@@ -83,6 +84,7 @@ enum { kTableAny = 0, kTableHalves = 1, kTableE2m1 = 2, kTableMx = 3, kTableClas
 struct RouteSums {
     const float* part[kTableClasses] = {};
     int splits[kTableClasses] = {};
+    int rows = 0;  // of every route's partials and of y
 };
 
 // Whether 8-output chunks may leave as 16-byte stores: every row of y (or of the split-K

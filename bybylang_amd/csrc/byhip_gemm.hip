@@ -1552,6 +1552,7 @@ int choose_split(GemmArgs& a, long tiles, int nsteps, int min_steps, int forced,
 
 void launch_splitk_sum(const GemmArgs& a, int splits) {
     RouteSums s, &to = a.sums ? *a.sums : s;
+    if (a.sums && a.sums->rows != a.M) fail("byhip: internal: a sum of %d rows among routes of %d", a.M, a.sums->rows);
     const int c = a.gate ? a.gate_want : 0;
     to.part[c] = a.part;
     to.splits[c] = splits;

@@ -915,7 +915,7 @@ bool launch_fp4km_prepare(const GemmArgs& a, bool mx, bool e2m1, int* flag) {
 }
 
 void launch_gemm_planes(BFormat fmt, const GemmArgs& a0) {
-    const size_t rows = (size_t)planes_pass_rows(fmt, a0);
+    const size_t rows = (size_t)(a0.prepared ? a0.M : planes_pass_rows(fmt, a0));
     for (size_t m = 0; m < (size_t)a0.M; m += rows) {
         GemmArgs a = a0;
         a.M = (int)std::min<size_t>(rows, (size_t)a0.M - m);

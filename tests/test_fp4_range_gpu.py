@@ -192,10 +192,11 @@ def test_three_term_tiles(hip, monkeypatch, M, K, N, splits):
     check(run(hip, x, codes, sb, mx_table()), x, codes, sb, mx_table())
 
 
-@pytest.mark.parametrize("M,K,N", [(2, 128, 40), (40, 1152, 130), (130, 640, 72)])
+@pytest.mark.parametrize("M,K,N", [(2, 128, 40), (40, 1152, 130), (130, 640, 72), (1000, 4096, 2120), (1024, 4096, 40)])
 def test_recorded_rows_follow_the_table(hip, M, K, N):
     """A recording of more than one row queues every route and runs the one for the table the buffer holds at each
-    replay: E8M0 scales, scales whose products are halves, other values with halves, any values."""
+    replay: E8M0 scales, scales whose products are halves, other values with halves, any values. K = 4096: 1023
+    rows' planes fit the scratch."""
     from bybylang_amd import _abi, synth
     from bybylang_amd import gpubackend as gb
     g = synth.rng(M + N)
